@@ -72,6 +72,7 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in
   constexpr int P = row_lanes(M);
   using F = Fft4<T, M, P, -1>;
   constexpr int Q = F::Q;
+  static_assert(kR2cBlock % P == 0, "every thread of the block belongs to a row slot");
   constexpr int RB = kR2cBlock / P;
   constexpr int SS = slot_stride(F::SCR > M ? F::SCR : M);
   __shared__ cx<T> lds[RB * SS];
@@ -203,6 +204,7 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restr
   constexpr int P = row_lanes(M);
   using F = Fft4<T, M, P, +1>;
   constexpr int Q = F::Q;
+  static_assert(row_block<T>() % P == 0, "every thread of the block belongs to a row slot");
   constexpr int RB = row_block<T>() / P;
   constexpr int SS = slot_stride(F::SCR);
   __shared__ cx<T> lds[RB * SS];

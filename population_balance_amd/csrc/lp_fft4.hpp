@@ -27,10 +27,12 @@ template <typename T> struct V2;
 template <> struct V2<double> { using t = double2; };
 template <> struct V2<float> { using t = float2; };
 
-// lanes per row transform of M complex points (P) -- M = P*Q
+// lanes per row transform of M complex points (P) -- M = P*Q.  P divides 64, so that the
+// slots of a block tile it exactly: with 6 and 12 lanes the last threads of a block (252..255)
+// had a row and an LDS slot past the block's own
 __host__ __device__ constexpr int row_lanes(int M) {
-  return M == 16 ? 4 : M == 24 ? 4 : M == 32 ? 4 : M == 48 ? 4 : M == 64 ? 8 : M == 72 ? 6
-       : M == 96 ? 8 : M == 128 ? 8 : M == 144 ? 12 : M == 192 ? 8 : 0;
+  return M == 16 ? 4 : M == 24 ? 4 : M == 32 ? 4 : M == 48 ? 4 : M == 64 ? 8 : M == 72 ? 8
+       : M == 96 ? 8 : M == 128 ? 8 : M == 144 ? 16 : M == 192 ? 8 : 0;
 }
 
 // LDS stride (elements) of a transform slot holding n elements: rounded so that
