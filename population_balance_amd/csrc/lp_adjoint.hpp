@@ -78,106 +78,6 @@ __global__ void k_adj_dpdz(const double *__restrict__ apz, double *__restrict__ 
   ap[i] = v;
 }
 
-// press_stag_array.f90:149-329 with tridag_array.f90, transposed, one thread per mode.
-// Input spectra (forward y transforms of the r2c, pitch `pitch` complex per row):
-// Sp[j] of the adjoint of p (planes 0..nz-1), Sx[j-1], Sy[j-1] of the adjoints of dpdx,
-// dpdy (j = 1..nz-1).  The adjoint of p_hat is W (Sp - i kx Sx - i ky Sy), W = 2 on the
-// interior kx (c2r^T).  The transposed system A^T lambda = that is solved (A: wall row
-// (-1, 1), interior rows (1/dz^2, bi, 1/dz^2), lid row (-1, 1)); the mean mode is a
-// reverse cumulative sum.  Outputs, already multiplied by the halving of the interior kx
-// (r2c^T) and the forward scales (cst/(1.5 dt) for H, cst for the wall and lid rows):
-// Hx, Hy, Hz planes 0..nz-2 (H levels 1..nz-1), bw, tw one plane each.
-__global__ __launch_bounds__(64) void k_press_adj(const cx<double> *__restrict__ Sp, const cx<double> *__restrict__ Sx,
-                                                  const cx<double> *__restrict__ Sy, const double *__restrict__ kxt,
-                                                  const double *__restrict__ kyt, cx<double> *__restrict__ Hx,
-                                                  cx<double> *__restrict__ Hy, cx<double> *__restrict__ Hz,
-                                                  cx<double> *__restrict__ bw, cx<double> *__restrict__ tw,
-                                                  double *__restrict__ gam, cx<double> *__restrict__ lam, int lh,
-                                                  int ny, int nz, long pitch, double dz, double sH, double sB) {
-  const long m = gtid();
-  const long nh = (long)lh * ny;
-  if (m >= nh) return;
-  const int jx = (int)(m % lh), jy = (int)(m / lh);
-  const long o = (long)jy * pitch + jx;
-  const long ps = pitch * ny;
-  const cx<double> z0 = mk<double>(0.0, 0.0);
-  if (jy == ny / 2 || jx == lh - 1) {  // Nyquist modes: p_hat is zero there
-    for (int j = 0; j < nz - 1; ++j) { Hx[j * ps + o] = z0; Hy[j * ps + o] = z0; Hz[j * ps + o] = z0; }
-    bw[o] = z0; tw[o] = z0;
-    return;
-  }
-  const double W = (jx == 0) ? 1.0 : 2.0, h = (jx == 0) ? 1.0 : 0.5;
-  const double kx = kxt[m], ky = kyt[m];
-  auto rhs = [&](int j) -> cx<double> {  // adjoint of p_hat(j), j = 0..nz
-    if (j >= nz) return z0;
-    cx<double> v = Sp[(long)j * ps + o];
-    if (j >= 1) {
-      const cx<double> a = Sx[(long)(j - 1) * ps + o], b = Sy[(long)(j - 1) * ps + o];
-      // -i kx a - i ky b
-      v = mk<double>(v.x + kx * a.y + ky * b.y, v.y - kx * a.x - ky * b.x);
-    }
-    return mk<double>(W * v.x, W * v.y);
-  };
-  if (m == 0) {  // mean mode :303-312: p(1) = -dz bw, p(j) = p(j-1) + dz Hz(j)
-    cx<double> acc = z0;
-    for (int j = nz; j >= 2; --j) {
-      const cx<double> r = rhs(j);
-      acc = mk<double>(acc.x + r.x, acc.y + r.y);
-      if (j <= nz - 1) Hz[(long)(j - 1) * ps + o] = mk<double>(h * sH * dz * acc.x, h * sH * dz * acc.y);
-    }
-    const cx<double> r1 = rhs(1);
-    acc = mk<double>(acc.x + r1.x, acc.y + r1.y);
-    bw[o] = mk<double>(h * sB * -dz * acc.x, h * sB * -dz * acc.y);
-    tw[o] = z0;
-    Hx[o] = z0; Hy[o] = z0;
-    for (int j = 1; j < nz - 1; ++j) { Hx[j * ps + o] = z0; Hy[j * ps + o] = z0; }
-    Hz[o] = z0;  // H level 1 of the mean mode is not read by the forward
-    return;
-  }
-  const double idz2 = 1.0 / (dz * dz);
-  const double bi = -(kx * kx + ky * ky + 2.0 / (dz * dz));
-  // A^T: a'_j = c_{j-1}, b'_j = b_j, c'_j = a_{j+1}
-  auto ap_ = [&](int j) { return j == 0 ? 0.0 : (j - 1 == 0 ? 1.0 : idz2); };
-  auto bp_ = [&](int j) { return j == 0 ? -1.0 : (j == nz ? 1.0 : bi); };
-  auto cp_ = [&](int j) { return j == nz ? 0.0 : (j + 1 == nz ? -1.0 : idz2); };
-  double bet = bp_(0);
-  cx<double> r0 = rhs(0);
-  cx<double> up = mk<double>(r0.x / bet, r0.y / bet);
-  lam[m] = up;
-  for (int j = 1; j <= nz; ++j) {
-    const double gm = cp_(j - 1) / bet;
-    gam[(long)j * nh + m] = gm;
-    bet = bp_(j) - ap_(j) * gm;
-    const cx<double> r = rhs(j);
-    const double a = ap_(j);
-    up = mk<double>((r.x - a * up.x) / bet, (r.y - a * up.y) / bet);
-    lam[(long)j * nh + m] = up;
-  }
-  // back substitution from lambda(nz) down; iteration j knows lambda(j) and lambda(j+1)
-  cx<double> nxt = up;  // lambda(nz)
-  tw[o] = mk<double>(h * sB * -dz * nxt.x, h * sB * -dz * nxt.y);
-  for (int j = nz - 1; j >= 0; --j) {
-    const cx<double> l0 = lam[(long)j * nh + m];
-    const double gm = gam[(long)(j + 1) * nh + m];
-    const cx<double> lj = mk<double>(l0.x - gm * nxt.x, l0.y - gm * nxt.y);
-    if (j >= 1) {  // row j: i (kx Hx(j) + ky Hy(j)) + (Hz(j+1) - Hz(j))/dz
-      const long q = (long)(j - 1) * ps + o;
-      Hx[q] = mk<double>(h * sH * kx * lj.y, h * sH * -kx * lj.x);  // -i kx lambda
-      Hy[q] = mk<double>(h * sH * ky * lj.y, h * sH * -ky * lj.x);
-    }
-    if (j <= nz - 2) {  // Hz(j+1): +lambda(j)/dz from row j (j >= 1), -lambda(j+1)/dz from row j+1
-      const double ax = (j >= 1 ? lj.x : 0.0) - nxt.x, ay = (j >= 1 ? lj.y : 0.0) - nxt.y;
-      Hz[(long)j * ps + o] = mk<double>(h * sH * ax / dz, h * sH * ay / dz);
-    }
-    if (j == 0) bw[o] = mk<double>(h * sB * -dz * lj.x, h * sB * -dz * lj.y);
-    nxt = lj;
-  }
-}
-
-}  // namespace lp
-
-namespace lp {
-
 // forward intermediates of the adjoint's base state: the wall-level dudz, dvdz of the
 // wall law (u / (zl denom), wallstress.f90:176-183 with the frozen u*) and the vorticity
 // of convec.f90:100-133 (jz = 1 on the uvp node)

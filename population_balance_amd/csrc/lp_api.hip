@@ -19,6 +19,7 @@
 #include "lp_lag.hpp"
 #include "lp_convec.hpp"
 #include "lp_adjoint.hpp"
+#include "lp_press.hpp"
 #include "lp_scalar.hpp"
 #include "lp_sgs_alt.hpp"
 
@@ -165,9 +166,9 @@ struct lp_ctx {
   void *Hs[3] = {};           // pressure RHS spectra
   void *bw = nullptr, *tw = nullptr;  // wall / lid divergence spectra
   double *gam = nullptr;      // Thomas scratch (nz+1) x lh x ny
-  // the pressure systems' elimination factors gam(j), 1/bet(j) ((nz+1) x lh x ny), fixed by
-  // the grid: computed once in lp_create (k_press_factors)
-  double *pgam = nullptr, *ibet = nullptr;
+  // the pressure systems' elimination factors bet(j) (binary32 contexts 1/bet(j)), (nz+1) x ny
+  // x sp, fixed by the grid: computed once in lp_create (k_press_factors)
+  double *bet = nullptr;
   void *pspec[3] = {};        // binary64 spectra for the p inverse
   // d_err[0]: zero pivot of a Thomas solve; d_err[1]: non-finite velocity written by a
   // step; d_err[2]: lp_check_finite's scratch flag
@@ -546,7 +547,7 @@ extern "C" int lp_destroy(lp_ctx *c) {
   for (auto p : c->lcon) fr(p);
   for (auto p : c->Fi) fr(p);
   for (auto p : c->Hs) fr(p);
-  fr(c->bw); fr(c->tw); fr(c->gam); fr(c->pgam); fr(c->ibet); fr(c->phat);
+  fr(c->bw); fr(c->tw); fr(c->gam); fr(c->bet); fr(c->phat);
   for (auto p : c->pspec) fr(p);
   fr(c->d_err); fr(c->d_part); fr(c->d_stats); fr(c->d_espec); fr(c->ushift); fr(c->nyq); fr(c->nyq_part); fr(c->adj_block); fr(c->adj_drop); fr(c->tavg); fr(c->d_pvol);
   fr(c->d_obuk); fr(c->tshift); fr(c->d_tbar);
@@ -706,12 +707,11 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
   CK(dalloc(&c->bw, (size_t)c->sp * g.ny * 2 * fe));
   CK(dalloc(&c->tw, (size_t)c->sp * g.ny * 2 * fe));
   CK(dalloc((void **)&c->gam, sizeof(double) * (size_t)g.lh * g.ny * (g.nz + 1)));
-  CK(dalloc((void **)&c->pgam, sizeof(double) * (size_t)g.lh * g.ny * (g.nz + 1)));
-  CK(dalloc((void **)&c->ibet, sizeof(double) * (size_t)g.lh * g.ny * (g.nz + 1)));
+  CK(dalloc((void **)&c->bet, sizeof(double) * (size_t)c->sp * g.ny * (g.nz + 1)));
   {
     const long nmodes = (long)g.lh * g.ny;
     hipLaunchKernelGGL(k_press_factors, grid1(nmodes), dim3(256), 0, c->s, (const double *)c->kx,
-                       (const double *)c->ky, c->pgam, c->ibet, g.lh, g.ny, g.nz, g.dz);
+                       (const double *)c->ky, c->bet, g.lh, g.ny, g.nz, c->sp, g.dz, c->fdt == F32 ? 1 : 0);
     CK(hipGetLastError() == hipSuccess && hipStreamSynchronize(c->s) == hipSuccess
            ? LP_OK
            : set_err(LP_ERR_HIP, "lp_create: pressure factors"));
@@ -1571,18 +1571,21 @@ static int do_press(lp_ctx *c) {
   // :149-329 + tridag_array
   HIPCHK(hipStreamWaitEvent(c->s, c->ev_aux, 0));
   cx<double> *ph = (cx<double> *)c->phat;
-  const dim3 grid_modes((unsigned)((nmodes + 63) / 64));  // 64 modes per block: every CU gets some
   prof_begin(c, LP_K_PRESS_TRIDIAG);
-  if (c->fdt == F64)
-    hipLaunchKernelGGL(k_press_tridiag<double>, grid_modes, dim3(64), 0, c->s, (const cx<double> *)c->Hs[0],
-                       (const cx<double> *)c->Hs[1], (const cx<double> *)c->Hs[2], (const cx<double> *)c->bw,
-                       (const cx<double> *)c->tw, c->kx, c->ky, ph, c->gam, c->ibet, gg.lh, gg.ny, gg.nz, c->sp,
-                       gg.dz, c->d_err);
-  else
-    hipLaunchKernelGGL(k_press_tridiag<float>, grid_modes, dim3(64), 0, c->s, (const cx<float> *)c->Hs[0],
-                       (const cx<float> *)c->Hs[1], (const cx<float> *)c->Hs[2], (const cx<float> *)c->bw,
-                       (const cx<float> *)c->tw, c->kx, c->ky, ph, c->pgam, c->ibet, gg.lh, gg.ny, gg.nz, c->sp,
-                       gg.dz, c->d_err);
+#define PRESS(S, R)                                                                                             \
+  FDISPATCH(c, T, hipLaunchKernelGGL((k_press_tridiag<T, S, R>), dim3((unsigned)(ps / kPsModes)),              \
+                                     dim3(kPsModes * S), 0, c->s, (const cx<T> *)c->Hs[0],                     \
+                                     (const cx<T> *)c->Hs[1], (const cx<T> *)c->Hs[2], (const cx<T> *)c->bw,   \
+                                     (const cx<T> *)c->tw, c->kx, c->ky, ph, (const double *)c->bet, gg.lh,   \
+                                     gg.ny, gg.nz, c->sp, gg.dz, c->d_err))
+  switch (press_segs(gg.nz + 1)) {
+    case 8: PRESS(8, false); break;
+    case 16: PRESS(16, false); break;
+    default:
+      if (press_rounds(gg.nz + 1)) PRESS(32, true);
+      else PRESS(32, false);
+  }
+#undef PRESS
   HIPCHK(hipGetLastError());
   // H_x, H_y, H_z read once, p_hat written once (binary64 complex)
   prof_end(c, LP_K_PRESS_TRIDIAG,
@@ -2487,7 +2490,7 @@ extern "C" int lp_set_frozen(lp_ctx *c, const void *nut, const void *ust) {
 }
 
 namespace {
-// the adjoint's binary64 scratch: NV volumes and NB 3/2-grid volumes, then lambda
+// the adjoint's binary64 scratch: NV volumes and NB 3/2-grid volumes
 constexpr int kAdjNV = 52, kAdjNB = 15;
 }  // namespace
 
@@ -2503,8 +2506,7 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
     return set_err(LP_ERR_ARG, "droplet adjoint: nz * npcon = %ld exceeds 65535", (long)gg.nz * cf.drop.npcon);
   const long nv = vol_el(c), np = plane_el(c);
   const long npb = (long)gg.ld_big * gg.ny2, nvb = npb * gg.nz;
-  const long nh = (long)gg.lh * gg.ny;
-  const size_t need = sizeof(double) * ((size_t)kAdjNV * nv + (size_t)kAdjNB * nvb) + sizeof(double) * 2 * nh * (gg.nz + 1);
+  const size_t need = sizeof(double) * ((size_t)kAdjNV * nv + (size_t)kAdjNB * nvb);
   if (!c->adj_block) {
     RCHK(dalloc((void **)&c->adj_block, need));
     c->adj_bytes = need;
@@ -2512,7 +2514,6 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
   double *V[kAdjNV], *B[kAdjNB];
   for (int q = 0; q < kAdjNV; ++q) V[q] = c->adj_block + (size_t)q * nv;
   for (int q = 0; q < kAdjNB; ++q) B[q] = c->adj_block + (size_t)kAdjNV * nv + (size_t)q * nvb;
-  cx<double> *lam = (cx<double> *)(c->adj_block + (size_t)kAdjNV * nv + (size_t)kAdjNB * nvb);
   AdjGeo ag{gg.nx, gg.ny, gg.nz, gg.ld, np};
   const dim3 gv = grid1(nv);
   const double dz = gg.dz, dt = cf.dt, cst = 1.0 / ((double)gg.nx * gg.ny);
@@ -2559,11 +2560,20 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
     ColOut o{c->spec[q], M_ONE};
     RCHK(col_small(c, c->spec[q], q == 0 ? gg.nz : gg.nz - 1, 1, 0, 1, &o));
   }
-  const dim3 gm((unsigned)((nh + 63) / 64));
-  hipLaunchKernelGGL(k_press_adj, gm, dim3(64), 0, c->s, (const cx<double> *)c->spec[0],
-                     (const cx<double> *)c->spec[1], (const cx<double> *)c->spec[2], c->kx, c->ky,
-                     (cx<double> *)c->Hs[0], (cx<double> *)c->Hs[1], (cx<double> *)c->Hs[2], (cx<double> *)c->bw,
-                     (cx<double> *)c->tw, c->gam, lam, gg.lh, gg.ny, gg.nz, c->sp, dz, cst / (1.5 * dt), cst);
+#define PRESS_ADJ(S, R)                                                                                             \
+  hipLaunchKernelGGL((k_press_adj<S, R>), dim3((unsigned)(ps / kPsModes)), dim3(kPsModes * S), 0, c->s,             \
+                     (const cx<double> *)c->spec[0], (const cx<double> *)c->spec[1], (const cx<double> *)c->spec[2], \
+                     c->kx, c->ky, (cx<double> *)c->Hs[0], (cx<double> *)c->Hs[1], (cx<double> *)c->Hs[2],          \
+                     (cx<double> *)c->bw, (cx<double> *)c->tw, (const double *)c->bet, (cx<double> *)c->phat,      \
+                     gg.lh, gg.ny, gg.nz, c->sp, dz, cst / (1.5 * dt), cst)
+  switch (press_segs(gg.nz + 1)) {
+    case 8: PRESS_ADJ(8, false); break;
+    case 16: PRESS_ADJ(16, false); break;
+    default:
+      if (press_rounds(gg.nz + 1)) PRESS_ADJ(32, true);
+      else PRESS_ADJ(32, false);
+  }
+#undef PRESS_ADJ
   HIPCHK(hipGetLastError());
   double *hx = V[27], *hy = V[28], *hz = V[29], *bwb = V[30], *twb = V[31];
   double *hout[3] = {hx, hy, hz};
@@ -2579,7 +2589,6 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
     RCHK(col_small(c, wl[q], 1, 0, 1, 1, &o));
     RCHK(c2r_small(c, wl[q], gg.lh, 1, wlo[q], F64));
   }
-  (void)ps;
   // ---- AB2, RHS assembly, Euler start ----
   double *afu = V[32], *afv = V[33], *afw = V[34], *acx = V[35], *acy = V[36], *acz = V[37];
   double *adx = V[38], *ady = V[39], *adz = V[40];

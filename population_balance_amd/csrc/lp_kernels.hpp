@@ -659,207 +659,6 @@ __global__ void k_project_bc(T *__restrict__ u, T *__restrict__ v, T *__restrict
   w[i] = T(0);
 }
 
-// press_stag_array.f90:149-329 + tridag_array.f90:30-155, one thread per (kx,ky) mode:
-// assemble the wall row, interior rows and lid row on the fly, binary64 Thomas sweep,
-// gauge-fixed cumulative sum for the mean mode, zero on the Nyquist row and column.
-// H levels 1..nz-1 at planes 0..nz-2 (complex TH, pitch lh), bottomw/topw planes.
-template <typename TH>
-__global__ __launch_bounds__(64) void k_press_tridiag(const cx<TH> *__restrict__ Hx, const cx<TH> *__restrict__ Hy,
-                                const cx<TH> *__restrict__ Hz, const cx<TH> *__restrict__ bw,
-                                const cx<TH> *__restrict__ tw_, const double *__restrict__ kxt,
-                                const double *__restrict__ kyt, cx<double> *__restrict__ ph,
-                                double *__restrict__ gam_w, const double *__restrict__ ibet, int lh, int ny,
-                                int nz, long pitch, double dz, int *__restrict__ err) {
-  // gam_w: the precomputed gam(j) (binary32 contexts, read only) or the scratch the
-  // forward sweep fills (binary64 contexts)
-  const double *gam = gam_w;
-  const long m = gtid();  // mode (kx, ky) = (m % lh, m / lh)
-  const long nh = (long)lh * ny;
-  if (m >= nh) return;
-  const int jx = (int)(m % lh), jy = (int)(m / lh);
-  const long o = (long)jy * pitch + jx;  // offset of the mode in a spectral plane
-  const long ps = pitch * ny;            // spectral plane (H, bw, tw, ph)
-  auto ld_h = [&](const cx<TH> *H, int level) -> cx<double> {  // H(level), level 1..nz
-    if (level >= nz) return mk<double>(0.0, 0.0);
-    cx<TH> v = H[(long)(level - 1) * ps + o];
-    return mk<double>((double)v.x, (double)v.y);
-  };
-  if (jy == ny / 2 || jx == lh - 1) {
-    for (int j = 0; j <= nz; ++j) ph[(long)j * ps + o] = mk<double>(0.0, 0.0);
-    return;
-  }
-  if (m == 0) {  // press_stag_array.f90:303-312
-    cx<double> acc = mk<double>(0.0, 0.0);
-    ph[0] = acc;
-    cx<TH> b0 = bw[0];
-    acc = mk<double>(acc.x - dz * (double)b0.x, acc.y - dz * (double)b0.y);
-    ph[ps] = acc;
-    for (int jz = 2; jz <= nz; ++jz) {
-      cx<double> hz = ld_h(Hz, jz);
-      acc = mk<double>(acc.x + hz.x * dz, acc.y + hz.y * dz);
-      ph[(long)jz * ps] = acc;
-    }
-    return;
-  }
-  const double kx = kxt[m], ky = kyt[m];
-  const double idz2 = 1.0 / (dz * dz);
-  const double bi = -(kx * kx + ky * ky + 2.0 / (dz * dz));
-  // row 0 (wall): b = -1, c = 1, r = -dz * bottomw.  The elimination factors gam(j) and
-  // 1/bet(j) depend on the mode and the grid only.  Binary32 contexts take them from the
-  // tables of k_press_factors (once per context): the forward sweep is then
-  // u(j) = (r(j) - a u(j-1)) * (1/bet(j)), without a division in its chain.  Binary64
-  // contexts form them on the way with the reference's divisions (tridag_array.f90:60-80),
-  // so that their rounding is the reference's.
-  constexpr bool kTab = sizeof(TH) == 4;
-  double bet = -1.0, cprev = 1.0;
-  cx<TH> b0 = bw[o];
-  cx<double> r0 = mk<double>(-dz * (double)b0.x, -dz * (double)b0.y);
-  cx<double> uprev;
-  if constexpr (kTab) {
-    const double ib0 = ibet[m];
-    uprev = mk<double>(r0.x * ib0, r0.y * ib0);
-  } else {
-    uprev = mk<double>(r0.x / bet, r0.y / bet);
-  }
-  ph[o] = uprev;
-  bool bad = false;
-  // The right-hand sides and the back-substitution inputs do not depend on the
-  // recurrence: they are loaded kCh levels at a time, and the loads of the next chunk are
-  // issued before the current chunk is swept (two register buffers), so that the latency
-  // of one chunk overlaps the recurrence of the other.  Levels beyond the system are
-  // loaded from clamped levels and not used.
-  constexpr int kCh = sizeof(TH) == 4 ? 16 : 8;
-  struct HChunk {
-    cx<TH> x[kCh], y[kCh], z[kCh];
-    double ib[kCh];
-  };
-  auto load_h = [&](int j0, HChunk &c) {
-#pragma unroll
-    for (int q = 0; q < kCh; ++q) {
-      const int j = j0 + q;
-      const int lx = j < nz ? j : nz - 1, lz = j + 1 < nz ? j + 1 : nz - 1;
-      c.x[q] = Hx[(long)(lx - 1) * ps + o];
-      c.y[q] = Hy[(long)(lx - 1) * ps + o];
-      c.z[q] = Hz[(long)(lz - 1) * ps + o];
-      if constexpr (kTab) c.ib[q] = ibet[(long)(j <= nz ? j : nz) * nh + m];
-    }
-  };
-  cx<double> hz_lo = ld_h(Hz, 1);  // Hz(j) for the next row j
-  auto sweep_h = [&](int j0, const HChunk &c) {
-#pragma unroll
-    for (int q = 0; q < kCh; ++q) {
-      const int j = j0 + q;
-      if (j > nz) break;
-      double a, b, cc;
-      cx<double> r;
-      if (j < nz) {
-        a = idz2; b = bi; cc = idz2;
-        const bool okz = j + 1 < nz;
-        const cx<double> hx = mk<double>((double)c.x[q].x, (double)c.x[q].y);
-        const cx<double> hy = mk<double>((double)c.y[q].x, (double)c.y[q].y);
-        const cx<double> hz1 = mk<double>(okz ? (double)c.z[q].x : 0.0, okz ? (double)c.z[q].y : 0.0);
-        const cx<double> hz0 = hz_lo;
-        // i*(kx Hx + ky Hy) + (Hz(j+1) - Hz(j))/dz
-        double sx = kx * hx.x + ky * hy.x, sy = kx * hx.y + ky * hy.y;
-        r = mk<double>(-sy + (hz1.x - hz0.x) / dz, sx + (hz1.y - hz0.y) / dz);
-        hz_lo = hz1;
-      } else {
-        cx<TH> t = tw_[o];
-        a = -1.0; b = 1.0; cc = 0.0;
-        r = mk<double>(-(double)t.x * dz, -(double)t.y * dz);
-      }
-      cx<double> uj;
-      if constexpr (kTab) {
-        const double ib = c.ib[q];
-        if (isinf(ib)) bad = true;  // bet(j) == 0
-        uj = mk<double>((r.x - a * uprev.x) * ib, (r.y - a * uprev.y) * ib);
-      } else {
-        double gm = cprev / bet;
-        gam_w[(long)j * nh + m] = gm;
-        bet = b - a * gm;
-        if (bet == 0.0) bad = true;
-        uj = mk<double>((r.x - a * uprev.x) / bet, (r.y - a * uprev.y) / bet);
-      }
-      ph[(long)j * ps + o] = uj;
-      uprev = uj;
-      cprev = cc;
-    }
-  };
-  {
-    HChunk ca, cb;
-    load_h(1, ca);
-    for (int j0 = 1; j0 <= nz; j0 += 2 * kCh) {
-      load_h(j0 + kCh, cb);
-      sweep_h(j0, ca);
-      load_h(j0 + 2 * kCh, ca);
-      sweep_h(j0 + kCh, cb);
-    }
-  }
-  // back substitution, from level nz-1 down to 0, with the same two-buffer prefetch
-  struct BChunk {
-    double g[kCh];
-    cx<double> u[kCh];
-  };
-  auto load_b = [&](int j0, BChunk &c) {
-#pragma unroll
-    for (int q = 0; q < kCh; ++q) {
-      const int j = j0 - q >= 0 ? j0 - q : 0;
-      c.g[q] = gam[(long)(j + 1) * nh + m];
-      c.u[q] = ph[(long)j * ps + o];
-    }
-  };
-  cx<double> unext = uprev;
-  auto sweep_b = [&](int j0, const BChunk &c) {
-#pragma unroll
-    for (int q = 0; q < kCh; ++q) {
-      const int j = j0 - q;
-      if (j < 0) break;
-      cx<double> uj = mk<double>(c.u[q].x - c.g[q] * unext.x, c.u[q].y - c.g[q] * unext.y);
-      ph[(long)j * ps + o] = uj;
-      unext = uj;
-    }
-  };
-  {
-    BChunk ca, cb;
-    load_b(nz - 1, ca);
-    for (int j0 = nz - 1; j0 >= 0; j0 -= 2 * kCh) {
-      load_b(j0 - kCh, cb);
-      sweep_b(j0, ca);
-      load_b(j0 - 2 * kCh, ca);
-      sweep_b(j0 - kCh, cb);
-    }
-  }
-  if (bad) atomicExch(err, 1);
-}
-
-// press_stag_array.f90:149-329 / tridag_array.f90:30-155: the elimination factors of each
-// mode's system (a = c = 1/dz^2, b = -(kx^2 + ky^2 + 2/dz^2) inside; the wall row b = -1,
-// c = 1; the lid row a = -1, b = 1), which depend on the grid only: gam(j) = c(j-1)/bet(j-1)
-// and 1/bet(j), bet(j) = b(j) - a(j) gam(j), in [(nz+1)][lh*ny].  Modes the solve skips
-// are left alone.
-static __global__ void k_press_factors(const double *__restrict__ kxt, const double *__restrict__ kyt,
-                                       double *__restrict__ gam, double *__restrict__ ibet, int lh, int ny, int nz,
-                                       double dz) {
-  const long m = gtid();
-  const long nh = (long)lh * ny;
-  if (m >= nh) return;
-  const int jx = (int)(m % lh), jy = (int)(m / lh);
-  if (jy == ny / 2 || jx == lh - 1 || m == 0) return;
-  const double kx = kxt[m], ky = kyt[m];
-  const double idz2 = 1.0 / (dz * dz);
-  const double bi = -(kx * kx + ky * ky + 2.0 / (dz * dz));
-  double bet = -1.0, cprev = 1.0;
-  ibet[m] = 1.0 / bet;
-  for (int j = 1; j <= nz; ++j) {
-    const double a = j < nz ? idz2 : -1.0, b = j < nz ? bi : 1.0, cc = j < nz ? idz2 : 0.0;
-    const double gm = cprev / bet;
-    gam[(long)j * nh + m] = gm;
-    bet = b - a * gm;
-    ibet[(long)j * nh + m] = 1.0 / bet;
-    cprev = cc;
-  }
-}
-
 // tridag_array.f90:30-155 with explicit a, b, c, r (all binary64); modes skipped as there
 static __global__ void k_tridag_arrays(const double *__restrict__ a, const double *__restrict__ b,
                                 const double *__restrict__ c, const cx<double> *__restrict__ r,

@@ -30,3 +30,80 @@ def test_dealias_uneven(nx, ny, nz):
     assert rel_l2(out, o.dealias2(ref), g.nx) < TOL
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nz", [4, 9, 71, 72, 143, 144, 287, 288, 320])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_pressure_row_segments(nz, prec):
+    """the pressure solve at both sides of each number of segments per block (72, 144 and
+    288 rows: nz + 1), with a last segment that is short or empty, and over several rounds;
+    two solves, the second from other fields.  FP64 against the oracle at 1e-12; mixed at
+    5e-6 (binary32 transforms of fields of order 1 without a mean flow: 6e-8 per operation
+    over the 2 log2(64 32) additions of a plane's transform)."""
+    from harness import random_fields
+    from oracle import Oracle
+    from population_balance_amd import ic
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(64, 32, nz, precision=abi.LP_MIXED if prec == "mixed" else abi.LP_FP64)
+    g = cfg.grid
+    o, lg = Oracle(abi.copy_config(cfg, precision=abi.LP_FP64)), Lesgo(cfg)
+    print(f"\n[case] pressure segments nz={nz} {prec}", flush=True)
+    for seed in (22, 23):
+        u, v, w = ic.turbulent_ic(g, seed=seed, log_law=False)
+        n = random_fields(cfg, ["u", "v", "w", "divtz"], seed=seed)
+        for name, a in (("u", u + 0.1 * n["u"]), ("v", v + 0.1 * n["v"]), ("w", w + 0.1 * n["w"]),
+                        ("divtz", n["divtz"])):
+            o.set_field(name, a)
+            lg.upload(name, a)
+        o.call("press_stag_array")
+        lg.press_stag_array()
+        for name, top in (("p", nz), ("dpdx", nz - 1), ("dpdy", nz - 1)):
+            err = rel_l2(lg.download(name)[:top], o.field(name)[:top], g.nx)
+            print(f"  {name}: {err:.2e}", end="")
+            assert err < (TOL if prec == "fp64" else 5e-6), (name, err)
+        print()
+    lg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("nz", [9, 72, 144, 290])
+def test_adjoint_row_segments(nz):
+    """the transposed pressure solve inside the adjoint step, against the oracle's adjoint
+    at 1e-12, over one and several rounds of segments"""
+    import ctypes as C
+    import torch
+    from harness import random_fields
+    from oracle import Oracle
+    from population_balance_amd import ic
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(32, 32, nz)
+    g = cfg.grid
+    print(f"\n[case] adjoint segments nz={nz}", flush=True)
+    vel = dict(zip(("u", "v", "w"), ic.turbulent_ic(g, seed=4)))
+    n = random_fields(cfg, ["u", "v", "w", "RHSx", "RHSy", "RHSz", "Nu_t", "ustar"], seed=5)
+    ub0 = np.stack([n["u"], n["v"], n["w"]])
+    rb0 = np.stack([n["RHSx"], n["RHSy"], n["RHSz"]])
+    rb0[:, -1] = 0.0
+    nut = 1e-3 * (1.0 + 0.1 * np.clip(n["Nu_t"], -3, 3))
+    ust = 1.0 + 0.1 * np.clip(n["ustar"], -3, 3)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    dp = C.POINTER(C.c_double)
+    o.L.or_step_adjoint.argtypes = [C.c_void_p, dp, dp, dp, dp]
+    p = lambda a: a.ctypes.data_as(dp)  # noqa: E731
+    for name, a in vel.items():
+        o.set_field(name, a)
+        lg.upload(name, a)
+    o.set_time(3)
+    lg.set_time(3)
+    ub_o, rb_o = ub0.copy(), rb0.copy()
+    assert o.L.or_step_adjoint(o.h, p(nut), p(ust), p(ub_o), p(rb_o)) == 0
+    ub, rb, tn, tu = (torch.from_numpy(a).to("cuda") for a in (ub0, rb0, nut, ust))
+    lg.step_adjoint(tn, tu, ub, rb)
+    for q in range(3):
+        eu = rel_l2(ub[q].cpu().numpy(), ub_o[q], g.nx)
+        er = rel_l2(rb[q].cpu().numpy()[:nz - 1], rb_o[q][:nz - 1], g.nx)
+        print(f"  {eu:.2e} {er:.2e}", end="")
+        assert eu < TOL and er < TOL, (q, eu, er)
+    print()
+    lg.close()
+    o.close()
