@@ -300,17 +300,29 @@ __global__ void k_adj_strain(const double *__restrict__ aS11, const double *__re
 
 // out = a - b - c on the physical columns, zero on the padding (filt_da transposed:
 // F(af) - Dx(ax) - Dy(ay)); with wall plane add: af(0) += gw before (the wall-law term)
-__global__ void k_adj_combine(double *__restrict__ out, const double *__restrict__ a, const double *__restrict__ b,
-                              const double *__restrict__ c, AdjGeo g) {
+__global__ void k_adj_combine(double *__restrict__ out, const double *__restrict__ fu, const double *__restrict__ fv,
+                              const double *__restrict__ fw, const double *__restrict__ ux,
+                              const double *__restrict__ vx, const double *__restrict__ wx,
+                              const double *__restrict__ uy, const double *__restrict__ vy,
+                              const double *__restrict__ wy, long nv, AdjGeo g) {
   const long i = gtid();
   if (i >= g.np * g.nz) return;
+  const int q = blockIdx.y;
+  const double *a = q == 0 ? fu : q == 1 ? fv : fw, *b = q == 0 ? ux : q == 1 ? vx : wx;
+  const double *c = q == 0 ? uy : q == 1 ? vy : wy;
   int k, x;
-  out[i] = adj_phys(g, i, k, x) ? a[i] - b[i] - c[i] : 0.0;
+  out[q * nv + i] = adj_phys(g, i, k, x) ? a[i] - b[i] - c[i] : 0.0;
 }
 
-__global__ void k_add_plane(double *__restrict__ a, const double *__restrict__ b, long n) {
+// a0 += b0, a1 += b1, a2 += b2 (blockIdx.y)
+__global__ void k_add_plane3(double *__restrict__ a0, double *__restrict__ a1, double *__restrict__ a2,
+                             const double *__restrict__ b0, const double *__restrict__ b1,
+                             const double *__restrict__ b2, long n) {
   const long i = gtid();
-  if (i < n) a[i] += b[i];
+  if (i >= n) return;
+  const int q = blockIdx.y;
+  double *a = q == 0 ? a0 : q == 1 ? a1 : a2;
+  a[i] += (q == 0 ? b0 : q == 1 ? b1 : b2)[i];
 }
 
 }  // namespace lp

@@ -118,7 +118,7 @@ struct lp_ctx {
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_aux_fork = nullptr, ev_aux = nullptr;
   bool prof_off = false;  // work on s2 that overlaps other kernels is not profiled
-  void *cv_spec[2] = {};  // convec's own spectral scratch (divstress runs meanwhile)
+  void *cv_spec[3] = {};  // convec's own spectral scratch (divstress runs meanwhile)
   bool fork_pending = false;  // the step's convec is still to be started on s2
   Dt fdt = F64;  // field type
   void *f[LP_NFIELDS] = {};
@@ -128,17 +128,20 @@ struct lp_ctx {
   SpecTables tab{};
   // scratch
   void *spec[4] = {};         // small spectra (lh x ny x nz) of the field type
-  void *specb[2] = {};        // big spectra (lh_big x ny2 x nz)
-  // Internal spectra keep rows of sp (small) / sb (big) complex values: lh and lh_big
-  // rounded up to 16, so that every row starts on a 128-byte boundary.
-  long sp = 0, sb = 0;
+  void *specb[3] = {};        // big spectra (the nx/2 kept columns, pitch cv_pitch) x ny2 x nz
+  // Internal spectra keep rows of sp complex values: lh rounded up to 16, so that every row
+  // starts on a 128-byte boundary.
+  long sp = 0;
+  // fields per launch of the spectral passes: as many as leave what one pass writes for the
+  // next in the 256 MB cache behind the L2s (see group_of)
+  int group = 1;
   void *phat = nullptr;       // binary64 p-hat (0..nz) in the sp layout
   void *uvw_spec[3] = {};     // x-spectra of the filtered u, v, w left by the step's filt_da
   // binary32 context: the per-level values that u and v entered filt_da's transform
   // shifted by ([2][nz]); the convective pass adds them back to the kept spectra
   double *ushift = nullptr;
-  double *nyq = nullptr;    // filt_da of binary64 velocities: A [nz][ny], B [nz][nx], C [nz]
-  double *nyq_part = nullptr;  // their partial column sums [nz][kNyqSlices][nx]
+  double *nyq = nullptr;    // filt_da of binary64 velocities, 3 fields: A [nz][ny], B [nz][nx], C [nz]
+  double *nyq_part = nullptr;  // their partial column sums [3][nz][kNyqSlices][nx]
   double *adj_drop = nullptr;  // droplet adjoint scratch: mu, ac, awi volumes + aui, avi faces
   double *tavg = nullptr;      // running time averages (tavg_nq binary64 volumes)
   int tavg_nq = 0;
@@ -256,6 +259,13 @@ static size_t esz_of(Dt d) { return d == F64 ? 8 : 4; }
 static long pad16(long n) { return (n + 15) / 16 * 16; }
 static long plane_el(const lp_ctx *c) { return (long)c->g.ld * c->g.ny; }
 static long vol_el(const lp_ctx *c) { return plane_el(c) * c->g.nz; }
+// Fields that go through a spectral pass together.  Batches pay where a pass is short (launch
+// and fill); where three fields no longer fit the 256 MB cache behind the L2s, the next pass
+// would read from HBM what a single field's pass leaves in that cache.
+static int group_of(size_t spec_bytes) {
+  const size_t n = ((size_t)96 << 20) / (spec_bytes ? spec_bytes : 1);
+  return n < 1 ? 1 : n > (size_t)kMaxSets ? kMaxSets : (int)n;
+}
 static Geo geo(const lp_ctx *c) {
   Geo g;
   g.nx = c->g.nx; g.ny = c->g.ny; g.nz = c->g.nz; g.ld = c->g.ld;
@@ -670,13 +680,13 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
   c->tab.lh = g.lh; c->tab.ny = g.ny;
   size_t fe = esz_of(c->fdt);
   c->sp = (g.lh + 15) / 16 * 16;
-  c->sb = (g.lh_big + 15) / 16 * 16;
+  c->cv_pitch = pad16(g.nx / 2);
   size_t spec_b = (size_t)c->sp * g.ny * g.nz * 2 * fe;
-  size_t specb_b = (size_t)c->sb * g.ny2 * g.nz * 2 * fe;
+  size_t specb_b = (size_t)c->cv_pitch * g.ny2 * g.nz * 2 * fe;
+  c->group = group_of(spec_b);
   size_t vol_b = (size_t)nv * fe;
   for (auto &p : c->spec) CK(dalloc(&p, spec_b));
   for (auto &p : c->specb) CK(dalloc(&p, specb_b));
-  c->cv_pitch = pad16(g.nx / 2);
   const size_t cv_field = (size_t)c->cv_pitch * g.ny2 * g.nz * 2 * fe;
   CK(dalloc(&c->cvb, 6 * cv_field));
   for (auto &p : c->uvw_spec) CK(dalloc(&p, spec_b));
@@ -720,8 +730,8 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
   CK(dalloc(&c->phat, sizeof(double) * 2 * (size_t)c->sp * g.ny * (g.nz + 1)));
   CK(dalloc((void **)&c->d_err, sizeof(int) * 4));
   CK(dalloc((void **)&c->ushift, sizeof(double) * 2 * (size_t)g.nz));
-  CK(dalloc((void **)&c->nyq, sizeof(double) * (size_t)g.nz * (g.ny + g.nx + 1)));
-  CK(dalloc((void **)&c->nyq_part, sizeof(double) * (size_t)g.nz * kNyqSlices * g.nx));
+  CK(dalloc((void **)&c->nyq, 3 * sizeof(double) * (size_t)g.nz * (g.ny + g.nx + 1)));
+  CK(dalloc((void **)&c->nyq_part, 3 * sizeof(double) * (size_t)g.nz * kNyqSlices * g.nx));
   CK(dalloc((void **)&c->d_stats, sizeof(double) * 10 * (size_t)(g.nz - 1)));
   if (cfg->scal.s_flag) {
     CK(dalloc((void **)&c->d_obuk, sizeof(double) * 8));
@@ -818,78 +828,136 @@ static double bytes_col(int nyi, int nyo, int ncols, int nlev, int nout, size_t 
   return (double)ncols * nlev * 2 * e * ((double)nyi + (double)nout * nyo);
 }
 
-// ncols_out < lh writes only the leading kx columns (a spectrum that the caller knows to
-// be zero beyond them)
-// ri: the rows' type and shift (RowIn; default: rows of the field type, no shift)
-static int r2c_small(lp_ctx *c, const void *in, int nlev, double scale, void *spec, int ncols_out = 0,
-                     RowIn ri = {}) {
+// ---- passes over lists of fields; each list is cut into launches of at most c->group sets ----
+// row pass into small spectra; din: the rows' type
+static int r2c_sets(lp_ctx *c, const R2cSet *sets, int n, Dt din) {
   const lp_grid &g = c->g;
-  if (ncols_out <= 0) ncols_out = g.lh;
-  const size_t ei = ri.din < 0 ? esz_of(c->fdt) : esz_of((Dt)ri.din);
-  prof_begin(c, LP_K_ROW_R2C);
-  HIPCHK(row_r2c(c->fdt, g.nx / 2, in, g.ld, plane_el(c), g.ny, nlev, scale, spec, c->sp,
-                 c->sp * g.ny, ncols_out, c->s, ri));
-  prof_end(c, LP_K_ROW_R2C, (double)g.ny * nlev * ((double)g.nx * ei + (double)ncols_out * 2 * esz_of(c->fdt)));
+  for (int i = 0; i < n; i += c->group) {
+    const int m = n - i < c->group ? n - i : c->group;
+    double bytes = 0;
+    for (int f = i; f < i + m; ++f)
+      bytes += (double)g.ny * sets[f].nplanes *
+               ((double)g.nx * esz_of(din) * (sets[f].comp >= 0 ? 2 : 1) + (double)g.lh * 2 * esz_of(c->fdt));
+    prof_begin(c, LP_K_ROW_R2C);
+    HIPCHK(row_r2c(c->fdt, din, g.nx / 2, sets + i, m, g.ld, plane_el(c), g.ny, c->sp, c->sp * g.ny,
+                   sets[i].comp >= 0 ? g.nx / 2 : g.lh, c->s));
+    prof_end(c, LP_K_ROW_R2C, bytes);
+  }
   return LP_OK;
 }
-// ikx: c->kx (its first row is kx of every column) to store the x-derivative instead;
-// shift: per-plane values added back in binary64 (dto F64 from a binary32 spectrum)
-static int c2r_small(lp_ctx *c, const void *spec, int ncols, int nlev, void *out, Dt dto,
-                     const double *ikx = nullptr, const double *shift = nullptr) {
+// row pass back; ikx: c->kx (its first row is kx of every column) to store the x-derivative
+// instead; cst: the div sets' 1/dz
+static int c2r_sets(lp_ctx *c, const C2rSet *sets, int n, int ncols, Dt dto, const double *ikx = nullptr,
+                    double cst = 0.0) {
   const lp_grid &g = c->g;
-  prof_begin(c, LP_K_ROW_C2R);
-  HIPCHK(row_c2r(c->fdt, dto, g.nx / 2, spec, c->sp, c->sp * g.ny, ncols, g.ny, nlev, out, g.ld,
-                 plane_el(c), c->s, ikx, shift));
-  prof_end(c, LP_K_ROW_C2R, bytes_c2r(g.nx, g.ny, nlev, ncols, esz_of(c->fdt), esz_of(dto)));
+  for (int i = 0; i < n; i += c->group) {
+    const int m = n - i < c->group ? n - i : c->group;
+    double bytes = 0;
+    for (int f = i; f < i + m; ++f)
+      bytes += bytes_c2r(g.nx, g.ny, sets[f].nplanes, ncols, esz_of(c->fdt), esz_of(dto)) +
+               (sets[f].div ? (double)plane_el(c) * sets[f].nplanes * esz_of(dto) : 0.0);
+    prof_begin(c, LP_K_ROW_C2R);
+    HIPCHK(row_c2r(c->fdt, dto, g.nx / 2, sets + i, m, c->sp, c->sp * g.ny, ncols, g.ny, g.ld, plane_el(c), c->s,
+                   ikx, cst));
+    prof_end(c, LP_K_ROW_C2R, bytes);
+  }
   return LP_OK;
 }
-// column map on small spectra: in -> nout outputs (same grid)
-static int col_small(lp_ctx *c, const void *in, int nlev, int fwd, int inv, int nout, ColOut *o, int ncols = 0) {
+// column map on small spectra (same grid)
+static int col_sets(lp_ctx *c, const ColSet *sets, int n, int fwd, int inv, const SpecTables *tab = nullptr) {
   const lp_grid &g = c->g;
   const long ps = c->sp * g.ny;
-  if (ncols <= 0) ncols = g.lh;
-  const LaunchEv ev = prof_attach(c, LP_K_COL_OP);
-  HIPCHK(col_op(c->fdt, g.ny, g.ny, 0, fwd, inv, in, c->sp, ps, ncols, nlev, nout, o, c->sp, ps, c->tab, c->s,
-                ev));
-  prof_attached(c, ev, bytes_col(g.ny, g.ny, ncols, nlev, nout, esz_of(c->fdt)));
+  for (int i = 0; i < n; i += c->group) {
+    const int m = n - i < c->group ? n - i : c->group;
+    double bytes = 0;
+    for (int f = i; f < i + m; ++f) bytes += bytes_col(g.ny, g.ny, g.lh, sets[f].nplanes, sets[f].nout, esz_of(c->fdt));
+    const LaunchEv ev = prof_attach(c, LP_K_COL_OP);
+    HIPCHK(col_op(c->fdt, g.ny, g.ny, 0, fwd, inv, sets + i, m, c->sp, ps, g.lh, c->sp, ps, tab ? *tab : c->tab, c->s,
+                  ev));
+    prof_attached(c, ev, bytes);
+  }
   return LP_OK;
 }
 
-// one input field -> derivative / filter outputs (multipliers), each output real field
-static int spectral_apply(lp_ctx *c, const void *f, int nlev, double scale, int nout, const int *mults,
-                          void *const *outs, RowIn ri = {}) {
-  RCHK(r2c_small(c, f, nlev, scale, c->spec[0], 0, ri));
-  ColOut o[3];
-  for (int j = 0; j < nout; ++j) o[j] = ColOut{c->spec[j], mults[j]};
-  RCHK(col_small(c, c->spec[0], nlev, 1, 1, nout, o));
-  for (int j = 0; j < nout; ++j) RCHK(c2r_small(c, c->spec[j], c->g.lh, nlev, outs[j], c->fdt));
+// one input field -> up to 3 derivative / filter outputs (multipliers), each a real field.
+// n fields of the same type; field f's spectra live in spec[f][0..nout-1], its input's in
+// spec[f][0]
+struct ApplyField {
+  const void *in;
+  int nlev;
+  double scale;
+  int nout;
+  int mult[3];
+  void *out[3];
+  void *spec[3];
+};
+static int spectral_apply(lp_ctx *c, const ApplyField *F, int n, Dt din, const SpecTables *tab = nullptr) {
+  for (int i = 0; i < n; i += c->group) {
+    const int m = n - i < c->group ? n - i : c->group;
+    R2cSet r[kMaxSets];
+    ColSet k[kMaxSets];
+    C2rSet o[3 * kMaxSets];
+    int no = 0;
+    for (int f = 0; f < m; ++f) {
+      const ApplyField &a = F[i + f];
+      r[f] = R2cSet{a.in, a.spec[0], a.nlev, a.scale};
+      k[f] = ColSet{a.spec[0], a.nlev, a.nout, {}};
+      for (int j = 0; j < a.nout; ++j) {
+        k[f].outs[j] = ColOut{a.spec[j], a.mult[j]};
+        o[no++] = C2rSet{a.spec[j], a.out[j], a.nlev};
+      }
+    }
+    RCHK(r2c_sets(c, r, m, din));
+    RCHK(col_sets(c, k, m, 1, 1, tab));
+    RCHK(c2r_sets(c, o, no, c->g.lh, c->fdt));
+  }
   return LP_OK;
 }
 
-// dealias1.f90: small field -> 3/2-grid physical field
-static int to_big(lp_ctx *c, const void *f, int nlev, void *out_big, RowIn ri = {}) {
+// dealias1.f90: small fields of nlev levels -> 3/2-grid physical fields (at most 3 at a time)
+static int to_big(lp_ctx *c, const void *const *f, int n, int nlev, void *const *out_big, Dt din) {
   const lp_grid &g = c->g;
-  double cst = 1.0 / ((double)g.nx * g.ny);
-  RCHK(r2c_small(c, f, nlev, cst, c->spec[0], 0, ri));
-  ColOut o{c->specb[0], M_ONE};
-  const long ps = c->sp * g.ny, pb = c->sb * g.ny2;
-  HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 1, 1, c->spec[0], c->sp, ps, g.nx / 2, nlev, 1, &o, c->sb, pb,
-                c->tab, c->s));
-  HIPCHK(row_c2r(c->fdt, c->fdt, g.nx2 / 2, c->specb[0], c->sb, pb, g.nx / 2, g.ny2, nlev, out_big,
-                 g.ld_big, (long)g.ld_big * g.ny2, c->s));
+  const double cst = 1.0 / ((double)g.nx * g.ny);
+  const long ps = c->sp * g.ny, pb = c->cv_pitch * g.ny2;
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < n; i += gr) {
+    const int m = n - i < gr ? n - i : gr;
+    R2cSet r[3];
+    ColSet k[3];
+    C2rSet o[3];
+    for (int q = 0; q < m; ++q) {
+      r[q] = R2cSet{f[i + q], c->spec[q], nlev, cst};
+      k[q] = ColSet{c->spec[q], nlev, 1, {ColOut{c->specb[q], M_ONE}}};
+      o[q] = C2rSet{c->specb[q], out_big[i + q], nlev};
+    }
+    RCHK(r2c_sets(c, r, m, din));
+    HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 1, 1, k, m, c->sp, ps, g.nx / 2, c->cv_pitch, pb, c->tab, c->s));
+    HIPCHK(row_c2r(c->fdt, c->fdt, g.nx2 / 2, o, m, c->cv_pitch, pb, g.nx / 2, g.ny2, g.ld_big,
+                   (long)g.ld_big * g.ny2, c->s));
+  }
   return LP_OK;
 }
 
-// dealias2.f90 core / convec.f90:161-170: 3/2-grid field (already scaled) -> small field
-static int from_big(lp_ctx *c, const void *fb, int nlev, double scale, void *out) {
+// dealias2.f90 core / convec.f90:161-170: 3/2-grid fields (already scaled) -> small fields
+static int from_big(lp_ctx *c, const void *const *fb, int n, int nlev, double scale, void *const *out) {
   const lp_grid &g = c->g;
-  const long pb = c->sb * g.ny2, ps = c->sp * g.ny;
-  HIPCHK(row_r2c(c->fdt, g.nx2 / 2, fb, g.ld_big, (long)g.ld_big * g.ny2, g.ny2, nlev, scale, c->specb[1],
-                 c->sb, pb, g.nx / 2, c->s));
-  ColOut o{c->spec[1], M_ONE};
-  HIPCHK(col_op(c->fdt, g.ny2, g.ny, 2, 1, 1, c->specb[1], c->sb, pb, g.nx / 2, nlev, 1, &o, c->sp, ps,
-                c->tab, c->s));
-  RCHK(c2r_small(c, c->spec[1], g.nx / 2, nlev, out, c->fdt));
+  const long pb = c->cv_pitch * g.ny2, ps = c->sp * g.ny;
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < n; i += gr) {
+    const int m = n - i < gr ? n - i : gr;
+    R2cSet r[3];
+    ColSet k[3];
+    C2rSet o[3];
+    for (int q = 0; q < m; ++q) {
+      r[q] = R2cSet{fb[i + q], c->specb[q], nlev, scale};
+      k[q] = ColSet{c->specb[q], nlev, 1, {ColOut{c->spec[q], M_ONE}}};
+      o[q] = C2rSet{c->spec[q], out[i + q], nlev};
+    }
+    HIPCHK(row_r2c(c->fdt, c->fdt, g.nx2 / 2, r, m, g.ld_big, (long)g.ld_big * g.ny2, g.ny2, c->cv_pitch, pb,
+                   g.nx / 2, c->s));
+    HIPCHK(col_op(c->fdt, g.ny2, g.ny, 2, 1, 1, k, m, c->cv_pitch, pb, g.nx / 2, c->sp, ps, c->tab, c->s));
+    RCHK(c2r_sets(c, o, m, g.nx / 2, c->fdt));
+  }
   return LP_OK;
 }
 
@@ -916,40 +984,58 @@ static int from_big(lp_ctx *c, const void *fb, int nlev, double scale, void *out
 // transform less their first value, recorded in shift[plane] and added back to the
 // filtered f in binary64 (filt_da(f - s) + s = filt_da(f), since a constant has only the
 // kx = ky = 0 mode).  keep then holds the spectrum of f - s.
-static int do_filt_da(lp_ctx *c, void *f, void *dfdx, void *dfdy, int nlev, void *keep = nullptr, bool vel = false,
-                      double *shift = nullptr) {
-  double cst = 1.0 / ((double)c->g.nx * c->g.ny);
-  RowIn ri;
-  if (vel) ri.din = F64;
-  if (vel && shift && c->fdt == F32) {
-    ri.shift = true;
-    ri.shift_out = shift;
-  } else {
-    shift = nullptr;
+struct FiltField {
+  void *f, *dfdx, *dfdy;
+  void *keep = nullptr;
+  double *shift = nullptr;
+};
+static int do_filt_da(lp_ctx *c, const FiltField *F, int n, int nlev, bool vel = false) {
+  const double cst = 1.0 / ((double)c->g.nx * c->g.ny);
+  const Dt din = vel ? F64 : c->fdt;
+  const bool mixed = vel && c->fdt == F32;
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < n; i += gr) {
+    const int m = n - i < gr ? n - i : gr;
+    R2cSet r[3];
+    ColSet k[3];
+    C2rSet ox[3], o[6];
+    int no = 0;
+    for (int q = 0; q < m; ++q) {
+      const FiltField &a = F[i + q];
+      void *s0 = a.keep ? a.keep : c->cv_spec[q];
+      r[q] = R2cSet{a.f, s0, nlev, cst};
+      if (mixed && a.shift) {
+        r[q].shift = true;
+        r[q].shift_out = a.shift;
+      }
+      k[q] = ColSet{s0, nlev, 2, {ColOut{s0, M_ONE}, ColOut{c->spec[q], M_IKY}}};
+      ox[q] = C2rSet{s0, a.dfdx, nlev};
+      o[no++] = C2rSet{c->spec[q], a.dfdy, nlev};
+      if (!mixed) o[no++] = C2rSet{s0, a.f, nlev};
+    }
+    RCHK(r2c_sets(c, r, m, din));
+    RCHK(col_sets(c, k, m, 1, 1));
+    if (mixed) {
+      // the filtered velocity in binary64: its oddball modes subtracted exactly (a binary32
+      // round trip would put about 3e-7 of the fluctuations' size back into u, v, w at
+      // every step)
+      Geo g = geo(c);
+      if (g.nx > kNyqMax || g.ny > kNyqMax) return set_err(LP_ERR_ARG, "filt_da: nx, ny above %d", kNyqMax);
+      NyqFields N{};
+      for (int q = 0; q < m; ++q) N.f[q] = (double *)F[i + q].f;
+      N.A = c->nyq;
+      N.B = N.A + 3 * (size_t)c->g.nz * g.ny;
+      N.C = N.B + 3 * (size_t)c->g.nz * g.nx;
+      N.P = c->nyq_part;
+      hipLaunchKernelGGL(k_nyq_part, dim3((unsigned)(nlev * kNyqSlices), (unsigned)m), dim3(256), 0, c->s, N, g);
+      hipLaunchKernelGGL(k_nyq_fin, dim3((unsigned)nlev, (unsigned)m), dim3(256), 0, c->s, N, g);
+      hipLaunchKernelGGL(k_nyq_remove, dim3(grid1(g.np * nlev).x, (unsigned)m), dim3(256), 0, c->s, N, g, nlev);
+      HIPCHK(hipGetLastError());
+    }
+    RCHK(c2r_sets(c, ox, m, c->g.lh, c->fdt, c->kx));
+    RCHK(c2r_sets(c, o, no, c->g.lh, c->fdt));
   }
-  RCHK(r2c_small(c, f, nlev, cst, c->spec[0], 0, ri));
-  void *s0 = keep ? keep : c->spec[0];
-  ColOut o[2] = {{s0, M_ONE}, {c->spec[2], M_IKY}};
-  RCHK(col_small(c, c->spec[0], nlev, 1, 1, 2, o));
-  if (vel && c->fdt == F32) {
-    // the filtered velocity in binary64: its oddball modes subtracted exactly (a binary32
-    // round trip would put about 3e-7 of the fluctuations' size back into u, v, w at
-    // every step)
-    Geo g = geo(c);
-    double *A = c->nyq, *B = A + (size_t)c->g.nz * g.ny, *Cc = B + (size_t)c->g.nz * g.nx;
-    if (g.nx > kNyqMax || g.ny > kNyqMax) return set_err(LP_ERR_ARG, "filt_da: nx, ny above %d", kNyqMax);
-    hipLaunchKernelGGL(k_nyq_part, dim3((unsigned)(nlev * kNyqSlices)), dim3(256), 0, c->s, (const double *)f, A,
-                       c->nyq_part, g);
-    hipLaunchKernelGGL(k_nyq_fin, dim3((unsigned)nlev), dim3(256), 0, c->s, (const double *)A,
-                       (const double *)c->nyq_part, B, Cc, g);
-    hipLaunchKernelGGL(k_nyq_remove, grid1(g.np * nlev), dim3(256), 0, c->s, (double *)f, (const double *)A,
-                       (const double *)B, (const double *)Cc, g, nlev);
-    HIPCHK(hipGetLastError());
-  } else {
-    RCHK(c2r_small(c, s0, c->g.lh, nlev, f, vel ? F64 : c->fdt, nullptr, shift));
-  }
-  RCHK(c2r_small(c, s0, c->g.lh, nlev, dfdx, c->fdt, c->kx));
-  return c2r_small(c, c->spec[2], c->g.lh, nlev, dfdy, c->fdt);
+  return LP_OK;
 }
 
 // vel: f is a binary64 velocity of the context (the difference is formed in binary64)
@@ -989,12 +1075,10 @@ static int do_wallstress(lp_ctx *c) {
     return LP_OK;
   }
   // wallstress.f90:103-104,139-140: test-filtered copies of u(1), v(1)
-  const int m[1] = {M_G1};
-  void *o1[1] = {c->tmp[0]}, *o2[1] = {c->tmp[1]};
-  RowIn vel;
-  vel.din = F64;
-  RCHK(spectral_apply(c, c->f[LP_U], 1, 1.0, 1, m, o1, vel));
-  RCHK(spectral_apply(c, c->f[LP_V], 1, 1.0, 1, m, o2, vel));
+  // (bw, tw: single-plane spectra, free until the pressure solve)
+  const ApplyField wf[2] = {{c->f[LP_U], 1, 1.0, 1, {M_G1}, {c->tmp[0]}, {c->bw}},
+                            {c->f[LP_V], 1, 1.0, 1, {M_G1}, {c->tmp[1]}, {c->tw}}};
+  RCHK(spectral_apply(c, wf, 2, F64));
   double zl = 0.5 * c->g.dz - cf.d0;
   double denom = std::log(zl / cf.z0);  // less psi_m (a plane from obukhov with theta on)
   if (c->frz_ust) {  // frozen coefficient: the base run's u*
@@ -1054,7 +1138,8 @@ static int theta_body(lp_ctx *c) {
   const long nv = g.np * g.nz;
   void *th = c->f[LP_THETA], *dTdx = c->f[LP_DTDX], *dTdy = c->f[LP_DTDY], *dTdz = c->f[LP_DTDZ];
   // :160, 175-178 (theta enters the binary32 transform less each level's first value)
-  RCHK(do_filt_da(c, th, dTdx, dTdy, gg.nz, nullptr, true, c->tshift));
+  const FiltField tf{th, dTdx, dTdy, c->Hs[0], c->tshift};
+  RCHK(do_filt_da(c, &tf, 1, gg.nz, true));
   RCHK(do_ddz_uv(c, dTdz, th, true));
   const size_t fe = esz_of(c->fdt);
   const double top = S.dTdz_top / S.T_scale * S.z_i;
@@ -1067,26 +1152,24 @@ static int theta_body(lp_ctx *c) {
                                      (const double *)c->d_obuk, (T *)dTdz, g, sflux, cf.vonk, gg.dz));
   HIPCHK(hipGetLastError());
   // :808-879 dealias1 of u, v, w, dsdx, dsdy, dsdz; the products; dealias2
-  RowIn vel;
-  vel.din = F64;
   const void *src[6] = {c->f[LP_U], c->f[LP_V], c->f[LP_W], dTdx, dTdy, dTdz};
-  for (int q = 0; q < 6; ++q) RCHK(to_big(c, src[q], gg.nz, c->tbig[q], q < 3 ? vel : RowIn{}));
+  RCHK(to_big(c, src, 3, gg.nz, c->tbig, F64));
+  RCHK(to_big(c, src + 3, 3, gg.nz, c->tbig + 3, c->fdt));
   FDISPATCH(c, T, hipLaunchKernelGGL(k_theta_adv<T>, grid1((long)gg.ld_big * gg.ny2 * gg.nz), dim3(256), 0, c->s,
                                      (T *)c->tbig[0], (const T *)c->tbig[1], (const T *)c->tbig[2],
                                      (const T *)c->tbig[3], (const T *)c->tbig[4], (const T *)c->tbig[5], gg.nx2,
                                      gg.ny2, gg.ld_big, gg.nz));
   HIPCHK(hipGetLastError());
-  RCHK(from_big(c, c->tbig[0], gg.nz, 1.0 / ((double)gg.nx2 * gg.ny2), c->f[LP_RHS_T]));
+  RCHK(from_big(c, c->tbig, 1, gg.nz, 1.0 / ((double)gg.nx2 * gg.ny2), &c->f[LP_RHS_T]));
   // :889-1060 the SGS flux divergence
   const double inv = 1.0 / S.Pr;
   FDISPATCH(c, T, hipLaunchKernelGGL(k_theta_flux_xy<T>, grid1(nv), dim3(256), 0, c->s, (const T *)c->f[LP_NU_T],
                                      (const T *)dTdx, (const T *)dTdy, (T *)c->tmp[0], (T *)c->tmp[1], g, inv));
   HIPCHK(hipGetLastError());
   const double cst = 1.0 / ((double)gg.nx * gg.ny);
-  const int mx[1] = {M_IKX}, my[1] = {M_IKY};
-  void *ox[1] = {c->tmp[2]}, *oy[1] = {c->tmp[3]};
-  RCHK(spectral_apply(c, c->tmp[0], gg.nz, cst, 1, mx, ox));
-  RCHK(spectral_apply(c, c->tmp[1], gg.nz, cst, 1, my, oy));
+  const ApplyField ff[2] = {{c->tmp[0], gg.nz, cst, 1, {M_IKX}, {c->tmp[2]}, {c->spec[0]}},
+                            {c->tmp[1], gg.nz, cst, 1, {M_IKY}, {c->tmp[3]}, {c->spec[1]}}};
+  RCHK(spectral_apply(c, ff, 2, c->fdt));
   FDISPATCH(c, T, hipLaunchKernelGGL(k_theta_flux_z<T>, grid1(nv), dim3(256), 0, c->s, (const T *)c->f[LP_NU_T],
                                      (const T *)dTdz, (T *)c->tmp[0], (double *)c->f[LP_SGS_T3], g, inv, sflux));
   HIPCHK(hipGetLastError());
@@ -1195,21 +1278,18 @@ static int do_lagrange(lp_ctx *c, bool use_u = false) {
   // :157-256 the y part of both test filters, all 21 fields in one pass
   {
     const long ps = pc * gg.ny;
-    ColOut o[2] = {{c->lbar, M_G1, p1, p1 * gg.ny, n1}, {c->lhat, M_G2, p2, p2 * gg.ny, n2}};
+    ColSet set{c->lspec, kNumLag * gg.nz, 2, {{c->lbar, M_G1, p1, p1 * gg.ny, n1}, {c->lhat, M_G2, p2, p2 * gg.ny, n2}}};
     // full groups of TX columns in the block-wide pass; one or two trailing columns (nx =
     // 256: the kx = 64 column that G_test keeps by rounding) one column per block
     const int tx = c->fdt == F64 ? 8 : 16;
     const int nmain = (nc % tx <= 2 && nc > tx) ? nc / tx * tx : nc;
     // not in the column-pass class: in a step this launch shares the GPU with convec
-    HIPCHK(col_op(c->fdt, gg.ny, gg.ny, 0, 1, 1, c->lspec, pc, ps, nmain, kNumLag * gg.nz, 2, o, pc, ps, c->tab,
-                  c->s));
+    HIPCHK(col_op(c->fdt, gg.ny, gg.ny, 0, 1, 1, &set, 1, pc, ps, nmain, pc, ps, c->tab, c->s));
     if (nmain < nc) {
-      ColOut ot[2];
-      int nt = 0;
-      if (nmain < n1) ot[nt++] = o[0];
-      if (nmain < n2) ot[nt++] = o[1];
-      HIPCHK(col_op_tail(c->fdt, gg.ny, c->lspec, pc, ps, nmain, nc, kNumLag * gg.nz, nt, ot, pc, ps, c->tab,
-                         c->s));
+      ColSet tail{c->lspec, kNumLag * gg.nz, 0, {}};
+      if (nmain < n1) tail.outs[tail.nout++] = set.outs[0];
+      if (nmain < n2) tail.outs[tail.nout++] = set.outs[1];
+      HIPCHK(col_op_tail(c->fdt, gg.ny, tail, pc, ps, nmain, nc, pc, ps, c->tab, c->s));
     }
   }
   RCHK(fork_convec(c));  // in a step: convec overlaps the rest of the model
@@ -1268,23 +1348,33 @@ static int do_dynamic_alt(lp_ctx *c) {
   HIPCHK(hipGetLastError());
   // the test filters (G_test, G_test_test carry the 1/(nx ny) of the transform)
   DynVol B{}, H{};
+  void *sp_[5] = {c->spec[0], c->spec[1], c->spec[2], c->spec[3], c->Hs[0]};  // free until divstress
+  ApplyField A[kDynIn];
   for (int q = 0; q < kDynIn; ++q) {
-    const void *src = (q >= 9 && q < 15) ? c->S[q - 9] : vol(c->dyn_in, q);
     const bool hat = model == 3 && !(q >= 3 && q < 9);
-    const int m[2] = {M_G1, M_G2};
-    void *o[2] = {vol(c->dyn_bar, q), hat ? vol(c->dyn_hat, q) : nullptr};
-    RCHK(spectral_apply(c, src, gg.nz, 1.0, hat ? 2 : 1, m, o));
+    A[q] = ApplyField{(q >= 9 && q < 15) ? c->S[q - 9] : vol(c->dyn_in, q), gg.nz, 1.0, hat ? 2 : 1, {M_G1, M_G2},
+                      {vol(c->dyn_bar, q), hat ? vol(c->dyn_hat, q) : nullptr}, {}};
     B.p[q] = vol(c->dyn_bar, q);
     if (model == 3) H.p[q] = vol(c->dyn_hat, q);
+  }
+  // two fields at a time (each takes up to two of the five spectra)
+  for (int q = 0; q < kDynIn; q += 2) {
+    const int m = kDynIn - q < 2 ? 1 : 2;
+    for (int j = 0; j < m; ++j) {
+      A[q + j].spec[0] = sp_[2 * j];
+      A[q + j].spec[1] = sp_[2 * j + 1];
+    }
+    RCHK(spectral_apply(c, A + q, m, c->fdt));
   }
   if (model == 3) {  // Q_ij: the 2-delta velocities' products, 4-delta filtered (input slots 3-8)
     FDISPATCH(c, T, hipLaunchKernelGGL(k_dyn_qprod<T>, grid1(nv), dim3(256), 0, c->s, (const T *)B.p[0],
                                        (const T *)B.p[1], (const T *)B.p[2], (T *)vol(c->dyn_in, 3), nv));
     HIPCHK(hipGetLastError());
-    for (int q = 3; q < 9; ++q) {
-      const int m[1] = {M_G2};
-      void *o[1] = {vol(c->dyn_hat, q)};
-      RCHK(spectral_apply(c, vol(c->dyn_in, q), gg.nz, 1.0, 1, m, o));
+    for (int q = 3; q < 9; q += 3) {
+      ApplyField Q[3];
+      for (int j = 0; j < 3; ++j)
+        Q[j] = ApplyField{vol(c->dyn_in, q + j), gg.nz, 1.0, 1, {M_G2}, {vol(c->dyn_hat, q + j)}, {sp_[j]}};
+      RCHK(spectral_apply(c, Q, 3, c->fdt));
     }
     FDISPATCH(c, T, hipLaunchKernelGGL(k_dyn_sums<T>, dim3(gg.nz), dim3(1024), 0, c->s, B, H, g, c->dyn_sums));
     hipLaunchKernelGGL(k_dyn_beta, grid1(gg.nz), dim3(256), 0, c->s, (const double *)c->dyn_sums, c->dyn_beta,
@@ -1400,58 +1490,77 @@ static int do_sgs_stag(lp_ctx *c) {
 // divstress_uv.f90:31-127 / divstress_w.f90:31-82 from the x-spectra of tx and ty: the
 // x- and y-derivatives summed in spectral space (col_div), the z-derivative of tz added
 // in the back-transform
-static int divstress_from_spectra(lp_ctx *c, void *divt, const void *sx, const void *sy, const void *tz,
-                                  int is_w, void *work) {
+struct DivField {
+  const void *sx, *sy, *tz;
+  void *work, *divt;
+  int is_w;
+};
+static int divstress_from_spectra(lp_ctx *c, const DivField *F, int n) {
   const lp_grid &g = c->g;
   const long ps = c->sp * g.ny;
   const size_t fe = esz_of(c->fdt);
-  prof_begin(c, LP_K_COL_DIV);
-  HIPCHK(col_div(c->fdt, g.ny, sx, sy, c->sp, ps, g.lh, g.nz, work, c->tab, c->s));
-  prof_end(c, LP_K_COL_DIV, 3.0 * g.lh * g.ny * g.nz * 2 * fe);
-  prof_begin(c, LP_K_ROW_C2R);
-  HIPCHK(row_c2r_div(c->fdt, g.nx / 2, work, c->sp, ps, g.lh, g.ny, g.nz, divt, g.ld, plane_el(c), tz,
-                     1.0 / g.dz, is_w, c->s));
-  prof_end(c, LP_K_ROW_C2R, bytes_c2r(g.nx, g.ny, g.nz, g.lh, fe, fe) + (double)g.ld * g.ny * g.nz * fe);
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < n; i += gr) {
+    const int m = n - i < gr ? n - i : gr;
+    DivSet d[3];
+    C2rSet o[3];
+    for (int q = 0; q < m; ++q) {
+      const DivField &a = F[i + q];
+      d[q] = DivSet{a.sx, a.sy, a.work};
+      o[q] = C2rSet{a.work, a.divt, g.nz, nullptr, a.tz, a.is_w ? 2 : 1};
+    }
+    prof_begin(c, LP_K_COL_DIV);
+    HIPCHK(col_div(c->fdt, g.ny, d, m, g.nz, c->sp, ps, g.lh, c->tab, c->s));
+    prof_end(c, LP_K_COL_DIV, 3.0 * m * g.lh * g.ny * g.nz * 2 * fe);
+    RCHK(c2r_sets(c, o, m, g.lh, c->fdt, nullptr, 1.0 / g.dz));
+  }
   return LP_OK;
 }
 
 static int do_divstress(lp_ctx *c, void *divt, const void *tx, const void *ty, const void *tz, int is_w) {
   const lp_grid &gg = c->g;
   const double cst = 1.0 / ((double)gg.nx * gg.ny);
-  RCHK(r2c_small(c, tx, gg.nz, cst, c->spec[0]));
-  RCHK(r2c_small(c, ty, gg.nz, cst, c->spec[1]));
-  return divstress_from_spectra(c, divt, c->spec[0], c->spec[1], tz, is_w, c->spec[2]);
+  const R2cSet r[2] = {{tx, c->spec[0], gg.nz, cst}, {ty, c->spec[1], gg.nz, cst}};
+  RCHK(r2c_sets(c, r, 2, c->fdt));
+  const DivField d{c->spec[0], c->spec[1], tz, c->spec[2], divt, is_w};
+  return divstress_from_spectra(c, &d, 1);
 }
 
-// main.f90:394-397: the three divergences; txy, txz and tyz are transformed once
+// main.f90:394-397: the three divergences; txy, txz and tyz are transformed once.  A
+// divergence's spectrum goes over the one of its inputs that no other reads.
 static int do_divstress_all(lp_ctx *c) {
   const lp_grid &gg = c->g;
   const double cst = 1.0 / ((double)gg.nx * gg.ny);
   void *sxx = c->spec[0], *sxy = c->spec[1], *syy = c->spec[2], *sxz = c->spec[3], *syz = c->Hs[0];
-  void *work = c->Hs[1];
-  RCHK(r2c_small(c, c->f[LP_TXX], gg.nz, cst, sxx));
-  RCHK(r2c_small(c, c->f[LP_TXY], gg.nz, cst, sxy));
-  RCHK(r2c_small(c, c->f[LP_TYY], gg.nz, cst, syy));
-  RCHK(r2c_small(c, c->f[LP_TXZ], gg.nz, cst, sxz));
-  RCHK(r2c_small(c, c->f[LP_TYZ], gg.nz, cst, syz));
-  RCHK(divstress_from_spectra(c, c->f[LP_DIVTX], sxx, sxy, c->f[LP_TXZ], 0, work));
-  RCHK(divstress_from_spectra(c, c->f[LP_DIVTY], sxy, syy, c->f[LP_TYZ], 0, work));
-  RCHK(divstress_from_spectra(c, c->f[LP_DIVTZ], sxz, syz, c->f[LP_TZZ], 1, work));
-  return LP_OK;
+  const R2cSet r[5] = {{c->f[LP_TXX], sxx, gg.nz, cst}, {c->f[LP_TXY], sxy, gg.nz, cst},
+                       {c->f[LP_TYY], syy, gg.nz, cst}, {c->f[LP_TXZ], sxz, gg.nz, cst},
+                       {c->f[LP_TYZ], syz, gg.nz, cst}};
+  RCHK(r2c_sets(c, r, 5, c->fdt));
+  const DivField d[3] = {{sxx, sxy, c->f[LP_TXZ], sxx, c->f[LP_DIVTX], 0},
+                         {sxy, syy, c->f[LP_TYZ], syy, c->f[LP_DIVTY], 0},
+                         {sxz, syz, c->f[LP_TZZ], sxz, c->f[LP_DIVTZ], 1}};
+  return divstress_from_spectra(c, d, 3);
 }
 
-// dealias1.f90 from the x-spectrum on: the column pass that pads it to ny2 and transforms
-// it back along y, into field q of c->cvb; scale multiplies the padded spectrum
-static int pad_y(lp_ctx *c, const void *spec, int q, double scale = 1.0) {
+// dealias1.f90 from the x-spectra on: the column pass that pads them to ny2 and transforms
+// them back along y, into fields q0.. of c->cvb; scale multiplies the padded spectra, dc (per
+// field, optional) is added to each plane's mean first
+static int pad_y(lp_ctx *c, void *const *spec, int q0, int n, double scale, const double *const *dc) {
   const lp_grid &g = c->g;
   const long ps = c->sp * g.ny, pb = c->cv_pitch * g.ny2;
   const size_t fe = esz_of(c->fdt);
-  ColOut o{(char *)c->cvb + (size_t)q * pb * g.nz * 2 * fe, M_ONE};
-  o.scale = scale;
-  prof_begin(c, LP_K_COL_PAD);
-  HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 1, 1, spec, c->sp, ps, g.nx / 2, g.nz, 1, &o, c->cv_pitch, pb, c->tab,
-                c->s));
-  prof_end(c, LP_K_COL_PAD, bytes_col(g.ny, g.ny2, g.nx / 2, g.nz, 1, fe));
+  for (int i = 0; i < n; i += c->group) {
+    const int m = n - i < c->group ? n - i : c->group;
+    ColSet k[kMaxSets];
+    for (int q = 0; q < m; ++q) {
+      k[q] = ColSet{spec[i + q], g.nz, 1, {ColOut{(char *)c->cvb + (size_t)(q0 + i + q) * pb * g.nz * 2 * fe, M_ONE}}};
+      k[q].outs[0].scale = scale;
+      k[q].dc = dc ? dc[i + q] : nullptr;
+    }
+    prof_begin(c, LP_K_COL_PAD);
+    HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 1, 1, k, m, c->sp, ps, g.nx / 2, c->cv_pitch, pb, c->tab, c->s));
+    prof_end(c, LP_K_COL_PAD, m * bytes_col(g.ny, g.ny2, g.nx / 2, g.nz, 1, fe));
+  }
   return LP_OK;
 }
 
@@ -1464,27 +1573,29 @@ static int do_convec(lp_ctx *c, bool kept) {
   const double cst = 1.0 / ((double)gg.nx * gg.ny);
   // convec.f90:76-98
   const int vel[3] = {LP_U, LP_V, LP_W};
-  RowIn vin;
-  vin.din = F64;
-  for (int q = 0; q < 3; ++q) {
-    if (!kept) RCHK(r2c_small(c, c->f[vel[q]], gg.nz, cst, c->uvw_spec[q], 0, vin));
-    if (kept && c->fdt == F32 && q < 2) {
-      // filt_da transformed u - s, v - s: the row means (kx = 0 column) get s back
-      hipLaunchKernelGGL(k_add_dc<float>, grid1((long)gg.ny * gg.nz), dim3(256), 0, c->s, (cx<float> *)c->uvw_spec[q],
-                         c->sp, gg.ny, gg.nz, (const double *)(c->ushift + (size_t)q * gg.nz));
-      HIPCHK(hipGetLastError());
-    }
-    // filt_da's spectrum went through an unnormalised y round trip: ny times the r2c
-    RCHK(pad_y(c, c->uvw_spec[q], q, kept ? 1.0 / gg.ny : 1.0));
+  if (!kept) {
+    R2cSet r[3];
+    for (int q = 0; q < 3; ++q) r[q] = R2cSet{c->f[vel[q]], c->uvw_spec[q], gg.nz, cst};
+    RCHK(r2c_sets(c, r, 3, F64));
   }
+  // in a binary32 context filt_da transformed u - s, v - s: the row means (kx = 0 column) get s
+  // back; filt_da's spectrum went through an unnormalised y round trip: ny times the r2c
+  const bool back = kept && c->fdt == F32;
+  const double *dc[3] = {back ? c->ushift : nullptr, back ? c->ushift + gg.nz : nullptr, nullptr};
+  RCHK(pad_y(c, c->uvw_spec, 0, 3, kept ? 1.0 / gg.ny : 1.0, dc));
   // convec.f90:100-133: each vorticity component formed inside its x transform
   const int va[3] = {LP_DWDY, LP_DWDX, LP_DVDX}, vb[3] = {LP_DVDZ, LP_DUDZ, LP_DUDY};
-  for (int q = 0; q < 3; ++q) {
-    prof_begin(c, LP_K_ROW_R2C);
-    HIPCHK(row_r2c_vort(c->fdt, gg.nx / 2, q, c->f[va[q]], c->f[vb[q]], gg.ld, plane_el(c), gg.ny, gg.nz, cst,
-                        c->cv_spec[0], c->sp, c->sp * gg.ny, gg.nx / 2, c->s));
-    prof_end(c, LP_K_ROW_R2C, bytes_r2c(gg.nx, gg.ny, gg.nz, gg.nx / 2, fe) + (double)vol_el(c) * fe);
-    RCHK(pad_y(c, c->cv_spec[0], 3 + q));
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < 3; i += gr) {
+    const int m = 3 - i < gr ? 3 - i : gr;
+    R2cSet r[3];
+    for (int q = 0; q < m; ++q) {
+      r[q] = R2cSet{c->f[va[i + q]], c->cv_spec[q], gg.nz, cst};
+      r[q].b = c->f[vb[i + q]];
+      r[q].comp = i + q;
+    }
+    RCHK(r2c_sets(c, r, m, c->fdt));
+    RCHK(pad_y(c, c->cv_spec, 3 + i, m, 1.0, nullptr));
   }
   // convec.f90:140-158, 180-221, 241-279 products (normalisation folded in) between the
   // x back- and forward transforms of the 3/2 grid, kx < nx/2 kept (dealias2)
@@ -1497,20 +1608,27 @@ static int do_convec(lp_ctx *c, bool kept) {
   // convec.f90:161-170, 227-236, 286-296: unpadd along y, c2r small
   void *outs[3] = {c->f[LP_RHSX], c->f[LP_RHSY], c->f[LP_RHSZ]};
   const long ps = c->sp * gg.ny;
-  for (int q = 0; q < 3; ++q) {
-    ColOut o{c->cv_spec[1], M_ONE};
+  for (int i = 0; i < 3; i += gr) {
+    const int m = 3 - i < gr ? 3 - i : gr;
+    ColSet k[3];
+    C2rSet o[3];
+    for (int q = 0; q < m; ++q) {
+      k[q] = ColSet{(const char *)c->cvp + (size_t)(i + q) * pb * gg.nz * 2 * fe, gg.nz - 1, 1,
+                    {ColOut{c->cv_spec[q], M_ONE}}};
+      o[q] = C2rSet{c->cv_spec[q], outs[i + q], gg.nz - 1};
+    }
     prof_begin(c, LP_K_COL_PAD);
-    HIPCHK(col_op(c->fdt, gg.ny2, gg.ny, 2, 1, 1, (const char *)c->cvp + (size_t)q * pb * gg.nz * 2 * fe,
-                  c->cv_pitch, pb, gg.nx / 2, gg.nz - 1, 1, &o, c->sp, ps, c->tab, c->s));
-    prof_end(c, LP_K_COL_PAD, bytes_col(gg.ny2, gg.ny, gg.nx / 2, gg.nz - 1, 1, fe));
-    RCHK(c2r_small(c, c->cv_spec[1], gg.nx / 2, gg.nz - 1, outs[q], c->fdt));
+    HIPCHK(col_op(c->fdt, gg.ny2, gg.ny, 2, 1, 1, k, m, c->cv_pitch, pb, gg.nx / 2, c->sp, ps, c->tab, c->s));
+    prof_end(c, LP_K_COL_PAD, m * bytes_col(gg.ny2, gg.ny, gg.nx / 2, gg.nz - 1, 1, fe));
+    RCHK(c2r_sets(c, o, m, gg.nx / 2, c->fdt));
   }
   // convec.f90:306-308 top level BOGUS
-  for (int q = 0; q < 3; ++q) {
-    FDISPATCH(c, T, hipLaunchKernelGGL(k_fill<T>, grid1(g.np), dim3(256), 0, c->s,
-                                       (T *)outs[q] + (long)(gg.nz - 1) * g.np, g.np, (T)LP_BOGUS));
-    HIPCHK(hipGetLastError());
-  }
+  FDISPATCH(c, T, {
+    Fill3<T> F{};
+    for (int q = 0; q < 3; ++q) F.p[q] = (T *)outs[q] + (long)(gg.nz - 1) * g.np;
+    hipLaunchKernelGGL(k_fill3<T>, dim3(grid1(g.np).x, 3), dim3(256), 0, c->s, F, g.np, (T)LP_BOGUS);
+  });
+  HIPCHK(hipGetLastError());
   return LP_OK;
 }
 
@@ -1527,21 +1645,15 @@ static int do_press(lp_ctx *c) {
   // transforms.  A zero pivot sets d_err, which check_err_flag reads and clears, so the
   // flag of every step of an lp_step call is reported.
   auto side = [&]() -> int {
-    RCHK(r2c_small(c, c->f[LP_DIVTZ], 1, cst, c->bw));
-    ColOut ob{c->bw, M_ONE};
-    RCHK(col_small(c, c->bw, 1, 1, 0, 1, &ob));
     const char *divtz_top = (const char *)c->f[LP_DIVTZ] + (size_t)(gg.nz - 1) * np * esz_of(c->fdt);
-    RCHK(r2c_small(c, divtz_top, 1, cst, c->tw));
-    ColOut ot{c->tw, M_ONE};
-    RCHK(col_small(c, c->tw, 1, 1, 0, 1, &ot));
-    hipLaunchKernelGGL(k_fill<double>, grid1(np), dim3(256), 0, c->s, (double *)c->f[LP_P] + (long)gg.nz * np, np,
-                       LP_BOGUS);
-    FDISPATCH(c, T, {
-      hipLaunchKernelGGL(k_fill<T>, grid1(np), dim3(256), 0, c->s, (T *)c->f[LP_DPDX] + (long)(gg.nz - 1) * np,
-                         np, (T)LP_BOGUS);
-      hipLaunchKernelGGL(k_fill<T>, grid1(np), dim3(256), 0, c->s, (T *)c->f[LP_DPDY] + (long)(gg.nz - 1) * np,
-                         np, (T)LP_BOGUS);
-    });
+    const R2cSet r[2] = {{c->f[LP_DIVTZ], c->bw, 1, cst}, {divtz_top, c->tw, 1, cst}};
+    RCHK(r2c_sets(c, r, 2, c->fdt));
+    const ColSet k[2] = {{c->bw, 1, 1, {{c->bw, M_ONE}}}, {c->tw, 1, 1, {{c->tw, M_ONE}}}};
+    RCHK(col_sets(c, k, 2, 1, 0));
+    FDISPATCH(c, T, hipLaunchKernelGGL(k_press_tops<T>, grid1(np), dim3(256), 0, c->s,
+                                       (double *)c->f[LP_P] + (long)gg.nz * np,
+                                       (T *)c->f[LP_DPDX] + (long)(gg.nz - 1) * np,
+                                       (T *)c->f[LP_DPDY] + (long)(gg.nz - 1) * np, np));
     HIPCHK(hipGetLastError());
     return LP_OK;
   };
@@ -1560,13 +1672,18 @@ static int do_press(lp_ctx *c) {
   // (the mean mode integrates H_z and the wall / lid rows), and it keeps the mean flow's
   // magnitude out of the transforms' rounding.
   const int fid[3] = {LP_U, LP_V, LP_W};
-  for (int q = 0; q < 3; ++q) {
-    RowIn ri;
-    ri.din = F64;
-    ri.shift = c->fdt == F32 && q < 2;
-    RCHK(r2c_small(c, c->f[fid[q]], gg.nz - 1, cst / tadv1 / cf.dt, c->Hs[q], 0, ri));
-    ColOut o{c->Hs[q], M_ONE};
-    RCHK(col_small(c, c->Hs[q], gg.nz - 1, 1, 0, 1, &o));
+  const int gr = c->group < 3 ? c->group : 3;
+  for (int i = 0; i < 3; i += gr) {
+    const int m = 3 - i < gr ? 3 - i : gr;
+    R2cSet r[3];
+    ColSet k[3];
+    for (int q = 0; q < m; ++q) {
+      r[q] = R2cSet{c->f[fid[i + q]], c->Hs[i + q], gg.nz - 1, cst / tadv1 / cf.dt};
+      r[q].shift = c->fdt == F32 && i + q < 2;
+      k[q] = ColSet{c->Hs[i + q], gg.nz - 1, 1, {{c->Hs[i + q], M_ONE}}};
+    }
+    RCHK(r2c_sets(c, r, m, F64));
+    RCHK(col_sets(c, k, m, 1, 0));
   }
   // :149-329 + tridag_array
   HIPCHK(hipStreamWaitEvent(c->s, c->ev_aux, 0));
@@ -1593,16 +1710,17 @@ static int do_press(lp_ctx *c) {
   // :339-352 inverse transforms in binary64: p(0..nz-1), dpdx, dpdy (1..nz-1); dpdx is
   // the back-transform of p's (kx, y) spectrum times i kx (kx is uniform along a column)
   {
-    ColOut o[2] = {{c->pspec[0], M_ONE}, {c->pspec[2], M_IKY}};
-    HIPCHK(col_op(F64, gg.ny, gg.ny, 0, 0, 1, ph, c->sp, ps, gg.lh, gg.nz, 2, o, c->sp, ps, c->tab, c->s));
+    const ColSet k{ph, gg.nz, 2, {{c->pspec[0], M_ONE}, {c->pspec[2], M_IKY}}};
+    HIPCHK(col_op(F64, gg.ny, gg.ny, 0, 0, 1, &k, 1, c->sp, ps, gg.lh, c->sp, ps, c->tab, c->s));
   }
-  HIPCHK(row_c2r(F64, F64, gg.nx / 2, c->pspec[0], c->sp, ps, gg.lh, gg.ny, gg.nz, c->f[LP_P], gg.ld, np,
-                 c->s));
-  Dt dto = c->fdt;
-  HIPCHK(row_c2r(F64, dto, gg.nx / 2, (const cx<double> *)c->pspec[0] + ps, c->sp, ps, gg.lh, gg.ny,
-                 gg.nz - 1, c->f[LP_DPDX], gg.ld, np, c->s, c->kx));
-  HIPCHK(row_c2r(F64, dto, gg.nx / 2, (const cx<double> *)c->pspec[2] + ps, c->sp, ps, gg.lh, gg.ny,
-                 gg.nz - 1, c->f[LP_DPDY], gg.ld, np, c->s));
+  const C2rSet op[2] = {{c->pspec[0], c->f[LP_P], gg.nz},
+                        {(const cx<double> *)c->pspec[2] + ps, c->f[LP_DPDY], gg.nz - 1}};
+  const C2rSet ox{(const cx<double> *)c->pspec[0] + ps, c->f[LP_DPDX], gg.nz - 1};
+  const Dt dto = c->fdt;
+  const int both = dto == F64 && c->group >= 2 ? 2 : 1;  // p and dpdy of one type: one launch
+  HIPCHK(row_c2r(F64, F64, gg.nx / 2, op, both, c->sp, ps, gg.lh, gg.ny, gg.ld, np, c->s));
+  HIPCHK(row_c2r(F64, dto, gg.nx / 2, &ox, 1, c->sp, ps, gg.lh, gg.ny, gg.ld, np, c->s, c->kx));
+  if (both == 1) HIPCHK(row_c2r(F64, dto, gg.nx / 2, op + 1, 1, c->sp, ps, gg.lh, gg.ny, gg.ld, np, c->s));
   return LP_OK;
 }
 
@@ -1723,9 +1841,9 @@ static int do_ke_dudt(lp_ctx *c) {
                                      (const double *)c->f[LP_U], (const double *)c->f[LP_V],
                                      (const double *)c->f[LP_W], (T *)c->tmp[0], g));
   HIPCHK(hipGetLastError());
-  const int m[2] = {M_IKX, M_IKY};
-  void *outs[2] = {c->tmp[1], c->tmp[2]};
-  RCHK(spectral_apply(c, c->tmp[0], gg.nz, 1.0 / ((double)gg.nx * gg.ny), 2, m, outs));
+  const ApplyField ke{c->tmp[0], gg.nz, 1.0 / ((double)gg.nx * gg.ny), 2, {M_IKX, M_IKY}, {c->tmp[1], c->tmp[2]},
+                      {c->spec[0], c->spec[1]}};
+  RCHK(spectral_apply(c, &ke, 1, c->fdt));
   FDISPATCH(c, T, hipLaunchKernelGGL(k_ke_add<T>, grid1(g.np * (g.nz - 1)), dim3(256), 0, c->s, (T *)c->f[LP_DUDT],
                                      (T *)c->f[LP_DVDT], (T *)c->f[LP_DWDT], (const T *)c->tmp[1],
                                      (const T *)c->tmp[2], (const T *)c->tmp[0], g, (T)(1.0 / gg.dz)));
@@ -1776,9 +1894,10 @@ static int step_body(lp_ctx *c) {
   const bool theta = cf.scal.s_flag != 0;
   if (theta) RCHK(do_obukhov(c));  // :257, from the unfiltered u(1), v(1)
   // :277-279 (u and v enter the binary32 transforms less a per-level value)
-  RCHK(do_filt_da(c, c->f[LP_U], c->f[LP_DUDX], c->f[LP_DUDY], gg.nz, c->uvw_spec[0], true, c->ushift));
-  RCHK(do_filt_da(c, c->f[LP_V], c->f[LP_DVDX], c->f[LP_DVDY], gg.nz, c->uvw_spec[1], true, c->ushift + gg.nz));
-  RCHK(do_filt_da(c, c->f[LP_W], c->f[LP_DWDX], c->f[LP_DWDY], gg.nz, c->uvw_spec[2], true));
+  const FiltField ff[3] = {{c->f[LP_U], c->f[LP_DUDX], c->f[LP_DUDY], c->uvw_spec[0], c->ushift},
+                           {c->f[LP_V], c->f[LP_DVDX], c->f[LP_DVDY], c->uvw_spec[1], c->ushift + gg.nz},
+                           {c->f[LP_W], c->f[LP_DWDX], c->f[LP_DWDY], c->uvw_spec[2]}};
+  RCHK(do_filt_da(c, ff, 3, gg.nz, true));
   // :315 wallstress (level 1 of txz, tyz, dudz, dvdz from the test-filtered u(1), v(1):
   // single-plane passes) on the second stream, beside the z-derivatives of the other levels
   HIPCHK(hipEventRecord(c->ev_aux_fork, c->s));
@@ -1790,9 +1909,11 @@ static int step_body(lp_ctx *c) {
   std::swap(c->s, c->s2);
   RCHK(rc_wall);
   HIPCHK(hipEventRecord(c->ev_aux, c->s2));
-  RCHK(do_ddz_uv(c, c->f[LP_DUDZ], c->f[LP_U], true));  // :284-288 (levels 2..nz-1)
-  RCHK(do_ddz_uv(c, c->f[LP_DVDZ], c->f[LP_V], true));
-  RCHK(do_ddz_w(c, c->f[LP_DWDZ], c->f[LP_W], true));
+  FDISPATCH(c, T, hipLaunchKernelGGL(k_ddz_vel<T>, dim3(grid1(g.np * g.nz).x, 3), dim3(256), 0, c->s,
+                                     (T *)c->f[LP_DUDZ], (T *)c->f[LP_DVDZ], (T *)c->f[LP_DWDZ],
+                                     (const double *)c->f[LP_U], (const double *)c->f[LP_V],
+                                     (const double *)c->f[LP_W], g, 1.0 / gg.dz));  // :284-288 (levels 2..nz-1)
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamWaitEvent(c->s, c->ev_aux, 0));  // sgs_stag reads level 1
   // convec (:419) needs u, v, w, their derivatives and the wall law's level-1 dudz, dvdz
   // only: it starts on the second stream here and overlaps the whole SGS model
@@ -2186,7 +2307,8 @@ extern "C" int lp_spectrum(lp_ctx *c, int32_t field, int32_t bin, double *out) {
   const Dt dt = f64 ? F64 : c->fdt;
   void *spec = f64 ? c->pspec[0] : c->spec[0];  // (nz+1) resp. nz levels of (sp, ny) complex
   const char *in = (const char *)c->f[field] + (size_t)bin * nv * c->esz[field];
-  HIPCHK(row_r2c(dt, nh, in, g.ld, plane_el(c), g.ny, nl, 1.0 / g.nx, spec, c->sp, c->sp * g.ny, nh, c->s));
+  const R2cSet r{in, spec, nl, 1.0 / g.nx};
+  HIPCHK(row_r2c(dt, dt, nh, &r, 1, g.ld, plane_el(c), g.ny, c->sp, c->sp * g.ny, nh, c->s));
   const dim3 grid((nh + 63) / 64, nl);
   if (f64)
     hipLaunchKernelGGL(k_spectrum<double>, grid, dim3(64), 0, c->s, (const double *)spec, c->sp, g.ny, nh,
@@ -2301,7 +2423,8 @@ extern "C" int lp_filt_da(lp_ctx *c, void *f, void *dfdx, void *dfdy, int32_t nl
   RCHK(a.bind(c, f, b, true, true));
   RCHK(x.bind(c, dfdx, b, false, true));
   RCHK(y.bind(c, dfdy, b, false, true));
-  RCHK(do_filt_da(c, a.dev, x.dev, y.dev, nlev));
+  const FiltField ff{a.dev, x.dev, y.dev};
+  RCHK(do_filt_da(c, &ff, 1, nlev));
   return finish_all(c, {&a, &x, &y});
 }
 
@@ -2311,13 +2434,10 @@ static int deriv_entry(lp_ctx *c, void *dfdx, void *dfdy, const void *f, int nle
   size_t b = vbytes(c, nlev);
   Arg a, x, y;
   RCHK(a.bind(c, f, b, true, false));
-  int m[2];
-  void *outs[2];
-  int n = 0;
-  if (dfdx) { RCHK(x.bind(c, dfdx, b, false, true)); m[n] = M_IKX; outs[n++] = x.dev; }
-  if (dfdy) { RCHK(y.bind(c, dfdy, b, false, true)); m[n] = M_IKY; outs[n++] = y.dev; }
-  double cst = 1.0 / ((double)c->g.nx * c->g.ny);
-  RCHK(spectral_apply(c, a.dev, nlev, cst, n, m, outs));
+  ApplyField F{a.dev, nlev, 1.0 / ((double)c->g.nx * c->g.ny), 0, {}, {}, {c->spec[0], c->spec[1]}};
+  if (dfdx) { RCHK(x.bind(c, dfdx, b, false, true)); F.mult[F.nout] = M_IKX; F.out[F.nout++] = x.dev; }
+  if (dfdy) { RCHK(y.bind(c, dfdy, b, false, true)); F.mult[F.nout] = M_IKY; F.out[F.nout++] = y.dev; }
+  RCHK(spectral_apply(c, &F, 1, c->fdt));
   return finish_all(c, {&a, &x, &y});
 }
 extern "C" int lp_ddx(lp_ctx *c, void *dfdx, const void *f, int32_t nlev) {
@@ -2361,9 +2481,8 @@ extern "C" int lp_padd(lp_ctx *c, void *u_big, const void *u, int32_t nplanes) {
   RCHK(a.bind(c, u, (size_t)ps * nplanes * 2 * fe, true, false));
   RCHK(o.bind(c, u_big, (size_t)pb * nplanes * 2 * fe, false, true));
   HIPCHK(hipMemsetAsync(o.dev, 0, o.bytes, c->s));  // padd.f90:12
-  ColOut co{o.dev, M_ONE};
-  HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 0, 0, a.dev, g.lh, ps, g.nx / 2, nplanes, 1, &co, g.lh_big, pb, c->tab,
-                c->s));
+  const ColSet k{a.dev, nplanes, 1, {{o.dev, M_ONE}}};
+  HIPCHK(col_op(c->fdt, g.ny, g.ny2, 1, 0, 0, &k, 1, g.lh, ps, g.nx / 2, g.lh_big, pb, c->tab, c->s));
   return finish_all(c, {&a, &o});
 }
 
@@ -2377,9 +2496,8 @@ extern "C" int lp_unpadd(lp_ctx *c, void *cc, const void *cc_big, int32_t nplane
   RCHK(o.bind(c, cc, (size_t)ps * nplanes * 2 * fe, true, true));
   // unpadd.f90:15-16 zero the Nyquist column and row; the column map writes the rest
   // (kx < nx/2).  The kx = nx/2 column is cleared by a zero-column map.
-  ColOut co{o.dev, M_ONE};
-  HIPCHK(col_op(c->fdt, g.ny2, g.ny, 2, 0, 0, a.dev, g.lh_big, pb, g.nx / 2, nplanes, 1, &co, g.lh, ps, c->tab,
-                c->s));
+  const ColSet k{a.dev, nplanes, 1, {{o.dev, M_ONE}}};
+  HIPCHK(col_op(c->fdt, g.ny2, g.ny, 2, 0, 0, &k, 1, g.lh_big, pb, g.nx / 2, g.lh, ps, c->tab, c->s));
   // Nyquist column jx = nx/2: write zeros via a padmode-0 map of ncols = lh that only
   // touches the last column: simplest is a strided fill kernel.
   for (int p = 0; p < nplanes; ++p) {
@@ -2395,7 +2513,8 @@ extern "C" int lp_dealias1(lp_ctx *c, const void *u, void *u_big, int32_t nlev) 
   Arg a, o;
   RCHK(a.bind(c, u, vbytes(c, nlev), true, false));
   RCHK(o.bind(c, u_big, (size_t)g.ld_big * g.ny2 * nlev * esz_of(c->fdt), false, true));
-  RCHK(to_big(c, a.dev, nlev, o.dev));
+  const void *in = a.dev;
+  RCHK(to_big(c, &in, 1, nlev, &o.dev, c->fdt));
   return finish_all(c, {&a, &o});
 }
 
@@ -2405,7 +2524,8 @@ extern "C" int lp_dealias2(lp_ctx *c, void *u, void *u_big, int32_t nlev) {
   Arg a, o;
   RCHK(a.bind(c, u_big, (size_t)g.ld_big * g.ny2 * nlev * esz_of(c->fdt), true, false));
   RCHK(o.bind(c, u, vbytes(c, nlev), false, true));
-  RCHK(from_big(c, a.dev, nlev, 1.0 / ((double)g.nx2 * g.ny2), o.dev));
+  const void *in = a.dev;
+  RCHK(from_big(c, &in, 1, nlev, 1.0 / ((double)g.nx2 * g.ny2), &o.dev));
   return finish_all(c, {&a, &o});
 }
 
@@ -2418,11 +2538,8 @@ extern "C" int lp_test_filter(lp_ctx *c, void *f, const double *G, int32_t nplan
   RCHK(gg.bind(c, G, gb, true, false));
   SpecTables t = c->tab;
   t.G1 = (const double *)gg.dev;
-  RCHK(r2c_small(c, a.dev, nplanes, 1.0, c->spec[0]));
-  ColOut o{c->spec[0], M_G1};
-  const long ps = c->sp * g.ny;
-  HIPCHK(col_op(c->fdt, g.ny, g.ny, 0, 1, 1, c->spec[0], c->sp, ps, g.lh, nplanes, 1, &o, c->sp, ps, t, c->s));
-  RCHK(c2r_small(c, c->spec[0], g.lh, nplanes, a.dev, c->fdt));
+  const ApplyField F{a.dev, nplanes, 1.0, 1, {M_G1}, {a.dev}, {c->spec[0]}};
+  RCHK(spectral_apply(c, &F, 1, c->fdt, &t));
   return finish_all(c, {&a, &gg});
 }
 
@@ -2528,9 +2645,8 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
   HIPCHK(hipMemcpyAsync(uf, c->f[LP_U], sizeof(double) * nv, hipMemcpyDeviceToDevice, c->s));
   HIPCHK(hipMemcpyAsync(vf, c->f[LP_V], sizeof(double) * nv, hipMemcpyDeviceToDevice, c->s));
   HIPCHK(hipMemcpyAsync(wf, c->f[LP_W], sizeof(double) * nv, hipMemcpyDeviceToDevice, c->s));
-  RCHK(do_filt_da(c, uf, ux, uy, gg.nz));
-  RCHK(do_filt_da(c, vf, vx, vy, gg.nz));
-  RCHK(do_filt_da(c, wf, wx, wy, gg.nz));
+  const FiltField ff[3] = {{uf, ux, uy}, {vf, vx, vy}, {wf, wx, wy}};
+  RCHK(do_filt_da(c, ff, 3, gg.nz));
   RCHK(do_ddz_uv(c, uz, uf));
   RCHK(do_ddz_uv(c, vz, vf));
   RCHK(do_ddz_w(c, wz, wf));
@@ -2538,12 +2654,9 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
                      1.0 / (zl * den), wall);
   HIPCHK(hipGetLastError());
   double *U1 = B[0], *U2 = B[1], *U3 = B[2], *O1 = B[3], *O2 = B[4], *O3 = B[5];
-  RCHK(to_big(c, uf, gg.nz, U1));
-  RCHK(to_big(c, vf, gg.nz, U2));
-  RCHK(to_big(c, wf, gg.nz, U3));
-  RCHK(to_big(c, om1, gg.nz, O1));
-  RCHK(to_big(c, om2, gg.nz, O2));
-  RCHK(to_big(c, om3, gg.nz, O3));
+  const void *bsrc[6] = {uf, vf, wf, om1, om2, om3};
+  void *bdst[6] = {U1, U2, U3, O1, O2, O3};
+  RCHK(to_big(c, bsrc, 6, gg.nz, bdst, F64));
   // ---- projection, boundary values, RHS -= grad p ----
   double *usx = V[15], *usy = V[16], *usz = V[17], *apx = V[18], *apy = V[19], *apz = V[20];
   double *arx = V[21], *ary = V[22], *arz = V[23], *aft = V[24], *aftv = V[25], *ap = V[26];
@@ -2553,12 +2666,17 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
   HIPCHK(hipGetLastError());
   // ---- pressure: c2r^T of p, dpdx, dpdy, the transposed solves, r2c^T of H, wall, lid ----
   const long ps = c->sp * gg.ny;
-  RCHK(r2c_small(c, ap, gg.nz, 1.0, c->spec[0]));
-  RCHK(r2c_small(c, apx, gg.nz - 1, 1.0, c->spec[1]));
-  RCHK(r2c_small(c, apy, gg.nz - 1, 1.0, c->spec[2]));
-  for (int q = 0; q < 3; ++q) {
-    ColOut o{c->spec[q], M_ONE};
-    RCHK(col_small(c, c->spec[q], q == 0 ? gg.nz : gg.nz - 1, 1, 0, 1, &o));
+  {
+    const double *src[3] = {ap, apx, apy};
+    R2cSet r[3];
+    ColSet k[3];
+    for (int q = 0; q < 3; ++q) {
+      const int nl = q == 0 ? gg.nz : gg.nz - 1;
+      r[q] = R2cSet{src[q], c->spec[q], nl, 1.0};
+      k[q] = ColSet{c->spec[q], nl, 1, {{c->spec[q], M_ONE}}};
+    }
+    RCHK(r2c_sets(c, r, 3, F64));
+    RCHK(col_sets(c, k, 3, 1, 0));
   }
 #define PRESS_ADJ(S, R)                                                                                             \
   hipLaunchKernelGGL((k_press_adj<S, R>), dim3((unsigned)(ps / kPsModes)), dim3(kPsModes * S), 0, c->s,             \
@@ -2576,18 +2694,18 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
 #undef PRESS_ADJ
   HIPCHK(hipGetLastError());
   double *hx = V[27], *hy = V[28], *hz = V[29], *bwb = V[30], *twb = V[31];
-  double *hout[3] = {hx, hy, hz};
-  for (int q = 0; q < 3; ++q) {
-    ColOut o{c->Hs[q], M_ONE};
-    RCHK(col_small(c, c->Hs[q], gg.nz - 1, 0, 1, 1, &o));
-    RCHK(c2r_small(c, c->Hs[q], gg.lh, gg.nz - 1, hout[q], F64));
-  }
-  void *wl[2] = {c->bw, c->tw};
-  double *wlo[2] = {bwb, twb};
-  for (int q = 0; q < 2; ++q) {
-    ColOut o{wl[q], M_ONE};
-    RCHK(col_small(c, wl[q], 1, 0, 1, 1, &o));
-    RCHK(c2r_small(c, wl[q], gg.lh, 1, wlo[q], F64));
+  {
+    void *sp_[5] = {c->Hs[0], c->Hs[1], c->Hs[2], c->bw, c->tw};
+    double *out[5] = {hx, hy, hz, bwb, twb};
+    ColSet k[5];
+    C2rSet o[5];
+    for (int q = 0; q < 5; ++q) {
+      const int nl = q < 3 ? gg.nz - 1 : 1;
+      k[q] = ColSet{sp_[q], nl, 1, {{sp_[q], M_ONE}}};
+      o[q] = C2rSet{sp_[q], out[q], nl};
+    }
+    RCHK(col_sets(c, k, 5, 0, 1));
+    RCHK(c2r_sets(c, o, 5, gg.lh, F64));
   }
   // ---- AB2, RHS assembly, Euler start ----
   double *afu = V[32], *afv = V[33], *afw = V[34], *acx = V[35], *acy = V[36], *acz = V[37];
@@ -2633,30 +2751,30 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
   }
   // ---- convection: P^T, the products transposed, T^T ----
   double *pbx = B[6], *pby = B[7], *pbz = B[8];
-  RCHK(to_big(c, acx, gg.nz, pbx));
-  RCHK(to_big(c, acy, gg.nz, pby));
-  RCHK(to_big(c, acz, gg.nz, pbz));
+  const void *asrc[3] = {acx, acy, acz};
+  void *adst[3] = {pbx, pby, pbz};
+  RCHK(to_big(c, asrc, 3, gg.nz, adst, F64));
   double *aU1 = B[9], *aU2 = B[10], *aU3 = B[11], *aO1 = B[12], *aO2 = B[13], *aO3 = B[14];
   const double tt = ((double)gg.nx * gg.ny) / ((double)gg.nx2 * gg.ny2);
   hipLaunchKernelGGL(k_adj_products, grid1(nvb), dim3(256), 0, c->s, pbx, pby, pbz, U1, U2, U3, O1, O2, O3, aU1, aU2,
                      aU3, aO1, aO2, aO3, npb, gg.nz, tt);
   HIPCHK(hipGetLastError());
   double *t1 = V[41], *ao1 = V[42], *ao2 = V[43], *ao3 = V[44];
-  double *aUb[3] = {aU1, aU2, aU3}, *afq[3] = {afu, afv, afw};
-  for (int q = 0; q < 3; ++q) {  // P^T = (nx2 ny2)/(nx ny) T: truncation scaled by 1/(nx ny)
-    RCHK(from_big(c, aUb[q], gg.nz, cst, t1));
-    hipLaunchKernelGGL(k_add_plane, gv, dim3(256), 0, c->s, afq[q], t1, nv);
+  double *afq[3] = {afu, afv, afw};
+  {  // P^T = (nx2 ny2)/(nx ny) T: truncation scaled by 1/(nx ny)
+    const void *src[6] = {aU1, aU2, aU3, aO1, aO2, aO3};
+    void *dst[6] = {t1, V[9], V[10], ao1, ao2, ao3};  // uz, vz are dead
+    RCHK(from_big(c, src, 6, gg.nz, cst, dst));
+    hipLaunchKernelGGL(k_add_plane3, dim3(gv.x, 3), dim3(256), 0, c->s, afu, afv, afw, (const double *)t1,
+                       (const double *)V[9], (const double *)V[10], nv);
+    HIPCHK(hipGetLastError());
   }
-  RCHK(from_big(c, aO1, gg.nz, cst, ao1));
-  RCHK(from_big(c, aO2, gg.nz, cst, ao2));
-  RCHK(from_big(c, aO3, gg.nz, cst, ao3));
   // ---- stress divergences: the x, y derivatives of their adjoints ----
   double *dxa = V[45], *dya = V[46], *dxb = V[47], *dyb = V[48], *dxc = V[49], *dyc = V[50];
-  const int mxy[2] = {M_IKX, M_IKY};
-  void *oa[2] = {dxa, dya}, *ob[2] = {dxb, dyb}, *oc[2] = {dxc, dyc};
-  RCHK(spectral_apply(c, adx, gg.nz, cst, 2, mxy, oa));
-  RCHK(spectral_apply(c, ady, gg.nz, cst, 2, mxy, ob));
-  RCHK(spectral_apply(c, adz, gg.nz, cst, 2, mxy, oc));
+  const ApplyField ad[3] = {{adx, gg.nz, cst, 2, {M_IKX, M_IKY}, {dxa, dya}, {c->spec[0], c->Hs[0]}},
+                            {ady, gg.nz, cst, 2, {M_IKX, M_IKY}, {dxb, dyb}, {c->spec[1], c->Hs[1]}},
+                            {adz, gg.nz, cst, 2, {M_IKX, M_IKY}, {dxc, dyc}, {c->spec[2], c->Hs[2]}}};
+  RCHK(spectral_apply(c, ad, 3, F64));
   // ---- stresses with the frozen Nu_t -> strain-rate adjoints (reuse the base volumes) ----
   double *aS11 = V[15], *aS12 = V[16], *aS13 = V[17], *aS22 = V[18], *aS23 = V[19], *aS33 = V[20];
   double *wtx = V[21], *wty = V[22];
@@ -2664,12 +2782,11 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
                      aS12, aS13, aS22, aS23, aS33, wtx, wty, ag, 1.0 / dz, cf.vonk / den, wall);
   HIPCHK(hipGetLastError());
   if (wall) {  // the wall law's test filter (symmetric) on the txz(1), tyz(1) adjoints
-    const int mg[1] = {M_G1};
-    void *o1[1] = {t1};
-    RCHK(spectral_apply(c, wtx, 1, 1.0, 1, mg, o1));
-    hipLaunchKernelGGL(k_add_plane, grid1(np), dim3(256), 0, c->s, afu, t1, np);
-    RCHK(spectral_apply(c, wty, 1, 1.0, 1, mg, o1));
-    hipLaunchKernelGGL(k_add_plane, grid1(np), dim3(256), 0, c->s, afv, t1, np);
+    double *t2 = t1 + np;
+    const ApplyField wf2[2] = {{wtx, 1, 1.0, 1, {M_G1}, {t1}, {c->bw}}, {wty, 1, 1.0, 1, {M_G1}, {t2}, {c->tw}}};
+    RCHK(spectral_apply(c, wf2, 2, F64));
+    hipLaunchKernelGGL(k_add_plane3, dim3(grid1(np).x, 2), dim3(256), 0, c->s, afu, afv, afv, (const double *)t1,
+                       (const double *)t2, (const double *)t2, np);
     HIPCHK(hipGetLastError());
   }
   double *aux = V[3], *auy = V[4], *avx = V[5], *avy = V[6], *awx = V[7], *awy = V[8];
@@ -2691,15 +2808,19 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
     HIPCHK(hipGetLastError());
   }
   // ---- filt_da transposed: F(af) - Dx(a*x) - Dy(a*y) ----
-  double *ff = V[9], *gx = V[10], *gy = V[11];
   double *axq[3] = {aux, avx, awx}, *ayq[3] = {auy, avy, awy};
-  const int m1[1] = {M_ONE}, mx[1] = {M_IKX}, my[1] = {M_IKY};
-  for (int q = 0; q < 3; ++q) {
-    void *of[1] = {ff}, *ox[1] = {gx}, *oy[1] = {gy};
-    RCHK(spectral_apply(c, afq[q], gg.nz, cst, 1, m1, of));
-    RCHK(spectral_apply(c, axq[q], gg.nz, cst, 1, mx, ox));
-    RCHK(spectral_apply(c, ayq[q], gg.nz, cst, 1, my, oy));
-    hipLaunchKernelGGL(k_adj_combine, gv, dim3(256), 0, c->s, ub + (size_t)q * nv, ff, gx, gy, ag);
+  {
+    // the nine fields and their images: the images go over the adjoints (each is read before
+    // it is written: all transforms of a launch precede the back-transforms)
+    void *sp_[9] = {c->spec[0], c->spec[1], c->spec[2], c->spec[3], c->Hs[0],
+                    c->Hs[1], c->Hs[2], c->cv_spec[0], c->cv_spec[1]};
+    double *in[9] = {afq[0], afq[1], afq[2], axq[0], axq[1], axq[2], ayq[0], ayq[1], ayq[2]};
+    ApplyField F[9];
+    for (int q = 0; q < 9; ++q)
+      F[q] = ApplyField{in[q], gg.nz, cst, 1, {q < 3 ? M_ONE : q < 6 ? M_IKX : M_IKY}, {in[q]}, {sp_[q]}};
+    RCHK(spectral_apply(c, F, 9, F64));
+    hipLaunchKernelGGL(k_adj_combine, dim3(gv.x, 3), dim3(256), 0, c->s, ub, afq[0], afq[1], afq[2], axq[0], axq[1],
+                       axq[2], ayq[0], ayq[1], ayq[2], nv, ag);
     HIPCHK(hipGetLastError());
   }
   return LP_OK;

@@ -83,7 +83,6 @@ __global__ __launch_bounds__((CvCfg<T, M>::NTHR)) void k_convec_rows(const cx<T>
     return x;
   };
   {
-    // merge (as row_c2r): Y[k] = (X[k] + conj X[M-k]) + i w^-k (X[k] - conj X[M-k])
     cx<T> xa_[Q], xb_[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -95,11 +94,7 @@ __global__ __launch_bounds__((CvCfg<T, M>::NTHR)) void k_convec_rows(const cx<T>
     cx<T> v[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      const int kk = t + P * q;
-      cx<T> xa = xa_[q], xb = conjg(xb_[q]);
-      cx<T> e = xa + xb, o = xa - xb;
-      cx<T> wo = cmul(conjg(tws[M + kk]), o);
-      v[q] = mk<T>(e.x - wo.y, e.y + wo.x);
+      v[q] = merge_c2r<true>(xa_[q], xb_[q], tws[M + t + P * q]);
     }
     cx<T> *sc = scr + (inv ? slot : 0) * K::SSI;
     if (inv) K::FI::stage1(v, t, sc, tws);
@@ -191,13 +186,9 @@ __global__ __launch_bounds__((CvCfg<T, M>::NTHR)) void k_convec_rows(const cx<T>
     }
   slot_sync<P>();
   if (fwd && k < nz - 1) {
-    // split: X[k] = (Z[k] + conj Z[M-k])/2 - i/2 w^k (Z[k] - conj Z[M-k]), w = exp(-2 pi i/2M)
     cx<T> *dst = C + c * fplane + ((long)k * ny2 + y) * pitch;
     for (int kk = t; kk < ncols; kk += P) {
-      cx<T> za = sc[kk % M], zb = conjg(sc[(M - kk) % M]);
-      cx<T> e = za + zb, o = za - zb;
-      cx<T> wo = cmul(tws[M + kk], o);
-      dst[kk] = mk<T>(T(0.5) * (e.x + wo.y), T(0.5) * (e.y - wo.x));
+      dst[kk] = split_r2c<true>(sc[kk % M], sc[(M - kk) % M], tws[M + kk]);
     }
   }
 }

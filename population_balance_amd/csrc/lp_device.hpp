@@ -8,7 +8,15 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+// The transforms' arithmetic is written out: fused multiply-adds where they stand and nowhere
+// else.  Left to the compiler, which products it fuses into which sums depends on the code
+// around them, so that the same transform rounds differently in two kernels.
+#pragma clang fp contract(off)
+
 namespace lp {
+
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return fma(a, b, c); }
 
 template <typename T> struct alignas(2 * sizeof(T)) cx {
   T x, y;
@@ -18,7 +26,7 @@ template <typename T> __device__ __forceinline__ cx<T> mk(T a, T b) { cx<T> r; r
 template <typename T> __device__ __forceinline__ cx<T> operator+(cx<T> a, cx<T> b) { return mk(a.x + b.x, a.y + b.y); }
 template <typename T> __device__ __forceinline__ cx<T> operator-(cx<T> a, cx<T> b) { return mk(a.x - b.x, a.y - b.y); }
 template <typename T> __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
-  return mk(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return mk(fmadd(-a.y, b.y, a.x * b.x), fmadd(a.x, b.y, a.y * b.x));
 }
 template <typename T> __device__ __forceinline__ cx<T> conjg(cx<T> a) { return mk(a.x, -a.y); }
 template <typename T> __device__ __forceinline__ cx<T> scal(cx<T> a, T s) { return mk(a.x * s, a.y * s); }
@@ -57,13 +65,14 @@ template <typename T, int SIGN> struct SmallDft<T, 3, SIGN> {
     const T s1 = T(SIGN) * T(0.86602540378443864676372317075294);
     cx<T> t1 = v[1] + v[2];
     cx<T> t2 = v[1] - v[2];
-    cx<T> m = mk(v[0].x + c1 * t1.x, v[0].y + c1 * t1.y);
-    // i*s1*t2
-    cx<T> j = mk(-s1 * t2.y, s1 * t2.x);
+    cx<T> m = mk(fmadd(c1, t1.x, v[0].x), fmadd(c1, t1.y, v[0].y));
     v[0] = v[0] + t1;
-    v[1] = m + j;
-    v[2] = m - j;
+    // m +- i*s1*t2
+    v[1] = mk(fmadd(-s1, t2.y, m.x), fmadd(s1, t2.x, m.y));
+    v[2] = mk(fmadd(s1, t2.y, m.x), fmadd(-s1, t2.x, m.y));
   }
 };
 
 }  // namespace lp
+
+#pragma clang fp contract(fast)

@@ -10,8 +10,12 @@
 // exchange; loads and stores go straight between HBM and registers.
 #include <hip/hip_ext.h>
 
+#include <climits>
+
 #include "lp_fft4.hpp"
 #include "lp_internal.hpp"
+
+#pragma clang fp contract(off)  // see lp_device.hpp
 
 namespace lp {
 
@@ -50,25 +54,54 @@ static unsigned r2c_grid(long ngroups, bool persistent) {
 }
 
 // ---------------------------------------------------------------------------------
+// Sets of a launch.  `first` is the first plane of each set in the launch (INT_MAX past the
+// last set); a plane's set is found by comparing, on scalars: every wavefront's rows lie in
+// one plane (64/P divides the rows of a plane), every column block's columns too.  What a block
+// needs of its set lies together, and a launch of one set is a kernel of its own (N = 1) with
+// no search and an eighth of the arguments: as one kernel, a lone 64 x 64 plane took 0.5 to
+// 2.4 us more in its three passes.
+// ---------------------------------------------------------------------------------
+template <typename Set, int N> struct Sets {
+  int first[N];
+  Set s[N];
+  __device__ __forceinline__ int of(int plane) const {
+    int f = 0;
+#pragma unroll
+    for (int i = 1; i < N; ++i) f += plane >= first[i] ? 1 : 0;
+    return f;
+  }
+};
+template <typename T, typename TI> struct R2cArg {
+  const TI *in;
+  cx<T> *out;
+  TI scale;
+  int flag;  // 1: shifted; vorticity: 1 negated, 2 averaged on plane 0
+  const T *b;
+  double *shift_out;
+};
+template <typename T, typename TO> struct C2rArg {
+  const cx<T> *in;
+  TO *out;
+  int np;
+  int w;  // div: 1 the w-node form
+  const TO *tz;
+  const double *shift;
+};
+
+// ---------------------------------------------------------------------------------
 // row_r2c: real rows of 2M values -> M+1 complex (half-length complex FFT + split)
 // ---------------------------------------------------------------------------------
-// PRO selects the input: 0 the rows of `in`; 1..3 a vorticity component formed from two
-// derivative volumes a, b (convec.f90:100-133): 1 w_y - v_z (a = dwdy, b = dvdz), 2
-// u_z - w_x (a = dwdx, b = dudz), 3 v_x - u_y (a = dvdx, b = dudy); on plane 0 (jz = 1)
-// w_y and w_x are averaged with plane 1 onto the uvp node.  a, b have in's layout.
-// TI is the type of `in` (binary64 velocities into a binary32 transform).  SH: every row
-// of a plane enters shifted by the plane's first value, (in - in[plane, 0, 0]) * scale,
-// which only moves the plane's kx = ky = 0 mode; the row y = 0 stores that value in
-// shift_out[plane] when shift_out is given.
-template <typename T, int M, int PRO = 0, typename TI = T, bool SH = false>
-__global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in, long in_pitch, long in_plane,
-                                                       int rows, int nplanes, TI scale, cx<T> *__restrict__ out,
-                                                       long out_pitch, long out_plane, int ncols_out,
+// VORT: the rows are a vorticity component formed from two derivative volumes (convec.f90:
+// 100-133): w_y - v_z, u_z - w_x, v_x - u_y; on plane 0 (jz = 1) w_y and w_x are averaged with
+// plane 1 onto the uvp node.  b has in's layout.
+// TI is the type of `in` (binary64 velocities into a binary32 transform); there, a shifted
+// set's rows enter as (in - in[plane, 0, 0]) * scale, which only moves the plane's kx = ky = 0
+// mode; the row y = 0 stores that value in shift_out[plane] when shift_out is given.
+template <typename T, int M, int N, bool VORT = false, typename TI = T>
+__global__ __launch_bounds__(kR2cBlock) void k_row_r2c(Sets<R2cArg<T, TI>, N> A, long in_pitch, long in_plane, unsigned rows,
+                                                       unsigned total, long out_pitch, long out_plane, int ncols_out,
                                                        const cx<T> *__restrict__ twM,
-                                                       const cx<T> *__restrict__ twN,
-                                                       const T *__restrict__ pa = nullptr,
-                                                       const T *__restrict__ pb = nullptr,
-                                                       double *__restrict__ shift_out = nullptr) {
+                                                       const cx<T> *__restrict__ twN) {
   constexpr int P = row_lanes(M);
   using F = Fft4<T, M, P, -1>;
   constexpr int Q = F::Q;
@@ -78,51 +111,57 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in
   __shared__ cx<T> lds[RB * SS];
   __shared__ cx<T> tws[2 * M + 1];  // twM[0..M), twN[0..M]: read from LDS by every group
   const int t = threadIdx.x % P, r = threadIdx.x / P;
-  const long total = (long)rows * nplanes;
-  const long ngroups = (total + RB - 1) / RB;
+  const unsigned ngroups = (total + RB - 1) / RB;
   cx<T> *sc = lds + r * SS;
   for (int i = threadIdx.x; i <= 2 * M; i += kR2cBlock) tws[i] = i < M ? twM[i] : twN[i - M];
   __syncthreads();
   using v2 = typename V2<T>::t;
-  // input of row group g (rows beyond the last read row 0 and are not stored)
-  auto load = [&](long g, cx<T> (&v)[Q]) {
-    const long grow = g * RB + r;
-    const bool valid = grow < total;
-    const long plane = valid ? grow / rows : 0, y = valid ? grow % rows : 0;
-    if constexpr (PRO == 0) {
+  // plane of this wavefront's rows in group g, and the row (beyond the last: row 0 of plane 0,
+  // not stored)
+  auto where = [&](unsigned g, unsigned &y) -> int {
+    const unsigned grow = g * RB + r;
+    const unsigned pl = grow < total ? grow / rows : 0;
+    y = grow < total ? grow - pl * rows : 0;
+    return __builtin_amdgcn_readfirstlane((int)pl);
+  };
+  auto load = [&](unsigned g, cx<T> (&v)[Q]) {
+    unsigned y;
+    const int pg = where(g, y);
+    const int f = A.of(pg), plane = pg - A.first[f];
+    const R2cArg<T, TI> &S = A.s[f];
+    const TI scale = S.scale;
+    if constexpr (!VORT) {
       using vi2 = typename V2<TI>::t;
-      const TI *src = in + plane * in_plane + y * in_pitch;
+      const TI *src0 = S.in + (long)plane * in_plane;
+      const TI *src = src0 + y * in_pitch;
       TI s0 = TI(0);
-      if constexpr (SH) s0 = in[plane * in_plane];
+      if constexpr (sizeof(TI) > sizeof(T)) s0 = S.flag ? src0[0] : TI(0);
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         const vi2 p = *reinterpret_cast<const vi2 *>(src + 2 * (t + P * q));
-        if constexpr (SH)
+        if constexpr (sizeof(TI) > sizeof(T))
           v[q] = mk<T>((T)((p.x - s0) * scale), (T)((p.y - s0) * scale));
         else
           v[q] = mk<T>((T)(p.x * scale), (T)(p.y * scale));
       }
-      if constexpr (SH) {
-        if (shift_out && valid && y == 0 && t == 0) shift_out[plane] = (double)s0;
+      if constexpr (sizeof(TI) > sizeof(T)) {
+        if (S.shift_out && g * RB + r < total && y == 0 && t == 0) S.shift_out[plane] = (double)s0;
       }
     } else {
-      const long o = plane * in_plane + y * in_pitch;
-      const long up = (PRO != 3 && plane == 0) ? in_plane : 0;  // clamped: same row above jz = 1
+      const long o = (long)plane * in_plane + y * in_pitch;
+      const bool avg = (S.flag & 2) && plane == 0, neg = S.flag & 1;
+      const long up = avg ? in_plane : 0;  // clamped: same row above jz = 1
+      const T *pa = S.in + o, *pb = S.b + o;
       const T h = T(0.5);
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        const long x = o + 2 * (t + P * q);
+        const int x = 2 * (t + P * q);
         const v2 a0 = *reinterpret_cast<const v2 *>(pa + x);
         const v2 b0 = *reinterpret_cast<const v2 *>(pb + x);
-        v2 rr;
-        if constexpr (PRO == 3) {
-          rr = v2{a0.x - b0.x, a0.y - b0.y};
-        } else {
-          const v2 a1 = *reinterpret_cast<const v2 *>(pa + x + up);
-          const v2 av{h * (a0.x + a1.x), h * (a0.y + a1.y)};
-          const v2 aa = plane == 0 ? av : a0;
-          rr = PRO == 1 ? v2{aa.x - b0.x, aa.y - b0.y} : v2{b0.x - aa.x, b0.y - aa.y};
-        }
+        const v2 a1 = *reinterpret_cast<const v2 *>(pa + x + up);
+        const v2 av{h * (a0.x + a1.x), h * (a0.y + a1.y)};
+        const v2 aa = avg ? av : a0;
+        const v2 rr = neg ? v2{b0.x - aa.x, b0.y - aa.y} : v2{aa.x - b0.x, aa.y - b0.y};
         v[q] = mk<T>(rr.x * scale, rr.y * scale);
       }
     }
@@ -130,16 +169,13 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in
   // binary32: persistent blocks, the next group's loads issued before this group's
   // transform; binary64 (twice the registers per value): one group per block
   constexpr bool PF = r2c_persistent<T>();
-  long g = blockIdx.x;
+  unsigned g = blockIdx.x;
   cx<T> v[Q];
   if (PF && g < ngroups) load(g, v);
   for (; g < ngroups; g += gridDim.x) {
     cx<T> vn[Q];
     if (!PF) load(g, v);
     else if (g + gridDim.x < ngroups) load(g + gridDim.x, vn);
-    const long grow = g * RB + r;
-    const bool valid = grow < total;
-    const long plane = valid ? grow / rows : 0, y = valid ? grow % rows : 0;
     F::stage1(v, t, sc, tws);
     slot_sync<P>();
     cx<T> a[F::G][P];
@@ -154,14 +190,13 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in
         for (int k1 = 0; k1 < P; ++k1) sc[t + P * j + Q * k1] = a[j][k1];
       }
     slot_sync<P>();
-    // split: X[k] = (Z[k] + conj Z[M-k])/2 - i/2 w^k (Z[k] - conj Z[M-k]), w = exp(-2 pi i/2M)
-    if (valid) {
-      cx<T> *dst = out + plane * out_plane + y * out_pitch;
+    if (g * RB + r < total) {
+      unsigned y;
+      const int pg = where(g, y);
+      const int f = A.of(pg);
+      cx<T> *dst = A.s[f].out + (long)(pg - A.first[f]) * out_plane + y * out_pitch;
       for (int k = t; k <= M && k < ncols_out; k += P) {
-        cx<T> za = sc[k % M], zb = conjg(sc[(M - k) % M]);
-        cx<T> e = za + zb, o = za - zb;
-        cx<T> wo = cmul(tws[M + k], o);
-        dst[k] = mk<T>(T(0.5) * (e.x + wo.y), T(0.5) * (e.y - wo.x));
+        dst[k] = split_r2c<false>(sc[k % M], sc[(M - k) % M], tws[M + k]);
       }
     }
     if (!PF) break;
@@ -171,36 +206,24 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(const TI *__restrict__ in
   }
 }
 
-// merge of the half spectrum into the M-point complex input of a 2M-point real inverse
-// transform: Y[k] = (X[k] + conj X[M-k]) + i w^-k (X[k] - conj X[M-k]), w = exp(-2 pi i/2M)
-template <typename T> __device__ __forceinline__ cx<T> merge_c2r(cx<T> xa, cx<T> xm, cx<T> w) {
-  const cx<T> xb = conjg(xm);
-  const cx<T> e = xa + xb, o = xa - xb;
-  const cx<T> wo = cmul(conjg(w), o);
-  return mk<T>(e.x - wo.y, e.y + wo.x);
-}
-
 // ---------------------------------------------------------------------------------
 // row_c2r: M+1 complex (first ncols_in present; imaginary parts of kx = 0 and kx = M
 // ignored, as FFTW2's halfcomplex c2r) -> 2M reals, columns [2M, out_pitch) zeroed
 // ---------------------------------------------------------------------------------
-// EPI selects what is stored: 0 the transform; 1 (divstress_uv.f90:88-89,116-125) the
-// transform plus dz^-1 (tz(k+1) - tz(k)), BOGUS on the top level; 2 (divstress_w.f90:35,
-// 46-81 with the wall at level 1 and no lid term) the transform plus dz^-1 (tz(k) - tz(k-1))
-// on levels 1..nz-2.  The padding columns are zero (BOGUS on the uv top level).  tz has the
-// layout of out.  ikx (optional): the input is multiplied by i*ikx[kx] first, which turns
-// the (kx, y) spectrum of f into that of df/dx (ddx.f90:15-24; kx is uniform along y).
-// shift (optional, EPI 0): shift[plane] is added to every stored value of the plane in
-// binary64 (the inverse of k_row_r2c's SH; padding columns stay zero).
-template <typename T, typename TO, int M, int EPI, bool IKX = false>
-__global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restrict__ in, long in_pitch, long in_plane,
-                                                       int ncols_in, int rows, int nplanes,
-                                                       TO *__restrict__ out, long out_pitch, long out_plane,
-                                                       const cx<T> *__restrict__ twM,
-                                                       const cx<T> *__restrict__ twN,
-                                                       const TO *__restrict__ tz, TO cst,
-                                                       const double *__restrict__ ikx,
-                                                       const double *__restrict__ shift, int xorder) {
+// DIV: what is stored is, per set, (divstress_uv.f90:88-89,116-125) the transform plus
+// dz^-1 (tz(k+1) - tz(k)), BOGUS on the top level; or (w: divstress_w.f90:35, 46-81 with the
+// wall at level 1 and no lid term) the transform plus dz^-1 (tz(k) - tz(k-1)) on levels
+// 1..nz-2.  The padding columns are zero (BOGUS on the uv top level).  tz has the layout of
+// out.  IKX: the input is multiplied by i*ikx[kx] first, which turns the (kx, y) spectrum of f
+// into that of df/dx (ddx.f90:15-24; kx is uniform along y).  shift (optional): shift[plane] is
+// added to every stored value of the plane in binary64 (the inverse of k_row_r2c's shift;
+// padding columns stay zero).
+template <typename T, typename TO, int M, int N, bool DIV, bool IKX = false>
+__global__ __launch_bounds__(row_block<T>()) void k_row_c2r(Sets<C2rArg<T, TO>, N> A, long in_pitch, long in_plane,
+                                                       int ncols_in, unsigned rows, unsigned total, long out_pitch,
+                                                       long out_plane, const cx<T> *__restrict__ twM,
+                                                       const cx<T> *__restrict__ twN, TO cst,
+                                                       const double *__restrict__ ikx, int xorder) {
   constexpr int P = row_lanes(M);
   using F = Fft4<T, M, P, +1>;
   constexpr int Q = F::Q;
@@ -210,18 +233,30 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restr
   __shared__ cx<T> lds[RB * SS];
   __shared__ cx<T> tws[2 * M];  // twM[0..M), twN[0..M): read from LDS by every row
   const int t = threadIdx.x % P, r = threadIdx.x / P;
-  long blk = blockIdx.x;
-  if (xorder) {  // XCD order, first-written planes first; the grid has 8 max_j(planes of j) gpp blocks
-    const int gpp = rows / RB, xj = (int)(blockIdx.x & 7u);
-    const long xi = blockIdx.x >> 3, kq = xi / gpp;
-    if (kq >= xcd_planes(nplanes, xj)) return;  // uniform over the block
-    blk = (long)(xj + 8 * kq) * gpp + xi % gpp;
+  int f, plane;
+  unsigned y;
+  bool valid;
+  if (xorder) {  // XCD order, first-written planes first; the grid has 8 groups gpp blocks
+    const unsigned gpp = rows / RB, xi = blockIdx.x >> 3;
+    const int gq = (int)(xi / gpp);
+    f = A.of(gq);
+    plane = (int)(blockIdx.x & 7u) + 8 * (gq - A.first[f]);
+    if (plane >= A.s[f].np) return;  // uniform over the block
+    y = (xi % gpp) * RB + r;
+    valid = true;
+  } else {
+    const unsigned grow = blockIdx.x * RB + r;
+    valid = grow < total;
+    const unsigned pl = valid ? grow / rows : 0;
+    y = valid ? grow - pl * rows : 0;
+    const int pg = __builtin_amdgcn_readfirstlane((int)pl);
+    f = A.of(pg);
+    plane = pg - A.first[f];
   }
-  const long grow = blk * RB + r;
-  const bool valid = grow < (long)rows * nplanes;
-  const long plane = valid ? grow / rows : 0, y = valid ? grow % rows : 0;
+  const C2rArg<T, TO> &S = A.s[f];
+  const int nplanes = S.np;
   cx<T> *sc = lds + r * SS;
-  const cx<T> *src = in + plane * in_plane + y * in_pitch;
+  const cx<T> *src = S.in + (long)plane * in_plane + y * in_pitch;
   for (int i = threadIdx.x; i < 2 * M; i += row_block<T>()) tws[i] = i < M ? twM[i] : twN[i - M];
   __shared__ T ikxs[IKX ? M + 1 : 1];  // the multipliers, in the transform's type
   if constexpr (IKX)
@@ -239,34 +274,33 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restr
       const int k = t + P * q;
       const T sa = ikxs[k], sb = ikxs[M - k];
       const cx<T> ra = ld(k), rb = ld(M - k);
-      v[q] = merge_c2r(mk<T>(-ra.y * sa, ra.x * sa), mk<T>(-rb.y * sb, rb.x * sb), tws[M + k]);
+      v[q] = merge_c2r<false>(mk<T>(-ra.y * sa, ra.x * sa), mk<T>(-rb.y * sb, rb.x * sb), tws[M + k]);
     }
   } else {
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int k = t + P * q;
-      v[q] = merge_c2r(ld(k), ld(M - k), tws[M + k]);
+      v[q] = merge_c2r<false>(ld(k), ld(M - k), tws[M + k]);
     }
   }
   F::stage1(v, t, sc, tws);
   slot_sync<P>();
-  TO *dst = out + plane * out_plane + y * out_pitch;
-  const TO *tzr = tz + plane * out_plane + y * out_pitch;
+  const long od = (long)plane * out_plane + y * out_pitch;
+  TO *dst = S.out + od;
   const bool top = plane == nplanes - 1;
   const bool mid = plane >= 1 && plane <= nplanes - 2;
-  const long up = top ? 0 : out_plane, dn = mid ? out_plane : 0;  // neighbour levels, clamped
-  const double sh = (EPI == 0 && shift && valid) ? shift[plane] : 0.0;
+  const bool isw = DIV && S.w;
+  // neighbour levels, clamped: uv k + 1 and k, w k and k - 1
+  const TO *tzr = DIV ? S.tz + od : nullptr;
+  const long up = isw || top ? 0 : out_plane, dn = isw && mid ? out_plane : 0;
+  const double *shp = DIV ? nullptr : S.shift;
+  const double sh = shp && valid ? shp[plane] : 0.0;
   auto fin = [&](T v, int x) -> TO {
-    if constexpr (EPI == 1) {
-      const TO d = cst * (tzr[x + up] - tzr[x]);
-      return top ? (TO)LP_BOGUS : (TO)v + d;
-    } else if constexpr (EPI == 2) {
-      TO r = (TO)v;
-      const TO d = cst * (tzr[x] - tzr[x - dn]);
-      if (mid) r += d;
-      return r;
+    if constexpr (DIV) {
+      const TO r = fmadd(cst, tzr[x + up] - tzr[x - dn], (TO)v);
+      return isw ? (mid ? r : (TO)v) : (top ? (TO)LP_BOGUS : r);
     } else {
-      if (shift) return (TO)((double)v + sh);  // the plane's shift back, in binary64
+      if (shp) return (TO)((double)v + sh);  // the plane's shift back, in binary64
       return (TO)v;
     }
   };
@@ -283,7 +317,7 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restr
     }
   }
   if (valid) {
-    const TO pad = (EPI == 1 && top) ? (TO)LP_BOGUS : (TO)0;
+    const TO pad = (DIV && !isw && top) ? (TO)LP_BOGUS : (TO)0;
     for (long n = 2 * M + t; n < out_pitch; n += P) dst[n] = pad;
   }
 }
@@ -297,16 +331,17 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(const cx<T> *__restr
 // ---------------------------------------------------------------------------------
 struct ColSlot {
   void *ptr;
-  long pitch;  // complex elements between y rows of this output
-  long plane;  // complex elements between planes of this output
-  int mult;
-  int tpitch;  // row length of the multiplier tables (lh of the small grid)
-  int ncols;   // columns stored (kx < ncols)
   double scale;  // factor on the padded / truncated spectrum (padmode 1, 2)
+  int pitch;     // complex elements between y rows of this output
+  int plane;     // complex elements between planes of this output
+  int mult;
+  int ncols;     // columns stored (kx < ncols)
 };
-struct ColParams {
+struct ColArg {
+  const void *in;
+  const double *dc;
+  int np, nout;
   ColSlot outs[3];
-  int nout;
 };
 static constexpr int kColLanes = 16;
 template <typename T> __host__ __device__ constexpr int col_tx() { return 128 / (int)sizeof(cx<T>); }
@@ -351,12 +386,11 @@ __device__ __forceinline__ void col_forward(cx<T> (&sp)[NY / kColLanes], int t, 
 
 // TX columns per block (16 for binary32, 8 for binary64: one 128-byte run per y); TX = 1
 // serves a single trailing column.  Block column c handles kx = col0 + blockIdx.x*TX + c.
-template <typename T, int NYI, int NYO, int TX = col_tx<T>()>
+template <typename T, int NYI, int NYO, int N, int TX = col_tx<T>()>
 __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
-    const cx<T> *__restrict__ in, long in_pitch, long in_plane, int ncols, int fwd, int inv, ColParams Pr,
-    long out_pitch, long out_plane, const double *__restrict__ kxt, const double *__restrict__ kyt,
+    Sets<ColArg, N> Pr, int ngroups, long in_pitch, long in_plane, int ncols, int fwd, int inv, const double *__restrict__ kxt, const double *__restrict__ kyt,
     const double *__restrict__ G1, const double *__restrict__ G2, int lh_s, int ny_s,
-    const cx<T> *__restrict__ twI, const cx<T> *__restrict__ twO, int col0, int nplanes) {
+    const cx<T> *__restrict__ twI, const cx<T> *__restrict__ twO, int col0) {
   constexpr int PL = kColLanes;
   using FI = Fft4<T, NYI, PL, -1>;
   using FO = Fft4<T, NYO, PL, +1>;
@@ -370,15 +404,18 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
   constexpr bool TWL = sizeof(T) == 4;
   __shared__ cx<T> lds[TX * SS + (TWL ? NYI + NYO : 0)];
   const int c = threadIdx.x % TX, t = threadIdx.x / TX;
-  int plane = blockIdx.y, cg = blockIdx.x;
-  if constexpr (xcd_order<T>()) {  // last-written planes first; the grid has gx x 8 max_j(planes of j) blocks
+  int plane = blockIdx.y, cg = blockIdx.x, f;
+  if constexpr (xcd_order<T>()) {  // last-written planes first; the grid has gx x 8 groups blocks
     const int gx = gridDim.x;
     const long lin = blockIdx.x + (long)gx * blockIdx.y;
-    const int xj = (int)(lin & 7), kq = (int)((lin >> 3) / gx);
-    const int npj = xcd_planes(nplanes, xj);
-    if (kq >= npj) return;  // uniform over the block
-    plane = xj + 8 * (npj - 1 - kq);
+    const int gq = ngroups - 1 - (int)((lin >> 3) / gx);
+    f = Pr.of(gq);
+    plane = (int)(lin & 7) + 8 * (gq - Pr.first[f]);
+    if (plane >= Pr.s[f].np) return;  // uniform over the block
     cg = (int)((lin >> 3) % gx);
+  } else {
+    f = Pr.of(plane);
+    plane -= Pr.first[f];
   }
   const int kx = col0 + cg * TX + c;
   const bool cv = kx < ncols;
@@ -391,7 +428,8 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
     __syncthreads();
   }
   // invalid columns load column ncols-1 and discard it (no divergent loads)
-  const cx<T> *src = in + (long)plane * in_plane + (cv ? kx : ncols - 1) + (long)t * in_pitch;
+  const cx<T> *src = reinterpret_cast<const cx<T> *>(Pr.s[f].in) + (long)plane * in_plane + (cv ? kx : ncols - 1) +
+                     (long)t * in_pitch;
   const long istep = (long)PL * in_pitch;
   cx<T> sp[QI];  // D16: sp[m] = spectrum[t + 16 m]
 #pragma unroll
@@ -399,14 +437,23 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
     const cx<T> x = src[m * istep];
     sp[m] = cv ? x : mk<T>(0, 0);
   }
+  if constexpr (PM == 1) {
+    if (Pr.s[f].dc && kx == 0) {
+      const double dc = Pr.s[f].dc[plane];
+#pragma unroll
+      for (int m = 0; m < QI; ++m) sp[m].x = (T)((double)sp[m].x + dc);
+    }
+  }
   if (fwd) col_forward<T, NYI>(sp, t, sc, twI);
-  for (int jo = 0; jo < Pr.nout; ++jo) {
-    const int mult = Pr.outs[jo].mult;
+  const int nout = Pr.s[f].nout;
+  const ColSlot *outs = Pr.s[f].outs;
+  for (int jo = 0; jo < nout; ++jo) {
+    const int mult = outs[jo].mult;
     // one multiplier table per output: i*kx, i*ky (imaginary) or a filter (real)
     const double *mt = mult == M_IKX ? kxt : mult == M_IKY ? kyt : mult == M_G1 ? G1 : G2;
     const bool imag = mult == M_IKX || mult == M_IKY;
     const bool keep = cv && kx != lh_s - 1;
-    const int tp = Pr.outs[jo].tpitch;
+    const int tp = lh_s;  // row length of the multiplier tables
     const double *mrow = mt + (long)t * tp + (cv ? kx : 0);
     cx<T> v[QO];
     if constexpr (PM == 0) {
@@ -425,8 +472,8 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
       }
     }
     if constexpr (PM != 0) {
-      const T osc = (T)Pr.outs[jo].scale;
-      const bool scaled = Pr.outs[jo].scale != 1.0;
+      const T osc = (T)outs[jo].scale;
+      const bool scaled = outs[jo].scale != 1.0;
 #pragma unroll
       for (int q = 0; q < QO; ++q) {
         const int yo = t + PL * q;
@@ -443,9 +490,9 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
     }
     // addresses are formed from per-output values so that they are not hoisted out of
     // the output loop (which would keep 16 64-bit addresses live)
-    const long pitch = Pr.outs[jo].pitch;
-    const bool st = cv && kx < Pr.outs[jo].ncols;
-    cx<T> *dst = reinterpret_cast<cx<T> *>(Pr.outs[jo].ptr) + (long)plane * Pr.outs[jo].plane + kx;
+    const long pitch = outs[jo].pitch;
+    const bool st = cv && kx < outs[jo].ncols;
+    cx<T> *dst = reinterpret_cast<cx<T> *>(outs[jo].ptr) + (long)plane * outs[jo].plane + kx;
     if (inv) {
       FO::stage1(v, t, sc, twO);
       __syncthreads();
@@ -475,10 +522,12 @@ __global__ __launch_bounds__(TX * kColLanes) void k_col_op(
 // i kx A + i ky B with the Nyquist row and column zeroed (the ddx / ddy multipliers),
 // inverse y DFT into out.
 // ---------------------------------------------------------------------------------
+struct DivSets {
+  DivSet s[kMaxSets];
+};
 template <typename T, int NY>
 __global__ __launch_bounds__(col_tx<T>() * kColLanes) void k_col_div(
-    const cx<T> *__restrict__ A, const cx<T> *__restrict__ B, long pitch, long plane_el, int ncols,
-    cx<T> *__restrict__ out, const double *__restrict__ kxt, const double *__restrict__ kyt, int lh_s, int ny_s,
+    DivSets D, int nplanes, long pitch, long plane_el, int ncols, const double *__restrict__ kxt, const double *__restrict__ kyt, int lh_s, int ny_s,
     const cx<T> *__restrict__ tw) {
   constexpr int TX = col_tx<T>();
   constexpr int PL = kColLanes;
@@ -490,7 +539,10 @@ __global__ __launch_bounds__(col_tx<T>() * kColLanes) void k_col_div(
   const int c = threadIdx.x % TX, t = threadIdx.x / TX;
   const int kx = blockIdx.x * TX + c;
   const bool cv = kx < ncols;
-  const long plane = blockIdx.y;
+  const int f = blockIdx.y / nplanes;
+  const long plane = blockIdx.y % nplanes;
+  const cx<T> *A = reinterpret_cast<const cx<T> *>(D.s[f].A), *B = reinterpret_cast<const cx<T> *>(D.s[f].B);
+  cx<T> *out = reinterpret_cast<cx<T> *>(D.s[f].out);
   cx<T> *sc = lds + c * SS;
   if constexpr (TWL) {
     cx<T> *tl = lds + TX * SS;
@@ -521,7 +573,7 @@ __global__ __launch_bounds__(col_tx<T>() * kColLanes) void k_col_div(
   for (int q = 0; q < Q; ++q) {
     const int yo = t + PL * q;
     const cx<T> a = sa[q], b = sb[q];
-    const cx<T> x = mk<T>(-a.y * fx[q] + -b.y * fy[q], a.x * fx[q] + b.x * fy[q]);
+    const cx<T> x = mk<T>(fmadd(-a.y, fx[q], -b.y * fy[q]), fmadd(a.x, fx[q], b.x * fy[q]));
     v[q] = (!keep || yo == ny_s / 2) ? mk<T>(0, 0) : x;
   }
   FO::stage1(v, t, sc, tw);
@@ -540,23 +592,26 @@ __global__ __launch_bounds__(col_tx<T>() * kColLanes) void k_col_div(
 }
 
 template <typename T, int NY>
-static hipError_t launch_col_div(const void *A, const void *B, long pitch, long plane, int ncols, int nplanes,
-                                 void *out, const SpecTables &tab, hipStream_t s, Dt dt) {
+static hipError_t launch_col_div(const DivSet *sets, int n, int nplanes, long pitch, long plane, int ncols,
+                                 const SpecTables &tab, hipStream_t s, Dt dt) {
   const void *tw = tw_ptr(NY, dt);
-  if (!tw || ncols < 1 || ncols > tab.lh || pitch < ncols || tab.ny != NY) return hipErrorInvalidValue;
+  if (!tw || n < 1 || n > kMaxSets || ncols < 1 || ncols > tab.lh || pitch < ncols || tab.ny != NY)
+    return hipErrorInvalidValue;
   constexpr int TX = col_tx<T>();
-  dim3 grid((unsigned)((ncols + TX - 1) / TX), (unsigned)nplanes);
-  hipLaunchKernelGGL((k_col_div<T, NY>), grid, dim3(TX * kColLanes), 0, s, (const cx<T> *)A, (const cx<T> *)B,
-                     pitch, plane, ncols, (cx<T> *)out, tab.kx, tab.ky, tab.lh, tab.ny, (const cx<T> *)tw);
+  DivSets D{};
+  for (int f = 0; f < n; ++f) D.s[f] = sets[f];
+  dim3 grid((unsigned)((ncols + TX - 1) / TX), (unsigned)(n * nplanes));
+  hipLaunchKernelGGL((k_col_div<T, NY>), grid, dim3(TX * kColLanes), 0, s, D, nplanes, pitch, plane, ncols, tab.kx,
+                     tab.ky, tab.lh, tab.ny, (const cx<T> *)tw);
   return hipGetLastError();
 }
 
-hipError_t col_div(Dt dt, int ny, const void *A, const void *B, long pitch, long plane, int ncols, int nplanes,
-                   void *out, const SpecTables &tab, hipStream_t s) {
-#define CASE(n)                                                                                      \
-  case n:                                                                                            \
-    return dt == F64 ? launch_col_div<double, n>(A, B, pitch, plane, ncols, nplanes, out, tab, s, dt) \
-                     : launch_col_div<float, n>(A, B, pitch, plane, ncols, nplanes, out, tab, s, dt);
+hipError_t col_div(Dt dt, int ny, const DivSet *sets, int n, int nplanes, long pitch, long plane, int ncols,
+                   const SpecTables &tab, hipStream_t s) {
+#define CASE(n_)                                                                                \
+  case n_:                                                                                      \
+    return dt == F64 ? launch_col_div<double, n_>(sets, n, nplanes, pitch, plane, ncols, tab, s, dt) \
+                     : launch_col_div<float, n_>(sets, n, nplanes, pitch, plane, ncols, tab, s, dt);
   switch (ny) {
     CASE(32) CASE(48) CASE(64) CASE(96) CASE(128) CASE(144) CASE(192) CASE(256)
     default: return hipErrorInvalidValue;
@@ -578,70 +633,71 @@ bool fft_len_supported(int n) {
   }
 }
 
-template <typename T, int M, int PRO = 0, typename TI = T, bool SH = false>
-static hipError_t launch_r2c(const void *in, long in_pitch, long in_plane, int rows, int nplanes,
-                             double scale, void *out, long out_pitch, long out_plane, int ncols_out,
-                             hipStream_t s, Dt dt, const void *pa = nullptr, const void *pb = nullptr,
-                             double *shift_out = nullptr) {
+template <typename T, int M, int N, bool VORT, typename TI>
+static hipError_t launch_r2c_n(const R2cSet *sets, int n, long in_pitch, long in_plane, int rows, long out_pitch,
+                             long out_plane, int ncols_out, hipStream_t s, Dt dt) {
   const void *twM = tw_ptr(M, dt), *twN = tw_ptr(2 * M, dt);
-  if (!twM || !twN) return hipErrorInvalidValue;
-  constexpr int RPB = kR2cBlock / row_lanes(M);
-  long total = (long)rows * nplanes;
-  if (total < 1) return hipErrorInvalidValue;
+  constexpr int P = row_lanes(M), RPB = kR2cBlock / P;
+  if (!twM || !twN || n < 1 || n > N || rows < 1 || rows % (64 / P) != 0) return hipErrorInvalidValue;
+  Sets<R2cArg<T, TI>, N> A{};
+  long planes = 0;
+  for (int f = 0; f < N; ++f) {
+    A.first[f] = INT_MAX;
+    if (f >= n) continue;
+    const R2cSet &x = sets[f];
+    if (x.nplanes < 1 || (VORT && (!x.b || x.comp < 0 || x.comp > 2 || x.nplanes < 2))) return hipErrorInvalidValue;
+    A.first[f] = (int)planes;
+    A.s[f] = R2cArg<T, TI>{(const TI *)x.in, (cx<T> *)x.out, (TI)x.scale,
+                           VORT ? (x.comp == 1 ? 1 : 0) | (x.comp < 2 ? 2 : 0) : (x.shift ? 1 : 0), (const T *)x.b,
+                           x.shift_out};
+    planes += x.nplanes;
+  }
+  const long total = (long)rows * planes;
+  if (total > INT_MAX) return hipErrorInvalidValue;
   dim3 grid(r2c_grid((total + RPB - 1) / RPB, r2c_persistent<T>()));
-  hipLaunchKernelGGL((k_row_r2c<T, M, PRO, TI, SH>), grid, dim3(kR2cBlock), 0, s, (const TI *)in, in_pitch,
-                     in_plane, rows, nplanes, (TI)scale, (cx<T> *)out, out_pitch, out_plane, ncols_out,
-                     (const cx<T> *)twM, (const cx<T> *)twN, (const T *)pa, (const T *)pb, shift_out);
+  hipLaunchKernelGGL((k_row_r2c<T, M, N, VORT, TI>), grid, dim3(kR2cBlock), 0, s, A, in_pitch, in_plane,
+                     (unsigned)rows, (unsigned)total, out_pitch, out_plane, ncols_out, (const cx<T> *)twM,
+                     (const cx<T> *)twN);
   return hipGetLastError();
 }
 
-hipError_t row_r2c_vort(Dt dt, int M, int comp, const void *a, const void *b, long in_pitch, long in_plane,
-                        int rows, int nplanes, double scale, void *out, long out_pitch, long out_plane,
-                        int ncols_out, hipStream_t s) {
-  if (!a || !b || comp < 0 || comp > 2 || nplanes < 2) return hipErrorInvalidValue;
-#define CASE(m)                                                                                           \
-  case m:                                                                                                 \
-    if (dt == F64) {                                                                                      \
-      if (comp == 0) return launch_r2c<double, m, 1>(nullptr, in_pitch, in_plane, rows, nplanes, scale,   \
-                                                     out, out_pitch, out_plane, ncols_out, s, dt, a, b);  \
-      if (comp == 1) return launch_r2c<double, m, 2>(nullptr, in_pitch, in_plane, rows, nplanes, scale,   \
-                                                     out, out_pitch, out_plane, ncols_out, s, dt, a, b);  \
-      return launch_r2c<double, m, 3>(nullptr, in_pitch, in_plane, rows, nplanes, scale, out, out_pitch,  \
-                                      out_plane, ncols_out, s, dt, a, b);                                 \
-    }                                                                                                     \
-    if (comp == 0) return launch_r2c<float, m, 1>(nullptr, in_pitch, in_plane, rows, nplanes, scale, out, \
-                                                  out_pitch, out_plane, ncols_out, s, dt, a, b);          \
-    if (comp == 1) return launch_r2c<float, m, 2>(nullptr, in_pitch, in_plane, rows, nplanes, scale, out, \
-                                                  out_pitch, out_plane, ncols_out, s, dt, a, b);          \
-    return launch_r2c<float, m, 3>(nullptr, in_pitch, in_plane, rows, nplanes, scale, out, out_pitch,     \
-                                   out_plane, ncols_out, s, dt, a, b);
-  switch (M) {
-    LP_SMALL_ROW_LENGTHS(CASE)
-    default: return hipErrorInvalidValue;
-  }
-#undef CASE
+template <typename T, int M, bool VORT = false, typename TI = T>
+static hipError_t launch_r2c(const R2cSet *sets, int n, long in_pitch, long in_plane, int rows, long out_pitch,
+                             long out_plane, int ncols_out, hipStream_t s, Dt dt) {
+  return n == 1 ? launch_r2c_n<T, M, 1, VORT, TI>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane, ncols_out,
+                                                  s, dt)
+                : launch_r2c_n<T, M, kMaxSets, VORT, TI>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane,
+                                                         ncols_out, s, dt);
 }
 
-hipError_t row_r2c(Dt dt, int M, const void *in, long in_pitch, long in_plane, int rows, int nplanes,
-                   double scale, void *out, long out_pitch, long out_plane, int ncols_out, hipStream_t s,
-                   RowIn ri) {
-  const Dt din = ri.din < 0 ? dt : (Dt)ri.din;
-  if (ri.shift && !(dt == F32 && din == F64)) return hipErrorInvalidValue;
-  if (dt == F64 && din == F32) return hipErrorInvalidValue;
-#define CASE(m)                                                                                        \
-  case m:                                                                                              \
-    if (dt == F64)                                                                                     \
-      return launch_r2c<double, m>(in, in_pitch, in_plane, rows, nplanes, scale, out, out_pitch,       \
-                                   out_plane, ncols_out, s, dt);                                       \
-    if (din == F32)                                                                                    \
-      return launch_r2c<float, m>(in, in_pitch, in_plane, rows, nplanes, scale, out, out_pitch,        \
-                                  out_plane, ncols_out, s, dt);                                        \
-    if (ri.shift)                                                                                      \
-      return launch_r2c<float, m, 0, double, true>(in, in_pitch, in_plane, rows, nplanes, scale, out,  \
-                                                   out_pitch, out_plane, ncols_out, s, dt, nullptr,    \
-                                                   nullptr, ri.shift_out);                             \
-    return launch_r2c<float, m, 0, double, false>(in, in_pitch, in_plane, rows, nplanes, scale, out,   \
-                                                  out_pitch, out_plane, ncols_out, s, dt);
+hipError_t row_r2c(Dt dt, Dt din, int M, const R2cSet *sets, int n, long in_pitch, long in_plane, int rows,
+                   long out_pitch, long out_plane, int ncols_out, hipStream_t s) {
+  if (n < 1 || (dt == F64 && din == F32)) return hipErrorInvalidValue;
+  const bool vort = sets[0].comp >= 0;
+  for (int f = 0; f < n; ++f)
+    if ((sets[f].comp >= 0) != vort || (sets[f].shift && !(dt == F32 && din == F64))) return hipErrorInvalidValue;
+  if (vort) {
+    if (din != dt) return hipErrorInvalidValue;
+#define CASE(m)                                                                                                    \
+  case m:                                                                                                          \
+    return dt == F64 ? launch_r2c<double, m, true>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane,        \
+                                                   ncols_out, s, dt)                                               \
+                     : launch_r2c<float, m, true>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane,         \
+                                                  ncols_out, s, dt);
+    switch (M) {
+      LP_SMALL_ROW_LENGTHS(CASE)
+      default: return hipErrorInvalidValue;
+    }
+#undef CASE
+  }
+#define CASE(m)                                                                                                    \
+  case m:                                                                                                          \
+    if (dt == F64)                                                                                                 \
+      return launch_r2c<double, m>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane, ncols_out, s, dt);     \
+    if (din == F32)                                                                                                \
+      return launch_r2c<float, m>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane, ncols_out, s, dt);      \
+    return launch_r2c<float, m, false, double>(sets, n, in_pitch, in_plane, rows, out_pitch, out_plane, ncols_out, \
+                                               s, dt);
   switch (M) {
     LP_ROW_LENGTHS(CASE)
     default: return hipErrorInvalidValue;
@@ -649,74 +705,85 @@ hipError_t row_r2c(Dt dt, int M, const void *in, long in_pitch, long in_plane, i
 #undef CASE
 }
 
-template <typename T, typename TO, int M, int EPI = 0>
-static hipError_t launch_c2r(const void *in, long in_pitch, long in_plane, int ncols_in, int rows,
-                             int nplanes, void *out, long out_pitch, long out_plane, hipStream_t s, Dt dt,
-                             const void *tz = nullptr, double cst = 0.0, const double *ikx = nullptr,
-                             const double *shift = nullptr) {
+template <typename T, typename TO, int M, int N, bool DIV>
+static hipError_t launch_c2r_n(const C2rSet *sets, int n, long in_pitch, long in_plane, int ncols_in, int rows,
+                             long out_pitch, long out_plane, hipStream_t s, Dt dt, const double *ikx, double cst) {
   const void *twM = tw_ptr(M, dt), *twN = tw_ptr(2 * M, dt);
-  if (!twM || !twN) return hipErrorInvalidValue;
-  constexpr int RPB = row_block<T>() / row_lanes(M);
-  long total = (long)rows * nplanes;
+  constexpr int P = row_lanes(M), RPB = row_block<T>() / P;
+  if (!twM || !twN || n < 1 || n > N || rows < 1 || rows % (64 / P) != 0) return hipErrorInvalidValue;
   const int xorder = xcd_order<T>() && rows % RPB == 0 ? 1 : 0;
-  dim3 grid((unsigned)(xorder ? 8L * xcd_planes(nplanes, 0) * (rows / RPB) : (total + RPB - 1) / RPB));
+  Sets<C2rArg<T, TO>, N> A{};
+  long planes = 0, groups = 0;
+  for (int f = 0; f < N; ++f) {
+    A.first[f] = INT_MAX;
+    if (f >= n) continue;
+    const C2rSet &x = sets[f];
+    if (x.nplanes < 1 || (DIV && (!x.tz || x.nplanes < 2))) return hipErrorInvalidValue;
+    A.first[f] = (int)(xorder ? groups : planes);
+    A.s[f] = C2rArg<T, TO>{(const cx<T> *)x.in, (TO *)x.out, x.nplanes, x.div == 2 ? 1 : 0, (const TO *)x.tz, x.shift};
+    planes += x.nplanes;
+    groups += xcd_planes(x.nplanes, 0);
+  }
+  const long total = (long)rows * planes;
+  if (total > INT_MAX) return hipErrorInvalidValue;
+  dim3 grid((unsigned)(xorder ? 8L * groups * (rows / RPB) : (total + RPB - 1) / RPB));
   // the x derivative is its own kernel: the plain transform then holds no multiplier
   // registers
   if (ikx) {
-    if constexpr (EPI != 0) return hipErrorInvalidValue;  // no caller asks for both
+    if constexpr (DIV) return hipErrorInvalidValue;  // no caller asks for both
     else
-      hipLaunchKernelGGL((k_row_c2r<T, TO, M, EPI, true>), grid, dim3(row_block<T>()), 0, s, (const cx<T> *)in,
-                         in_pitch, in_plane, ncols_in, rows, nplanes, (TO *)out, out_pitch, out_plane,
-                         (const cx<T> *)twM, (const cx<T> *)twN, (const TO *)out, (TO)cst, ikx, shift, xorder);
+      hipLaunchKernelGGL((k_row_c2r<T, TO, M, N, DIV, true>), grid, dim3(row_block<T>()), 0, s, A, in_pitch, in_plane,
+                         ncols_in, (unsigned)rows, (unsigned)total, out_pitch, out_plane, (const cx<T> *)twM,
+                         (const cx<T> *)twN, (TO)cst, ikx, xorder);
   } else
-    hipLaunchKernelGGL((k_row_c2r<T, TO, M, EPI, false>), grid, dim3(row_block<T>()), 0, s, (const cx<T> *)in,
-                       in_pitch, in_plane, ncols_in, rows, nplanes, (TO *)out, out_pitch, out_plane,
-                       (const cx<T> *)twM, (const cx<T> *)twN, (const TO *)(EPI ? tz : out), (TO)cst, nullptr,
-                       shift, xorder);
+    hipLaunchKernelGGL((k_row_c2r<T, TO, M, N, DIV, false>), grid, dim3(row_block<T>()), 0, s, A, in_pitch, in_plane,
+                       ncols_in, (unsigned)rows, (unsigned)total, out_pitch, out_plane, (const cx<T> *)twM,
+                       (const cx<T> *)twN, (TO)cst, nullptr, xorder);
   return hipGetLastError();
 }
 
-hipError_t row_c2r_div(Dt dt, int M, const void *in, long in_pitch, long in_plane, int ncols_in, int rows,
-                       int nplanes, void *out, long out_pitch, long out_plane, const void *tz, double cst,
-                       int is_w, hipStream_t s) {
-  if (!tz || nplanes < 2 || out_pitch < 2 * M) return hipErrorInvalidValue;
-#define CASE(m)                                                                                          \
-  case m:                                                                                                \
-    if (dt == F64)                                                                                       \
-      return is_w ? launch_c2r<double, double, m, 2>(in, in_pitch, in_plane, ncols_in, rows, nplanes,    \
-                                                     out, out_pitch, out_plane, s, dt, tz, cst)          \
-                  : launch_c2r<double, double, m, 1>(in, in_pitch, in_plane, ncols_in, rows, nplanes,    \
-                                                     out, out_pitch, out_plane, s, dt, tz, cst);         \
-    return is_w ? launch_c2r<float, float, m, 2>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,   \
-                                                 out_pitch, out_plane, s, dt, tz, cst)                   \
-                : launch_c2r<float, float, m, 1>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,   \
-                                                 out_pitch, out_plane, s, dt, tz, cst);
-  switch (M) {
-    LP_SMALL_ROW_LENGTHS(CASE)
-    default: return hipErrorInvalidValue;
-  }
-#undef CASE
+template <typename T, typename TO, int M, bool DIV = false>
+static hipError_t launch_c2r(const C2rSet *sets, int n, long in_pitch, long in_plane, int ncols_in, int rows,
+                             long out_pitch, long out_plane, hipStream_t s, Dt dt, const double *ikx, double cst) {
+  return n == 1 ? launch_c2r_n<T, TO, M, 1, DIV>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s,
+                                                 dt, ikx, cst)
+                : launch_c2r_n<T, TO, M, kMaxSets, DIV>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch,
+                                                        out_plane, s, dt, ikx, cst);
 }
 
-hipError_t row_c2r(Dt dtc, Dt dto, int M, const void *in, long in_pitch, long in_plane, int ncols_in,
-                   int rows, int nplanes, void *out, long out_pitch, long out_plane, hipStream_t s,
-                   const double *ikx, const double *shift) {
-  if (shift && !(dtc == F32 && dto == F64)) return hipErrorInvalidValue;
-#define CASE(m)                                                                                         \
-  case m:                                                                                               \
-    if (dtc == F64 && dto == F64)                                                                       \
-      return launch_c2r<double, double, m>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,        \
-                                           out_pitch, out_plane, s, dtc, nullptr, 0.0, ikx);            \
-    if (dtc == F64 && dto == F32)                                                                       \
-      return launch_c2r<double, float, m>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,         \
-                                          out_pitch, out_plane, s, dtc, nullptr, 0.0, ikx);             \
-    if (dtc == F32 && dto == F32)                                                                       \
-      return launch_c2r<float, float, m>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,          \
-                                         out_pitch, out_plane, s, dtc, nullptr, 0.0, ikx);              \
-    if (dtc == F32 && dto == F64)                                                                       \
-      return launch_c2r<float, double, m>(in, in_pitch, in_plane, ncols_in, rows, nplanes, out,         \
-                                          out_pitch, out_plane, s, dtc, nullptr, 0.0, ikx, shift);      \
-    return hipErrorInvalidValue;
+hipError_t row_c2r(Dt dtc, Dt dto, int M, const C2rSet *sets, int n, long in_pitch, long in_plane, int ncols_in,
+                   int rows, long out_pitch, long out_plane, hipStream_t s, const double *ikx, double cst) {
+  if (n < 1) return hipErrorInvalidValue;
+  const bool div = sets[0].div != 0;
+  for (int f = 0; f < n; ++f)
+    if ((sets[f].div != 0) != div || (sets[f].shift && !(dtc == F32 && dto == F64))) return hipErrorInvalidValue;
+  if (div) {
+    if (dtc != dto || ikx || out_pitch < 2 * M) return hipErrorInvalidValue;
+#define CASE(m)                                                                                                   \
+  case m:                                                                                                         \
+    return dtc == F64 ? launch_c2r<double, double, m, true>(sets, n, in_pitch, in_plane, ncols_in, rows,          \
+                                                            out_pitch, out_plane, s, dtc, nullptr, cst)           \
+                      : launch_c2r<float, float, m, true>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, \
+                                                          out_plane, s, dtc, nullptr, cst);
+    switch (M) {
+      LP_SMALL_ROW_LENGTHS(CASE)
+      default: return hipErrorInvalidValue;
+    }
+#undef CASE
+  }
+#define CASE(m)                                                                                                     \
+  case m:                                                                                                           \
+    if (dtc == F64 && dto == F64)                                                                                   \
+      return launch_c2r<double, double, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s,    \
+                                           dtc, ikx, cst);                                                          \
+    if (dtc == F64 && dto == F32)                                                                                   \
+      return launch_c2r<double, float, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s,     \
+                                          dtc, ikx, cst);                                                           \
+    if (dtc == F32 && dto == F32)                                                                                   \
+      return launch_c2r<float, float, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s, dtc, \
+                                         ikx, cst);                                                                 \
+    return launch_c2r<float, double, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s, dtc,  \
+                                        ikx, cst);
   switch (M) {
     LP_ROW_LENGTHS(CASE)
     default: return hipErrorInvalidValue;
@@ -725,59 +792,75 @@ hipError_t row_c2r(Dt dtc, Dt dto, int M, const void *in, long in_pitch, long in
 }
 
 // col0 > 0: the columns col0..ncols-1 only (same grid, one column per block)
-template <typename T, int NYI, int NYO>
-static hipError_t launch_col(int padmode, int fwd, int inv, const void *in, long in_pitch, long in_plane,
-                             int ncols, int nplanes, int nout, const ColOut *outs, long out_pitch,
-                             long out_plane, const SpecTables &tab, hipStream_t s, Dt dt, int col0 = 0,
-                             LaunchEv ev = {}) {
+template <typename T, int NYI, int NYO, int N>
+static hipError_t launch_col_n(int padmode, int fwd, int inv, const ColSet *sets, int n, long in_pitch, long in_plane,
+                               int ncols, long out_pitch, long out_plane, const SpecTables &tab, hipStream_t s,
+                               Dt dt, int col0, LaunchEv ev) {
   const void *twI = tw_ptr(NYI, dt), *twO = tw_ptr(NYO, dt);
-  if (!twI || !twO || col0 < 0 || col0 >= ncols) return hipErrorInvalidValue;
+  if (!twI || !twO || n < 1 || n > N || col0 < 0 || col0 >= ncols) return hipErrorInvalidValue;
   // the map is fixed by the lengths: same grid (0), padd (1), unpadd (2)
   if (padmode != (NYI == NYO ? 0 : (NYO > NYI ? 1 : 2))) return hipErrorInvalidValue;
   constexpr int TX = col_tx<T>();
-  ColParams P;
-  P.nout = nout;
-  for (int j = 0; j < 3; ++j) {
-    if (j >= nout) {
-      P.outs[j] = ColSlot{nullptr, 0, 0, 0, 0, 0, 1.0};
-      continue;
+  Sets<ColArg, N> P{};
+  long planes = 0, groups = 0;
+  for (int f = 0; f < N; ++f) {
+    P.first[f] = INT_MAX;
+    if (f >= n) continue;
+    const ColSet &x = sets[f];
+    if (x.nplanes < 1 || x.nout < 1 || x.nout > 3 || (x.dc && padmode != 1)) return hipErrorInvalidValue;
+    P.first[f] = (int)(xcd_order<T>() ? groups : planes);
+    ColArg &A = P.s[f];
+    A.in = x.in;
+    A.dc = x.dc;
+    A.np = x.nplanes;
+    A.nout = x.nout;
+    for (int j = 0; j < x.nout; ++j) {
+      const ColOut &o = x.outs[j];
+      if (padmode == 0 && o.scale != 1.0) return hipErrorInvalidValue;
+      const long pl = o.plane ? o.plane : out_plane;
+      if (pl > INT_MAX) return hipErrorInvalidValue;
+      A.outs[j] = ColSlot{o.ptr, o.scale, (int)(o.pitch ? o.pitch : out_pitch), (int)pl, o.mult,
+                          o.ncols ? o.ncols : ncols};
     }
-    const ColOut &o = outs[j];
-    if (padmode == 0 && o.scale != 1.0) return hipErrorInvalidValue;
-    P.outs[j] = ColSlot{o.ptr, o.pitch ? o.pitch : out_pitch, o.plane ? o.plane : out_plane, o.mult, tab.lh,
-                        o.ncols ? o.ncols : ncols, o.scale};
+    planes += x.nplanes;
+    groups += xcd_planes(x.nplanes, 0);
   }
+  const unsigned gy = (unsigned)(xcd_order<T>() ? 8 * groups : planes);
+  if (gy > 65535u) return hipErrorInvalidValue;
   if (col0 > 0) {
     if constexpr (NYI == NYO) {
-      dim3 grid((unsigned)(ncols - col0), (unsigned)(xcd_order<T>() ? 8 * xcd_planes(nplanes, 0) : nplanes));
-      hipExtLaunchKernelGGL((k_col_op<T, NYI, NYO, 1>), grid, dim3(kColLanes), 0, s, ev.start, ev.stop, 0,
-                            (const cx<T> *)in, in_pitch, in_plane, ncols, fwd, inv, P, out_pitch, out_plane,
-                            tab.kx, tab.ky, tab.G1, tab.G2, tab.lh, tab.ny, (const cx<T> *)twI,
-                            (const cx<T> *)twO, col0, nplanes);
+      hipExtLaunchKernelGGL((k_col_op<T, NYI, NYO, N, 1>), dim3((unsigned)(ncols - col0), gy), dim3(kColLanes), 0, s,
+                            ev.start, ev.stop, 0, P, (int)groups, in_pitch, in_plane, ncols, fwd, inv, tab.kx, tab.ky, tab.G1,
+                            tab.G2, tab.lh, tab.ny, (const cx<T> *)twI, (const cx<T> *)twO, col0);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
     }
   }
-  dim3 grid((unsigned)((ncols + TX - 1) / TX),
-            (unsigned)(xcd_order<T>() ? 8 * xcd_planes(nplanes, 0) : nplanes));
-  hipExtLaunchKernelGGL((k_col_op<T, NYI, NYO>), grid, dim3(TX * kColLanes), 0, s, ev.start, ev.stop, 0,
-                        (const cx<T> *)in, in_pitch, in_plane, ncols, fwd, inv, P, out_pitch, out_plane, tab.kx,
-                        tab.ky, tab.G1, tab.G2, tab.lh, tab.ny, (const cx<T> *)twI, (const cx<T> *)twO, 0,
-                        nplanes);
+  hipExtLaunchKernelGGL((k_col_op<T, NYI, NYO, N>), dim3((unsigned)((ncols + TX - 1) / TX), gy), dim3(TX * kColLanes), 0,
+                        s, ev.start, ev.stop, 0, P, (int)groups, in_pitch, in_plane, ncols, fwd, inv, tab.kx, tab.ky, tab.G1,
+                        tab.G2, tab.lh, tab.ny, (const cx<T> *)twI, (const cx<T> *)twO, 0);
   return hipGetLastError();
 }
 
-hipError_t col_op_tail(Dt dt, int ny, const void *in, long in_pitch, long in_plane, int col0, int ncols,
-                       int nplanes, int nout, const ColOut *outs, long out_pitch, long out_plane,
-                       const SpecTables &tab, hipStream_t s, LaunchEv ev) {
-  if (nout < 1 || nout > 3) return hipErrorInvalidValue;
-#define CASE(n)                                                                                          \
-  case n:                                                                                                \
-    return dt == F64 ? launch_col<double, n, n>(0, 1, 1, in, in_pitch, in_plane, ncols, nplanes, nout,  \
-                                                outs, out_pitch, out_plane, tab, s, dt, col0, ev)       \
-                     : launch_col<float, n, n>(0, 1, 1, in, in_pitch, in_plane, ncols, nplanes, nout,   \
-                                               outs, out_pitch, out_plane, tab, s, dt, col0, ev);
+template <typename T, int NYI, int NYO>
+static hipError_t launch_col(int padmode, int fwd, int inv, const ColSet *sets, int n, long in_pitch, long in_plane,
+                             int ncols, long out_pitch, long out_plane, const SpecTables &tab, hipStream_t s, Dt dt,
+                             int col0 = 0, LaunchEv ev = {}) {
+  return n == 1 ? launch_col_n<T, NYI, NYO, 1>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols, out_pitch,
+                                               out_plane, tab, s, dt, col0, ev)
+                : launch_col_n<T, NYI, NYO, kMaxSets>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols,
+                                                      out_pitch, out_plane, tab, s, dt, col0, ev);
+}
+
+hipError_t col_op_tail(Dt dt, int ny, const ColSet &set, long in_pitch, long in_plane, int col0, int ncols,
+                       long out_pitch, long out_plane, const SpecTables &tab, hipStream_t s, LaunchEv ev) {
+#define CASE(n)                                                                                                  \
+  case n:                                                                                                        \
+    return dt == F64 ? launch_col<double, n, n>(0, 1, 1, &set, 1, in_pitch, in_plane, ncols, out_pitch,          \
+                                                out_plane, tab, s, dt, col0, ev)                                 \
+                     : launch_col<float, n, n>(0, 1, 1, &set, 1, in_pitch, in_plane, ncols, out_pitch,           \
+                                               out_plane, tab, s, dt, col0, ev);
   switch (ny) {
     CASE(32) CASE(48) CASE(64) CASE(96) CASE(128) CASE(144) CASE(192) CASE(256) CASE(288) CASE(384)
     default: return hipErrorInvalidValue;
@@ -785,26 +868,19 @@ hipError_t col_op_tail(Dt dt, int ny, const void *in, long in_pitch, long in_pla
 #undef CASE
 }
 
-hipError_t col_op(Dt dt, int nyi, int nyo, int padmode, int fwd, int inv, const void *in, long in_pitch,
-                  long in_plane, int ncols, int nplanes, int nout, const ColOut *outs, long out_pitch,
-                  long out_plane, const SpecTables &tab, hipStream_t s, LaunchEv ev) {
-  if (nout < 1 || nout > 3) return hipErrorInvalidValue;
-#define SAME(n)                                                                                         \
-  if (nyi == n && nyo == n)                                                                             \
-    return dt == F64 ? launch_col<double, n, n>(padmode, fwd, inv, in, in_pitch, in_plane, ncols,       \
-                                                nplanes, nout, outs, out_pitch, out_plane, tab, s, dt, 0, ev) \
-                     : launch_col<float, n, n>(padmode, fwd, inv, in, in_pitch, in_plane, ncols,        \
-                                               nplanes, nout, outs, out_pitch, out_plane, tab, s, dt, 0, ev);
-#define PAIR(a, b)                                                                                      \
-  if (nyi == a && nyo == b)                                                                             \
-    return dt == F64 ? launch_col<double, a, b>(padmode, fwd, inv, in, in_pitch, in_plane, ncols,       \
-                                                nplanes, nout, outs, out_pitch, out_plane, tab, s, dt, 0, ev) \
-                     : launch_col<float, a, b>(padmode, fwd, inv, in, in_pitch, in_plane, ncols,        \
-                                               nplanes, nout, outs, out_pitch, out_plane, tab, s, dt, 0, ev);
-  SAME(32) SAME(48) SAME(64) SAME(96) SAME(128) SAME(144) SAME(192) SAME(256) SAME(288) SAME(384)
+hipError_t col_op(Dt dt, int nyi, int nyo, int padmode, int fwd, int inv, const ColSet *sets, int n, long in_pitch,
+                  long in_plane, int ncols, long out_pitch, long out_plane, const SpecTables &tab, hipStream_t s,
+                  LaunchEv ev) {
+#define PAIR(a, b)                                                                                            \
+  if (nyi == a && nyo == b)                                                                                   \
+    return dt == F64 ? launch_col<double, a, b>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols,        \
+                                                out_pitch, out_plane, tab, s, dt, 0, ev)                      \
+                     : launch_col<float, a, b>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols,         \
+                                               out_pitch, out_plane, tab, s, dt, 0, ev);
+  PAIR(32, 32) PAIR(48, 48) PAIR(64, 64) PAIR(96, 96) PAIR(128, 128) PAIR(144, 144) PAIR(192, 192) PAIR(256, 256)
+  PAIR(288, 288) PAIR(384, 384)
   PAIR(32, 48) PAIR(48, 32) PAIR(64, 96) PAIR(96, 64) PAIR(96, 144) PAIR(144, 96)
   PAIR(128, 192) PAIR(192, 128) PAIR(192, 288) PAIR(288, 192) PAIR(256, 384) PAIR(384, 256)
-#undef SAME
 #undef PAIR
   return hipErrorInvalidValue;
 }

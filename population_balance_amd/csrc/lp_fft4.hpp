@@ -16,6 +16,8 @@
 #pragma once
 #include "lp_device.hpp"
 
+#pragma clang fp contract(off)  // see lp_device.hpp
+
 namespace lp {
 
 // exp(-2*pi*i*m/144), rounded to binary64 from 40-digit values
@@ -79,7 +81,7 @@ template <typename T, int R, int SIGN> struct Dft {
     } else if constexpr (R == 2 || R == 3 || R == 4) {
       SmallDft<T, R, SIGN>::run(v);
     } else {
-      constexpr int A = (R % 4 == 0) ? 4 : (R % 2 == 0) ? 2 : 3;
+      constexpr int A = (R == 8) ? 2 : (R == 12) ? 3 : (R % 4 == 0) ? 4 : (R % 2 == 0) ? 2 : 3;
       constexpr int B = R / A;
       cx<T> y[A][B];
 #pragma unroll
@@ -135,4 +137,30 @@ template <typename T, int N, int P, int SIGN> struct Fft4 {
   }
 };
 
+// merge of the half spectrum into the M-point complex input of a 2M-point real inverse
+// transform: Y[k] = (X[k] + conj X[M-k]) + i w^-k (X[k] - conj X[M-k]), w = exp(-2 pi i/2M).
+// CHAIN: the product is accumulated onto the sum (4 fused operations instead of 2 products,
+// 2 fused operations and 2 sums), for the kernels that are bound by VALU issue.
+template <bool CHAIN, typename T> __device__ __forceinline__ cx<T> merge_c2r(cx<T> xa, cx<T> xm, cx<T> w) {
+  const cx<T> xb = conjg(xm);
+  const cx<T> e = xa + xb, o = xa - xb;
+  if constexpr (CHAIN)
+    return mk<T>(fmadd(-w.x, o.y, fmadd(w.y, o.x, e.x)), fmadd(w.x, o.x, fmadd(w.y, o.y, e.y)));
+  const cx<T> wo = cmul(conjg(w), o);
+  return mk<T>(e.x - wo.y, e.y + wo.x);
+}
+
+// split of the M-point complex transform Z of a row of 2M reals:
+// X[k] = (Z[k] + conj Z[M-k])/2 - i/2 w^k (Z[k] - conj Z[M-k]), w = exp(-2 pi i/2M)
+template <bool CHAIN, typename T> __device__ __forceinline__ cx<T> split_r2c(cx<T> za, cx<T> zm, cx<T> w) {
+  const cx<T> zb = conjg(zm);
+  const cx<T> e = za + zb, o = za - zb;
+  if constexpr (CHAIN)
+    return mk<T>(T(0.5) * fmadd(w.x, o.y, fmadd(w.y, o.x, e.x)), T(0.5) * fmadd(w.y, o.y, fmadd(-w.x, o.x, e.y)));
+  const cx<T> wo = cmul(w, o);
+  return mk<T>(T(0.5) * (e.x + wo.y), T(0.5) * (e.y - wo.x));
+}
+
 }  // namespace lp
+
+#pragma clang fp contract(fast)

@@ -35,16 +35,24 @@ __global__ void k_ddz_w(T *__restrict__ dfdz, const TI *__restrict__ f, Geo g, T
   else if (x < g.nx) dfdz[i] = (T)(cst * (f[i + g.np] - f[i]));
 }
 
-// the kx = 0 column of x-spectra in physical y ([nplanes][ny][pitch] complex): add a
-// per-plane value to the real part of every y, i.e. to the plane's mean (the inverse of
-// row_r2c's shift on a spectrum that keeps the row means there)
+// the velocities' three z-derivatives (blockIdx.y: u, v by ddz_uv, w by ddz_w), formed in
+// binary64 and stored in T
 template <typename T>
-__global__ void k_add_dc(cx<T> *__restrict__ spec, long pitch, int ny, int nplanes, const double *__restrict__ dc) {
-  long i = gtid();
-  if (i >= (long)ny * nplanes) return;
-  const int k = (int)(i / ny);
-  cx<T> &e = spec[i * pitch];
-  e.x = (T)((double)e.x + dc[k]);
+__global__ void k_ddz_vel(T *__restrict__ dudz, T *__restrict__ dvdz, T *__restrict__ dwdz,
+                          const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w,
+                          Geo g, double cst) {
+  const long i = gtid();
+  if (i >= g.np * g.nz) return;
+  const int q = blockIdx.y;
+  const int k = (int)(i / g.np), x = (int)(i % g.ld);
+  T *d = q == 0 ? dudz : q == 1 ? dvdz : dwdz;
+  const double *f = q == 0 ? u : q == 1 ? v : w;
+  if (k == g.nz - 1) {
+    d[i] = T(0);
+  } else if (x < g.nx) {
+    if (q == 2) d[i] = (T)(cst * (f[i + g.np] - f[i]));
+    else if (k >= 1) d[i] = (T)(cst * (f[i] - f[i - g.np]));
+  }
 }
 
 // filt_da.f90's zeroing of the kx = nx/2 and ky = ny/2 modes ("oddballs") on a binary64
@@ -62,8 +70,16 @@ constexpr int kNyqMax = 384;  // largest nx, ny of the transforms
 // partials added in LDS); k_nyq_fin adds the slices' partials in slice order for B and
 // forms C from A.  Every sum has a fixed order: the result does not depend on timing.
 constexpr int kNyqSlices = 16, kNyqRU = 4;
-static __global__ __launch_bounds__(256) void k_nyq_part(const double *__restrict__ f, double *__restrict__ A,
-                                                         double *__restrict__ P, Geo g) {
+// up to three fields a launch (blockIdx.y); A [3][nz][ny], B [3][nz][nx], C [3][nz],
+// P [3][nz][kNyqSlices][nx]
+struct NyqFields {
+  double *f[3];
+  double *A, *B, *C, *P;
+};
+static __global__ __launch_bounds__(256) void k_nyq_part(NyqFields N, Geo g) {
+  const double *__restrict__ f = N.f[blockIdx.y];
+  double *__restrict__ A = N.A + (long)blockIdx.y * g.nz * g.ny;
+  double *__restrict__ P = N.P + (long)blockIdx.y * g.nz * kNyqSlices * g.nx;
   __shared__ double colp[4][kNyqMax];
   const int lane = threadIdx.x % 64, grp = threadIdx.x / 64;
   const int k = blockIdx.x / kNyqSlices, sl = blockIdx.x % kNyqSlices;
@@ -111,8 +127,10 @@ static __global__ __launch_bounds__(256) void k_nyq_part(const double *__restric
     P[((long)k * kNyqSlices + sl) * g.nx + x] = s;
   }
 }
-static __global__ __launch_bounds__(256) void k_nyq_fin(const double *__restrict__ A, const double *__restrict__ P,
-                                                        double *__restrict__ B, double *__restrict__ Cc, Geo g) {
+static __global__ __launch_bounds__(256) void k_nyq_fin(NyqFields N, Geo g) {
+  const double *__restrict__ A = N.A + (long)blockIdx.y * g.nz * g.ny;
+  const double *__restrict__ P = N.P + (long)blockIdx.y * g.nz * kNyqSlices * g.nx;
+  double *__restrict__ B = N.B + (long)blockIdx.y * g.nz * g.nx, *__restrict__ Cc = N.C + (long)blockIdx.y * g.nz;
   const int k = blockIdx.x;
   for (int x = threadIdx.x; x < g.nx; x += blockDim.x) {
     double s = 0.0;
@@ -133,8 +151,11 @@ static __global__ __launch_bounds__(256) void k_nyq_fin(const double *__restrict
 }
 
 // f -= the oddball modes (padding columns x >= nx set to zero, as a back-transform leaves them)
-static __global__ void k_nyq_remove(double *__restrict__ f, const double *__restrict__ A, const double *__restrict__ B,
-                             const double *__restrict__ Cc, Geo g, int nlev) {
+static __global__ void k_nyq_remove(NyqFields N, Geo g, int nlev) {
+  double *__restrict__ f = N.f[blockIdx.y];
+  const double *__restrict__ A = N.A + (long)blockIdx.y * g.nz * g.ny;
+  const double *__restrict__ B = N.B + (long)blockIdx.y * g.nz * g.nx;
+  const double *__restrict__ Cc = N.C + (long)blockIdx.y * g.nz;
   const long i = gtid();
   if (i >= g.np * nlev) return;
   const int x = (int)(i % g.ld), y = (int)((i / g.ld) % g.ny), k = (int)(i / g.np);
@@ -177,6 +198,24 @@ template <typename T>
 __global__ void k_fill(T *__restrict__ a, long n, T v) {
   long i = gtid();
   if (i < n) a[i] = v;
+}
+
+template <typename T> struct Fill3 {
+  T *p[3];
+};
+template <typename T>
+__global__ void k_fill3(Fill3<T> F, long n, T v) {
+  const long i = gtid();
+  if (i < n) F.p[blockIdx.y][i] = v;
+}
+// press_stag_array.f90:355-357: the BOGUS top levels of p, dpdx, dpdy
+template <typename T>
+__global__ void k_press_tops(double *__restrict__ p, T *__restrict__ dpdx, T *__restrict__ dpdy, long n) {
+  const long i = gtid();
+  if (i >= n) return;
+  p[i] = LP_BOGUS;
+  dpdx[i] = (T)LP_BOGUS;
+  dpdy[i] = (T)LP_BOGUS;
 }
 
 template <typename T> __device__ __forceinline__ T smag(T s11, T s12, T s13, T s22, T s23, T s33) {

@@ -159,10 +159,7 @@ __global__ __launch_bounds__(256) void k_lag_r2c(LagIn<T> in, Geo g, cx<T> *__re
     if (act) {  // split (as k_row_r2c), leading nc columns
       cx<T> *dst = spec + (((long)q * g.nz + k) * g.ny + y) * pitch;
       for (int kk = t; kk < nc; kk += P) {
-        cx<T> za = sc[kk % M], zb = conjg(sc[(M - kk) % M]);
-        cx<T> e = za + zb, o = za - zb;
-        cx<T> wo = cmul(tws[M + kk], o);
-        dst[kk] = mk<T>(T(0.5) * (e.x + wo.y), T(0.5) * (e.y - wo.x));
+        dst[kk] = split_r2c<true>(sc[kk % M], sc[(M - kk) % M], tws[M + kk]);
       }
     }
     slot_sync<P>();
@@ -206,8 +203,7 @@ __global__ __launch_bounds__(256) void k_lag_c2r_contract(const cx<T> *__restric
   // twiddles in LDS, behind the transforms' slots (2M values, read by every lane)
   cx<T> *tw = reinterpret_cast<cx<T> *>(smem + tw_off);
   for (int i = threadIdx.x; i < 2 * M; i += blockDim.x) tw[i] = i < M ? twM[i] : twN[i - M];
-  // merge (as k_row_c2r): Y[k] = (X[k] + conj X[M-k]) + i w^-k (X[k] - conj X[M-k]).  The
-  // loads of a q2 whose columns all lie at or past nin for every lane are skipped by a
+  // merge (as k_row_c2r).  The loads of a q2 whose columns all lie at or past nin for every lane are skipped by a
   // uniform branch.
   cx<T> xa_[Q], xb_[Q];
 #pragma unroll
@@ -229,10 +225,7 @@ __global__ __launch_bounds__(256) void k_lag_c2r_contract(const cx<T> *__restric
     const int kk = t + PL * q2;
     cx<T> xa = xa_[q2], xb = xb_[q2];
     if (kk == 0) { xa.y = 0; xb.y = 0; }  // X[0] and X[M] (M - kk == M only for kk == 0)
-    xb = conjg(xb);
-    cx<T> e = xa + xb, o = xa - xb;
-    cx<T> wo = cmul(conjg(tw[M + kk]), o);
-    v[q2] = mk<T>(e.x - wo.y, e.y + wo.x);
+    v[q2] = merge_c2r<true>(xa, xb, tw[M + kk]);
   }
   cx<T> *sc = scr + (act ? slot : 0) * SS;
   if (act) F::stage1(v, t, sc, tw);

@@ -107,3 +107,29 @@ def test_adjoint_row_segments(nz):
     print()
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,kw", [(96, 32, 10, {}), (64, 96, 9, {"lbc_mom": abi.LP_LBC_STRESS_FREE}),
+                                         (32, 192, 13, {"model": 4})])
+def test_steps_uneven(nx, ny, nz, kw):
+    """whole binary64 steps with the passes over several fields in one launch, at level
+    counts that leave the last group of eight planes of each field part full"""
+    from harness import load_gpu, load_oracle, seeded_state
+    from oracle import Oracle
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(nx, ny, nz, **kw)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    print(f"\n[case] steps uneven {nx}x{ny}x{nz} {kw}", flush=True)
+    st = seeded_state(cfg)
+    load_oracle(o, st)
+    load_gpu(lg, st)
+    for _ in range(3):
+        o.step(1)
+        lg.step(1)
+    for n, top in [(n, nz - 1) for n in ("u", "v", "w", "RHSx", "RHSy", "RHSz")] + [("p", nz)]:
+        err = rel_l2(lg.download(n)[:top], o.field(n)[:top], nx)
+        print(f"  {n}: {err:.2e}", end="")
+        assert err < TOL, (n, err)
+    print()
+    lg.close()
+    o.close()
