@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256) void k_lag_c2r_contract(const cx<T> *__restric
 constexpr int kRx = 64, kRy = 4;  // kRx = one wavefront, kRy wavefronts per block
 constexpr int kHx = kRx + 2, kHy = kRy + 2;
 constexpr int kLagRows = 4 * kHy;  // staged rows of one level: 4 fields x kHy
-constexpr int kRz = 16;            // levels per block, at most (the runs are balanced)
+constexpr int kRz = 8;             // levels per block, at most (the runs are balanced)
 
 // The padding columns x = nx .. ld-1, which interpolag_Sdep.f90 leaves alone: point t of
 // the (ld - nx) ny nz padding points is relaxed from its old values (no interpolation).
@@ -562,7 +562,16 @@ static hipError_t launch_lag_relax(void *const C[4], const double *const Fold[4]
   if (g.ny % kRy != 0 || g.nz < 2) return hipErrorInvalidValue;
   if (P.powcoeff != -0.125 || P.bexp != 1.0) return hipErrorInvalidValue;
   const int ntx = (g.nx + kRx - 1) / kRx, cg = (ntx * (g.ny / kRy) + 7) / 8;
-  const int nkc = (g.nz + kRz - 1) / kRz;  // level runs of nz/nkc levels (rounded)
+  // Level runs: a block takes its levels one after the other (1.4 us each, the latency of
+  // the square roots and divisions) and reads two levels beside its own.  Runs of at most
+  // kRz levels, halved down to 2 while the chip has fewer than two blocks per CU.  Binary64
+  // 32x32x33: 24.4 us in runs of 16, 13.0 of 4, 8.5 of 2; mixed 128x96x50: 30.4 of 16, 28.6
+  // of 8, 24.2 of 4, 26.3 of 2; 192x192x128: 128.6, 121.6, 128.6, 140.8; 256^3: 468, 443,
+  // 447, 500.
+  const long tiles = (long)ntx * (g.ny / kRy);
+  int lev = kRz;
+  while (lev > 2 && tiles * ((g.nz + lev - 1) / lev) < 512) lev /= 2;
+  const int nkc = (g.nz + lev - 1) / lev;
   const long npts = (long)(g.ld - g.nx) * g.ny * g.nz;
   const int npb = (int)((npts + 255) / 256 + 7) / 8 * 8;
   const dim3 grid((unsigned)(npb + 8L * cg * nkc));

@@ -133,3 +133,31 @@ def test_steps_uneven(nx, ny, nz, kw):
     print()
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(32, 32, 4), (32, 32, 5), (96, 32, 7), (128, 64, 65)])
+def test_lag_level_runs(nx, ny, nz):
+    """the Lagrangian relaxation in level runs of 1, 2, 3 and 4 (the 128-point test of fifty
+    steps takes runs of 8): three binary64 steps, each with a new coefficient.  RHS at 1e-11
+    and the coefficient at 1e-6: its averages are rounded to REAL(4) (6e-8 where a last bit
+    of binary64 flips one), the SGS part is some 1e-2 of RHS and a flip one of 4000 points."""
+    from harness import load_gpu, load_oracle, seeded_state
+    from oracle import Oracle
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(nx, ny, nz, cs_count=1)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    print(f"\n[case] lag runs {nx}x{ny}x{nz}", flush=True)
+    st = seeded_state(cfg)
+    load_oracle(o, st)
+    load_gpu(lg, st)
+    for _ in range(3):
+        o.step(1)
+        lg.step(1)
+    for n, top in [(n, nz - 1) for n in ("u", "v", "w", "RHSx", "RHSy", "RHSz")] \
+            + [(n, nz) for n in ("Cs_opt2", "F_LM", "F_QN")]:
+        err = rel_l2(lg.download(n)[:top], o.field(n)[:top], nx)
+        print(f"  {n}: {err:.2e}", end="")
+        assert err < (1e-6 if n[0] in "CF" else 1e-11 if n[0] == "R" else TOL), (n, err)
+    print()
+    lg.close()
+    o.close()
