@@ -490,7 +490,11 @@ static int droplet_setup(lp_ctx *c, Arena &A_) {
     const double V = M_PI / 6 * (dd * dd * dd);
     vfac[b] = gh * (D.rho_c / D.rho_w - 1.0) * V;
   }
-  RCHK(A_.table((void **)&c->d_ws, D.settling_vel, sizeof(double) * n));
+  // settling velocities, then their inertial time scales (:2255)
+  std::vector<double> ws(D.settling_vel, D.settling_vel + n);
+  const double ghat = D.g / (D.u_star * D.u_star / D.z_i);
+  for (int b = 0; b < n; ++b) ws.push_back(ws[b] / ghat);
+  RCHK(A_.table((void **)&c->d_ws, ws.data(), sizeof(double) * 2 * n));
   RCHK(A_.table((void **)&c->d_qsrc, D.Q_src, sizeof(double) * n));
   RCHK(A_.table((void **)&c->d_vfac, vfac.data(), sizeof(double) * n));
   std::vector<double> pvol(n);
@@ -1770,11 +1774,24 @@ static int do_pollen_rhs(lp_ctx *c, const double *prev, bool fuse_step = false, 
   P.src_k0 = D.src_k - 1;
   const double nb = (double)dg.nv * dg.npc * 8.0;
   prof_begin(c, LP_K_POLLEN_RHS);
-  const dim3 pgrid((unsigned)((dg.nv + 255) / 256), (unsigned)((dg.npc + kPollenBins - 1) / kPollenBins));
-  FDISPATCH(c, T, hipLaunchKernelGGL(k_pollen_rhs<T>, pgrid, dim3(256), 0, c->s, PC, RH, prev, c->ui0,
-                                     c->vi0, (const double *)c->f[LP_W], (const T *)c->f[LP_DUDT],
-                                     (const T *)c->f[LP_DVDT], (const T *)c->f[LP_DWDT], c->kcell, c->d_ws,
-                                     c->d_qsrc, c->d_foot, dg, P));
+  const long prow = 256 / pollen_tile(gg.nx), pgrp = (dg.npc + kPollenBins - 1) / kPollenBins;
+  const long pblk = ((gg.ny + prow - 1) / prow * (gg.nx / pollen_tile(gg.nx)) + 7) / 8 * 8;
+  // level runs of at most kPollenLevels, halved down to 2 while there are fewer than two
+  // blocks per CU (a run computes its first face and reads four levels before its own work)
+  int lev = kPollenLevels;
+  while (lev > 2 && pblk * pgrp * ((gg.nz - 1 + lev - 1) / lev) < 512) lev /= 2;
+  const dim3 pgrid((unsigned)(pblk + 8), (unsigned)pgrp, (unsigned)((gg.nz - 1 + lev - 1) / lev));
+  auto rhs = [&](auto kern, auto T_) {
+    using T = decltype(T_);
+    hipLaunchKernelGGL(kern, pgrid, dim3(256), 0, c->s, PC, RH, prev, c->ui0, c->vi0, (const double *)c->f[LP_W],
+                       (const T *)c->f[LP_DUDT], (const T *)c->f[LP_DVDT], (const T *)c->f[LP_DWDT], c->kcell, c->d_ws,
+                       c->d_qsrc, c->d_foot, dg, P);
+  };
+  const bool signs = D.bc_x == 2 || D.bc_y == 2, inert = D.settling && D.inertia;
+  if (signs && inert) FDISPATCH(c, T, rhs(k_pollen_rhs<T, true, true>, T()));
+  else if (signs) FDISPATCH(c, T, rhs(k_pollen_rhs<T, true, false>, T()));
+  else if (inert) FDISPATCH(c, T, rhs(k_pollen_rhs<T, false, true>, T()));
+  else FDISPATCH(c, T, rhs(k_pollen_rhs<T, false, false>, T()));
   HIPCHK(hipGetLastError());
   // PCon read once, RHS_PCon written once, plus the bin-independent inputs
   prof_end(c, LP_K_POLLEN_RHS, 2.0 * nb + (double)dg.nv * (8.0 + 3.0 * esz_of(c->fdt)) + 4.0 * dg.fp * gg.nz * 8.0);

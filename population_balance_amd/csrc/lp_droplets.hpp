@@ -149,189 +149,266 @@ struct PollenParams {
   int src_on, src_k0;       // source active this step; its lower level (0-based)
 };
 
-// pollen_RHS_calc2 at one cell for a group of G bins: face velocities of the bin
-// (:2243-2276), ghosts (:2478-2590), SMART faces (:2877-3475), flux divergence and SGS
-// diffusion (:3559-3677) and the point source (:4222-4256).  A thread takes one point and
-// G consecutive bins (blockIdx.y = bin group), so the bin-independent inputs (face
-// velocities, accelerations, Kc_t) are loaded once per G bins.  Every load of a bin is
-// issued unconditionally from a clamped index and the stencil logic selects among the
-// loaded values; the row and column end values are loaded only where a face or ghost of
-// the row or column end is formed.  Points outside the cells keep the values of the
-// previous RHS: when the caller has moved it to RF (RHS_PCon_f = RHS_PCon, :1521, done by
-// exchanging the two buffers) they are copied back from RF, otherwise (RF null) they are
-// left alone.
-static constexpr int kPollenBins = 8;  // bins per thread
-template <typename T>
-__global__ __launch_bounds__(256) void k_pollen_rhs(
+// Half of the SMART face's correction, psi(r) den / 2 (smart_face): num and den with the sign
+// that makes den positive, and the result with its sign again; 0 where den is 0.
+__device__ __forceinline__ double smart_half(double num, double den) {
+  const unsigned long long m = den > 0.0 ? 0ull : 0x8000000000000000ull;
+  const double n = __longlong_as_double(__double_as_longlong(num) ^ m), d = fabs(den);
+  const double t = fmax(0.0, fmin(fmin(n, 0.375 * n + 0.125 * d), d + d));
+  return __longlong_as_double(__double_as_longlong(t) ^ m);
+}
+
+// The SMART value at the face between cells L and R = L + d0, with the differences across
+// the faces before (dm) and after (dp): smart_face(L, LL, R) for flow from L, and
+// smart_face(R, RR, L) otherwise, where num and den both change sign.
+__device__ __forceinline__ double smart_between(double vel, double L, double R, double dm, double d0, double dp) {
+  const bool fwd = vel >= 0.0;
+  const double h = smart_half(d0, fwd ? dm : dp);
+  return fwd ? L + h : R - h;
+}
+
+// A value at a 32-bit byte offset from a uniform address (the address in scalar registers, no
+// 64-bit vector arithmetic); offsets at or past n bytes read as 0.
+template <typename V> __device__ __forceinline__ V buf_load(const V *base, unsigned n, unsigned bytes) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<V *>(base), 0, (int)n, 0x00027000);
+  if constexpr (sizeof(V) == 8) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(V, (u2)__builtin_amdgcn_raw_buffer_load_b64(r, (int)bytes, 0, 0));
+  } else {
+    return __builtin_bit_cast(V, (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)bytes, 0, 0));
+  }
+}
+
+// pollen_RHS_calc2 at the cells of a run of levels for a group of kPollenBins bins: face
+// velocities of the bin (:2243-2276), ghosts (:2478-2590), SMART faces (:2877-3475), flux
+// divergence and SGS diffusion (:3559-3677) and the point source (:4222-4256).
+//
+// A thread takes one (x, y) and marches up the run of levels blockIdx.z with the
+// concentrations, differences, face values and diffusive fluxes of the last level of its
+// bins (blockIdx.y = group) in registers: a level loads one new value along z and computes
+// one z face instead of two; the bin-independent inputs (face velocities, accelerations,
+// Kc_t) are loaded once per group.  A periodic row or column needs no end cases (its end
+// faces use the face-1 velocity, which is that of face n + 1 too): the neighbours are read
+// at wrapped indices, and the ghosts of the other boundary conditions are loads too.
+// Offsets within a level are 32-bit bytes from uniform addresses.  XCD q (blockIdx.x % 8)
+// takes consecutive tiles of pollen_tile(nx) x (256 / pollen_tile(nx)) points, so that the
+// rows above and below are in its L2, and three of four in the CU's L1.
+// Points outside the cells keep the values of the previous RHS: when the caller has moved
+// it to RF (RHS_PCon_f = RHS_PCon, :1521, done by exchanging the two buffers) the last eight
+// blocks of each run copy them back from RF, otherwise (RF null) they are left alone.
+//
+// 192x192x128, 15 bins with inertia: 705 us for 1.56 GB of HBM traffic (2.2 TB/s).  One
+// point per thread with both faces of each direction and the end cells by branches was
+// bound by its vector instructions (630 per point and bin, now 190) and took 1155 us.  Now
+// the loads through L1 bound it (9 per point and bin and 23 per point and group): without
+// the arithmetic it takes 700 us, without the neighbours along x 590, along y 620, without
+// both 470.  Groups of 3 bins 752, of 4 724, of 5 705 (more do not fit three wavefronts per
+// SIMD); the value two levels up or the next bin's loads in flight early: no gain.
+static constexpr int kPollenBins = 5;   // bins per thread
+__host__ __device__ inline int pollen_tile(int nx) { return nx % 64 == 0 ? 64 : 32; }  // nx % 32 == 0
+static constexpr unsigned kGone = 0xfffffff0u;  // past any level: reads 0
+// levels per run, at most (8: 745 us, 32: 770, 64: 875 at 192x192x128)
+static constexpr int kPollenLevels = 16;
+template <typename T, bool SIGNS, bool INERT>
+__global__ __launch_bounds__(256, SIGNS ? 2 : 3) void k_pollen_rhs(
     const double *__restrict__ PC, double *__restrict__ RH, const double *__restrict__ RF,
     const double *__restrict__ ui0, const double *__restrict__ vi0, const double *__restrict__ w,
     const T *__restrict__ dudt, const T *__restrict__ dvdt, const T *__restrict__ dwdt, const double *__restrict__ kc,
     const double *__restrict__ wsb, const double *__restrict__ qsrc, const double *__restrict__ foot, DropGeo g,
     PollenParams P) {
-  const long s = gtid();
-  const int b0 = blockIdx.y * kPollenBins;  // first bin of the group (uniform)
-  if (s >= g.nv) return;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const long np = g.np, ld = g.ld;
-  const int k = (int)(s / np);
-  const int j = (int)((s % np) / ld);
-  const int i = (int)(s % ld);
-  if (k >= nz - 1 || i >= nx) {
-    if (RF)
-#pragma unroll
-      for (int bb = 0; bb < kPollenBins; ++bb)
-        if (b0 + bb < g.npc) RH[(long)(b0 + bb) * g.nv + s] = RF[(long)(b0 + bb) * g.nv + s];
+  constexpr int G = kPollenBins;
+  constexpr unsigned D = sizeof(double), S = sizeof(T);
+  const int nx = g.nx, ny = g.ny, nz = g.nz, ld = g.ld, np = (int)g.np;
+  const int b0 = blockIdx.y * G;  // first bin of the group (uniform)
+  const int nb = g.npc - b0 < G ? g.npc - b0 : G;
+  const int kb = (int)((long)blockIdx.z * (nz - 1) / gridDim.z), ke = (int)((long)(blockIdx.z + 1) * (nz - 1) / gridDim.z);
+  const int nblk = ((int)gridDim.x - 8) / 8;
+  if ((int)blockIdx.x >= 8 * nblk) {  // points outside the cells
+    if (!RF) return;
+    const int pad = ld - nx, lev = pad * ny;
+    const int n = lev * (ke - kb) + (ke == nz - 1 ? np : 0);
+    for (int t = ((int)blockIdx.x - 8 * nblk) * 256 + (int)threadIdx.x; t < n; t += 8 * 256) {
+      const int k = kb + t / lev, q = t % lev;
+      const long o = t < lev * (ke - kb) ? (long)k * np + (q / pad) * ld + nx + q % pad
+                                         : (long)(nz - 1) * np + (t - lev * (ke - kb));
+      for (int bb = 0; bb < nb; ++bb) RH[(long)(b0 + bb) * g.nv + o] = RF[(long)(b0 + bb) * g.nv + o];
+    }
     return;
   }
-  const int im = (i == 0) ? nx - 1 : i - 1, ip = (i == nx - 1) ? 0 : i + 1;
-  const int jm = (j == 0) ? ny - 1 : j - 1, jp = (j == ny - 1) ? 0 : j + 1;
-  const long row = (long)k * np + (long)j * ld;  // start of this x row
-  const long col = (long)k * np + i;             // start of this y column
-  // clamped neighbour indices (values outside the row / column are selected away below)
-  const int i_m2 = i >= 2 ? i - 2 : 0, i_m1 = i >= 1 ? i - 1 : 0;
-  const int i_p1 = i + 1 <= nx - 1 ? i + 1 : nx - 1, i_p2 = i + 2 <= nx - 1 ? i + 2 : nx - 1;
-  const int j_m2 = j >= 2 ? j - 2 : 0, j_m1 = j >= 1 ? j - 1 : 0;
-  const int j_p1 = j + 1 <= ny - 1 ? j + 1 : ny - 1, j_p2 = j + 2 <= ny - 1 ? j + 2 : ny - 1;
-  const int k_m2 = k >= 2 ? k - 2 : 0, k_m1 = k >= 1 ? k - 1 : 0;
-  const int k_p2 = k + 2 <= nz - 1 ? k + 2 : nz - 1;  // k + 1 <= nz - 1 always
-  const long pl = (long)j * ld + i;                   // offset of this point in a level
-  const bool xends = i <= 1 || i >= nx - 2;           // faces or ghosts of the row ends used
-  const bool yends = j <= 1 || j >= ny - 2;
-  // bin-independent inputs: faces i, i+1 and 1 of the row / column
-  const double *ur = ui0 + (long)k * g.fp + (long)j * ld;
-  const double *vc = vi0 + (long)k * g.fp + i;
-  const double u0 = ur[i], u1 = ur[i + 1], uF = ur[0];
-  const double v0 = vc[(long)j * ld], v1 = vc[(long)(j + 1) * ld], vF = vc[0];
-  const double w0 = (double)w[s], w1 = (double)w[s + np];
-  double ax0 = 0.0, ax1 = 0.0, axF = 0.0, ay0 = 0.0, ay1 = 0.0, ayF = 0.0, az0 = 0.0, az1 = 0.0;
-  const bool inert = P.settling && P.inertia;
-  if (inert) {  // accelerations on the faces (:2255-2270)
-    const T *a = dudt + row;
-    const double am = (double)a[i_m1], a0 = (double)a[i], ap = (double)a[i_p1];
-    const double aL = (double)a[nx - 1], aR = (double)a[0];
-    axF = 0.5 * (aL + aR);
-    ax0 = (i == 0) ? axF : 0.5 * (am + a0);
-    ax1 = (i == nx - 1) ? axF : 0.5 * (a0 + ap);
-    const T *bcol = dvdt + col;
-    const double bm = (double)bcol[(long)j_m1 * ld], bc0 = (double)bcol[(long)j * ld];
-    const double bp = (double)bcol[(long)j_p1 * ld];
-    const double bL = (double)bcol[(long)(ny - 1) * ld], bR = (double)bcol[0];
-    ayF = 0.5 * (bL + bR);
-    ay0 = (j == 0) ? ayF : 0.5 * (bm + bc0);
-    ay1 = (j == ny - 1) ? ayF : 0.5 * (bc0 + bp);
-    az0 = (double)dwdt[s];
-    az1 = (double)dwdt[s + np];
-  }
-  // Kc_t stencil
-  const double K0 = kc[s];
-  const double Kxm = kc[row + im], Kxp = kc[row + ip];
-  const double Kym = kc[col + (long)jm * ld], Kyp = kc[col + (long)jp * ld];
-  const double kzm_v = kc[s - (k > 0 ? np : 0)], kzp_v = kc[s + np];
-  const double Kzm = (k > 0) ? kzm_v : 0.0;
-  const double Kzp = (k < nz - 2) ? kzp_v : 0.0;
-  const bool src_here = P.src_on && (k == P.src_k0 || k == P.src_k0 + 1);
-  const double fsrc = src_here ? foot[(long)j * nx + i] : 0.0;
-  const double fr = (k == P.src_k0) ? P.frac : P.frac1;
-
+  const int tile = (int)(blockIdx.x & 7) * nblk + (int)(blockIdx.x >> 3), tw = pollen_tile(nx), ntx = nx / tw;
+  const int i = tile % ntx * tw + (int)threadIdx.x % tw, j = tile / ntx * (256 / tw) + (int)threadIdx.x / tw;
+  if (j >= ny) return;
+  const int p = j * ld + i;
+  const unsigned lvb = (unsigned)(D * np);  // bytes of a level
+  auto at = [&](const double *base, unsigned bytes) -> double { return buf_load<double>(base, lvb + D * ld, bytes); };
+  auto att = [&](const T *base, unsigned bytes) -> double { return (double)buf_load<T>(base, lvb, bytes); };
+  // byte offsets of binary64 values within a level: this cell, its neighbours around the row
+  // and the column (Kc_t, accelerations)
+  const int r0 = j * ld;
+  const unsigned o = D * p;
+  const unsigned kxm = D * (i == 0 ? r0 + nx - 1 : p - 1), kxp = D * (i == nx - 1 ? r0 : p + 1);
+  const unsigned kym = D * (j == 0 ? (ny - 1) * ld + i : p - ld), kyp = D * (j == ny - 1 ? i : p + ld);
+  // and of the concentrations, the ghosts included: the periodic cell; for an inlet the ghost
+  // is 0 (an offset past the level) or the end cell, for the upwind-sign ghosts the end cell
+  // times 0 or 1 (ghost_x, ghost_y)
+  const int wx = P.bc_x == 0 ? nx : 0, wy = P.bc_y == 0 ? ny : 0;
+  const bool inx = P.bc_x == 1, iny = P.bc_y == 1;
+  auto nb_x = [&](int q) -> unsigned {
+    const int lo = wx ? q + wx : 0, hi = wx ? q - wx : nx - 1, v = q < 0 ? lo : (q >= nx ? hi : q);
+    return (inx & (q < 0)) ? kGone : D * (r0 + v);
+  };
+  auto nb_y = [&](int q) -> unsigned {
+    const int lo = wy ? q + wy : 0, hi = wy ? q - wy : ny - 1, v = q < 0 ? lo : (q >= ny ? hi : q);
+    return (iny & (q >= ny)) ? kGone : D * (v * ld + i);
+  };
+  const unsigned oxmm = nb_x(i - 2), oxm = nb_x(i - 1), oxp = nb_x(i + 1), oxpp = nb_x(i + 2);
+  const unsigned oymm = nb_y(j - 2), oym = nb_y(j - 1), oyp = nb_y(j + 1), oypp = nb_y(j + 2);
+  // the end faces of a row or column that is not periodic carry the ghost
+  const bool xb = P.bc_x != 0 && i == 0, xt = P.bc_x != 0 && i == nx - 1;
+  const bool yb = P.bc_y != 0 && j == 0, yt = P.bc_y != 0 && j == ny - 1;
+  // the z face k of a bin: velocity, value (:3340, :3356: face 0 carries no flux, face 1 is
+  // central for upward flow, the top face nz-1 repeats the value of face nz-2)
+  auto w_at = [&](int k, double wk, T az, double ws, double f) {  // settling at faces 2..nz-1 of the reference
+    const bool in = k >= 1 && k <= nz - 2;  // uniform
+    return wk - (in ? ws : 0.0) - (double)az * (in ? f : 0.0);
+  };
+  auto z_face = [&](int k, double wf, double L, double R, double dm, double d0, double dp) {
+    const double c = smart_between(wf, L, R, dm, d0, dp);
+    return k == 1 && wf >= 0.0 ? (R + L) / 2.0 : c;
+  };
+  // state of the run at the bottom face of level kb
+  double c0[G], c1[G], d0z[G], zf[G], zd[G];
+  double K0 = at(kc + (long)kb * np, o), w0 = at(w + (long)kb * np, o);
+  T az0 = INERT ? buf_load<T>(dwdt + (long)kb * np, lvb, o / (D / S)) : T(0);
+  const double Kz0 = kb > 0 ? at(kc + (long)(kb - 1) * np, o) : 0.0;
 #pragma unroll
-  for (int bb = 0; bb < kPollenBins; ++bb) {
-    const int b = b0 + bb;
-    if (b >= g.npc) break;
-    // this bin's concentrations
-    const double *C = PC + (long)b * g.nv;
-    const double ci = C[s];
-    const double cx_m2 = C[row + i_m2], cx_m1 = C[row + i_m1], cx_p1 = C[row + i_p1], cx_p2 = C[row + i_p2];
-    const double cy_m2 = C[col + (long)j_m2 * ld], cy_m1 = C[col + (long)j_m1 * ld];
-    const double cy_p1 = C[col + (long)j_p1 * ld], cy_p2 = C[col + (long)j_p2 * ld];
-    const double cz_m2 = C[(long)k_m2 * np + pl], cz_m1 = C[(long)k_m1 * np + pl];
-    const double cz_p1 = C[(long)(k + 1) * np + pl], cz_p2 = C[(long)k_p2 * np + pl];
-    double cx_0 = 0.0, cx_1 = 0.0, cx_n2 = 0.0, cx_n1 = 0.0, cy_0 = 0.0, cy_1 = 0.0, cy_n2 = 0.0, cy_n1 = 0.0;
-    if (xends) { cx_0 = C[row]; cx_1 = C[row + 1]; cx_n2 = C[row + nx - 2]; cx_n1 = C[row + nx - 1]; }
-    if (yends) {
-      cy_0 = C[col]; cy_1 = C[col + ld];
-      cy_n2 = C[col + (long)(ny - 2) * ld]; cy_n1 = C[col + (long)(ny - 1) * ld];
-    }
-    // face velocities of this bin
-    const double ws = wsb[b];
-    double uf0 = u0, uf1 = u1, ufF = uF, vf0 = v0, vf1 = v1, vfF = vF, wf0 = w0, wf1 = w1;
-    if (P.settling) {  // w faces 2..nz-1 of the reference carry the settling velocity
-      if (k >= 1) wf0 -= ws;
-      if (k + 1 <= nz - 2) wf1 -= ws;
-      if (P.inertia) {
-        const double f = ws / P.ghat;
-        uf0 -= ax0 * f; uf1 -= ax1 * f; ufF -= axF * f;
-        vf0 -= ay0 * f; vf1 -= ay1 * f; vfF -= ayF * f;
-        if (k >= 1) wf0 -= az0 * f;
-        if (k + 1 <= nz - 2) wf1 -= az1 * f;
+  for (int bb = 0; bb < G; ++bb) {
+    c0[bb] = c1[bb] = d0z[bb] = zf[bb] = zd[bb] = 0.0;
+    if (bb < nb) {
+      const double *C = PC + (long)(b0 + bb) * g.nv;
+      const double cm2 = at(C + (long)(kb >= 2 ? kb - 2 : 0) * np, o);
+      const double cm1 = at(C + (long)(kb >= 1 ? kb - 1 : 0) * np, o);
+      c0[bb] = at(C + (long)kb * np, o);
+      c1[bb] = at(C + (long)(kb + 1) * np, o);
+      d0z[bb] = c0[bb] - cm1;
+      if (kb > 0) {
+        zf[bb] = z_face(kb, w_at(kb, w0, az0, P.settling ? wsb[b0 + bb] : 0.0, INERT ? wsb[g.npc + b0 + bb] : 0.0), cm1, c0[bb], cm1 - cm2, d0z[bb], c1[bb] - c0[bb]);
+        zd[bb] = ((K0 + Kz0) / 2.0) * d0z[bb];
       }
     }
-    // ghost cells -1 and n of the row / column (used only where xends / yends)
-    double gx0, gxL, gy0, gyL;
-    if (P.bc_x == 0) { gx0 = cx_n1; gxL = cx_0; }
-    else if (P.bc_x == 1) { gx0 = 0.0; gxL = cx_n1; }
-    else { gx0 = cx_0 * (1 - sign1(ufF)) / 2; gxL = cx_n1 * (1 - sign1(-ufF)) / 2; }
-    if (P.bc_y == 0) { gy0 = cy_n1; gyL = cy_0; }
-    else if (P.bc_y == 1) { gy0 = cy_0; gyL = 0.0; }
-    else { gy0 = cy_0 * (1 - sign1(vfF)) / 2; gyL = cy_n1 * (1 - sign1(-vfF)) / 2; }
-    // face f lies between cells f-1 and f; the end faces of a periodic row use the face-1
-    // sign
-    double cxb, cxt, cyb, cyt;
-    if (i == 0) {
-      cxb = (P.bc_x == 0) ? ((ufF >= 0.0) ? smart_face(cx_n1, cx_n2, cx_0) : smart_face(cx_0, cx_1, cx_n1)) : gx0;
-    } else {
-      const double cm2 = (i >= 2) ? cx_m2 : gx0, cp1 = (i + 1 <= nx - 1) ? cx_p1 : gxL;
-      cxb = (uf0 >= 0.0) ? smart_face(cx_m1, cm2, ci) : smart_face(ci, cp1, cx_m1);
-    }
-    if (i + 1 == nx) {
-      cxt = (P.bc_x == 0) ? ((ufF >= 0.0) ? smart_face(cx_n1, cx_n2, cx_0) : smart_face(cx_0, cx_1, cx_n1)) : gxL;
-    } else {
-      const double cm2 = (i + 1 >= 2) ? cx_m1 : gx0, cp1 = (i + 2 <= nx - 1) ? cx_p2 : gxL;
-      cxt = (uf1 >= 0.0) ? smart_face(ci, cm2, cx_p1) : smart_face(cx_p1, cp1, ci);
-    }
-    if (j == 0) {
-      cyb = (P.bc_y == 0) ? ((vfF >= 0.0) ? smart_face(cy_n1, cy_n2, cy_0) : smart_face(cy_0, cy_1, cy_n1)) : gy0;
-    } else {
-      const double cm2 = (j >= 2) ? cy_m2 : gy0, cp1 = (j + 1 <= ny - 1) ? cy_p1 : gyL;
-      cyb = (vf0 >= 0.0) ? smart_face(cy_m1, cm2, ci) : smart_face(ci, cp1, cy_m1);
-    }
-    if (j + 1 == ny) {
-      cyt = (P.bc_y == 0) ? ((vfF >= 0.0) ? smart_face(cy_n1, cy_n2, cy_0) : smart_face(cy_0, cy_1, cy_n1)) : gyL;
-    } else {
-      const double cm2 = (j + 1 >= 2) ? cy_m1 : gy0, cp1 = (j + 2 <= ny - 1) ? cy_p2 : gyL;
-      cyt = (vf1 >= 0.0) ? smart_face(ci, cm2, cy_p1) : smart_face(cy_p1, cp1, ci);
-    }
-    // z faces 1..nz-2 (0-based): face 0 carries no flux, face 1 is central for upward flow,
-    // and the top face nz-1 repeats face nz-2 (:3340, :3356)
-    double czb;
-    if (k == 0) czb = 0.0;
-    else if (k == 1) czb = (wf0 >= 0.0) ? (ci + cz_m1) / 2.0 : smart_face(ci, cz_p1, cz_m1);
-    else czb = (wf0 >= 0.0) ? smart_face(cz_m1, cz_m2, ci) : smart_face(ci, cz_p1, cz_m1);
-    double czt;
-    if (k + 1 == nz - 1) czt = czb;
-    else if (k == 0) czt = (wf1 >= 0.0) ? (cz_p1 + ci) / 2.0 : smart_face(cz_p1, cz_p2, ci);
-    else czt = (wf1 >= 0.0) ? smart_face(ci, cz_m1, cz_p1) : smart_face(cz_p1, cz_p2, ci);
-    double r = -P.idx * (uf1 * cxt - uf0 * cxb);
-    r = r - P.idy * (vf1 * cyt - vf0 * cyb);
-    r = r - P.idz * (wf1 * czt - wf0 * czb);
-    {
-      const double cm = (i == 0) ? gx0 : cx_m1;
-      const double cp = (i == nx - 1) ? gxL : cx_p1;
-      r = r + P.idx2 * (((K0 + Kxp) / 2.0) * (cp - ci) - ((K0 + Kxm) / 2.0) * (ci - cm));
-    }
-    {
-      const double cm = (j == 0) ? gy0 : cy_m1;
-      const double cp = (j == ny - 1) ? gyL : cy_p1;
-      r = r + P.idy2 * (((K0 + Kyp) / 2.0) * (cp - ci) - ((K0 + Kym) / 2.0) * (ci - cm));
-    }
-    if (k == 0)
-      r = r + P.idz2 * (((Kzp + K0) / 2.0) * (cz_p1 - ci)) + P.idz * P.psf;
-    else if (k == nz - 2)
-      r = r + P.idz2 * (0.0 - ((K0 + Kzm) / 2.0) * (ci - cz_m1));
-    else
-      r = r + P.idz2 * (((Kzp + K0) / 2.0) * (cz_p1 - ci) - ((K0 + Kzm) / 2.0) * (ci - cz_m1));
-    if (src_here) r += fr * qsrc[b] * fsrc;
-    RH[(long)b * g.nv + s] = r;
   }
+  double rp = 0.0, *Rp = nullptr;  // a value that is still to be stored, and its level
+  auto put = [&]() {
+    if (Rp) *reinterpret_cast<double *>(reinterpret_cast<char *>(Rp) + o) = rp;
+  };
+  for (int k = kb; k < ke; ++k) {
+    // hidden from the passes that would keep an address for each load in the loop
+    int ku = k;
+    asm volatile("" : "+s"(ku));
+    const long lv = (long)ku * np;  // uniform
+    // bin-independent inputs: faces i, i+1 and 1 of the row / column
+    const double *ul = ui0 + (long)ku * g.fp, *vl = vi0 + (long)ku * g.fp;
+    const double u0 = at(ul, o), u1 = at(ul, o + D);
+    const double v0 = at(vl, o), v1 = at(vl, o + D * ld);
+    const double w1 = at(w + lv + np, o);
+    const double Kxm = at(kc + lv, kxm), Kxp = at(kc + lv, kxp);
+    const double Kym = at(kc + lv, kym), Kyp = at(kc + lv, kyp);
+    const double K1 = at(kc + lv + np, o);  // used below the top cell only
+    T az1 = T(0);
+    double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, axF = 0.0, ayF = 0.0;
+    if constexpr (INERT) {  // accelerations on the faces (:2255-2270); the row's end faces are one
+      const T *a = dudt + lv, *b = dvdt + lv;
+      const double a0 = att(a, o / (D / S)), e0 = att(b, o / (D / S));
+      ax0 = 0.5 * (att(a, kxm / (D / S)) + a0);
+      ax1 = 0.5 * (a0 + att(a, kxp / (D / S)));
+      ay0 = 0.5 * (att(b, kym / (D / S)) + e0);
+      ay1 = 0.5 * (e0 + att(b, kyp / (D / S)));
+      az1 = buf_load<T>(dwdt + lv + np, lvb, o / (D / S));
+    }
+    double uF = 0.0, vF = 0.0;
+    if (SIGNS && P.bc_x == 2) {
+      uF = at(ul, D * r0);
+      if (INERT) axF = 0.5 * (att(dudt + lv, S * (r0 + nx - 1)) + att(dudt + lv, S * r0));
+    }
+    if (SIGNS && P.bc_y == 2) {
+      vF = at(vl, D * i);
+      if (INERT) ayF = 0.5 * (att(dvdt + lv, S * ((ny - 1) * ld + i)) + att(dvdt + lv, S * i));
+    }
+    const double Hxm = (K0 + Kxm) / 2.0, Hxp = (K0 + Kxp) / 2.0, Hym = (K0 + Kym) / 2.0, Hyp = (K0 + Kyp) / 2.0;
+    const double Hzp = (K1 + K0) / 2.0;
+    const bool top = k == nz - 2;
+    double q[9];  // the bin's new values: x and y neighbours, the cell two levels up
+    auto load_bin = [&](int bb) {
+      const double *C = PC + (long)(b0 + bb) * g.nv + lv;
+      q[0] = at(C, oxmm); q[1] = at(C, oxm); q[2] = at(C, oxp); q[3] = at(C, oxpp);
+      q[4] = at(C, oymm); q[5] = at(C, oym); q[6] = at(C, oyp); q[7] = at(C, oypp);
+      q[8] = at(C + (top ? 1 : 2) * (long)np, o);  // not used at the top cell
+    };
+#pragma unroll
+    for (int bb = 0; bb < G; ++bb) {
+      if (bb >= nb) break;
+      load_bin(bb);
+      put();  // the last bin's value, behind this bin's loads: waiting for them does not wait for it
+      double xm2 = q[0], xm1 = q[1], xp1 = q[2], xp2 = q[3], ym2 = q[4], ym1 = q[5], yp1 = q[6], yp2 = q[7];
+      const double c2 = q[8];
+      // settling velocity and its time scale, read again for each level (scalar loads)
+      const double ws = P.settling ? wsb[b0 + bb + (ku - k)] : 0.0, f = INERT ? wsb[g.npc + b0 + bb + (ku - k)] : 0.0;
+      const double ci = c0[bb];
+      const double uf0 = u0 - ax0 * f, uf1 = u1 - ax1 * f;
+      const double vf0 = v0 - ay0 * f, vf1 = v1 - ay1 * f;
+      const double wf0 = w_at(k, w0, az0, ws, f), wf1 = w_at(k + 1, w1, az1, ws, f);
+      if constexpr (SIGNS) {  // bc 2: the ghosts as cells 0 and n - 1, times (1 -+ sign of face 1) / 2
+        const double ufF = uF - axF * f, vfF = vF - ayF * f;
+        const double sx0 = P.bc_x == 2 ? (1 - sign1(ufF)) / 2 : 1.0, sxL = P.bc_x == 2 ? (1 - sign1(-ufF)) / 2 : 1.0;
+        const double sy0 = P.bc_y == 2 ? (1 - sign1(vfF)) / 2 : 1.0, syL = P.bc_y == 2 ? (1 - sign1(-vfF)) / 2 : 1.0;
+        xm2 *= i < 2 ? sx0 : 1.0;
+        xm1 *= i < 1 ? sx0 : 1.0;
+        xp1 *= i >= nx - 1 ? sxL : 1.0;
+        xp2 *= i >= nx - 2 ? sxL : 1.0;
+        ym2 *= j < 2 ? sy0 : 1.0;
+        ym1 *= j < 1 ? sy0 : 1.0;
+        yp1 *= j >= ny - 1 ? syL : 1.0;
+        yp2 *= j >= ny - 2 ? syL : 1.0;
+      }
+      const double dx0 = ci - xm1, dx1 = xp1 - ci, dy0 = ci - ym1, dy1 = yp1 - ci;
+      double cxb = smart_between(uf0, xm1, ci, xm1 - xm2, dx0, dx1);
+      double cxt = smart_between(uf1, ci, xp1, dx0, dx1, xp2 - xp1);
+      double cyb = smart_between(vf0, ym1, ci, ym1 - ym2, dy0, dy1);
+      double cyt = smart_between(vf1, ci, yp1, dy0, dy1, yp2 - yp1);
+      cxb = xb ? xm1 : cxb;
+      cxt = xt ? xp1 : cxt;
+      cyb = yb ? ym1 : cyb;
+      cyt = yt ? yp1 : cyt;
+      const double d1z = c1[bb] - ci, d2z = c2 - c1[bb];
+      // the top face: value, diffusive flux
+      const double zs = z_face(k + 1, wf1, ci, c1[bb], d0z[bb], d1z, d2z);
+      const double zt = top ? zf[bb] : zs, zg = top ? 0.0 : Hzp * d1z;
+      double r = -P.idx * (uf1 * cxt - uf0 * cxb);
+      r = r - P.idy * (vf1 * cyt - vf0 * cyb);
+      r = r - P.idz * (wf1 * zt - wf0 * zf[bb]);
+      r = r + P.idx2 * (Hxp * dx1 - Hxm * dx0);
+      r = r + P.idy2 * (Hyp * dy1 - Hym * dy0);
+      r = r + P.idz2 * (zg - zd[bb]);
+      if (k == 0) r = r + P.idz * P.psf;
+      rp = r;
+      Rp = RH + (long)(b0 + bb) * g.nv + lv;
+      zf[bb] = zt;
+      zd[bb] = zg;
+      c0[bb] = c1[bb];
+      c1[bb] = c2;
+      d0z[bb] = d1z;
+    }
+    K0 = K1;
+    w0 = w1;
+    az0 = az1;
+  }
+  put();
+  if (P.src_on)
+    for (int k = kb; k < ke; ++k)
+      if (k == P.src_k0 || k == P.src_k0 + 1) {  // its two levels
+        const double fr = (k == P.src_k0) ? P.frac : P.frac1, fsrc = foot[(long)j * nx + i];
+        for (int bb = 0; bb < nb; ++bb) RH[(long)(b0 + bb) * g.nv + (long)k * np + p] += fr * qsrc[b0 + bb] * fsrc;
+      }
 }
 
 // breakage-frequency fit of one bin (:2167-2230): the Ohnesorge-number coefficients and

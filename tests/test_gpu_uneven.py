@@ -161,3 +161,46 @@ def test_lag_level_runs(nx, ny, nz):
     print()
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,nb,bc,kw", [
+    (96, 32, 4, 2, (0, 1), dict(inertia=False)),       # 32-point tiles, two bins, runs of 1 and 2 levels
+    (32, 64, 5, 5, (1, 0), {}),                        # a full group
+    (64, 32, 20, 7, (2, 1), {}),                       # a group and a remainder, ghosts by sign along x
+    (64, 96, 9, 11, (1, 2), dict(settling=False)),
+    (192, 64, 34, 4, (0, 0), dict(inertia=False)),     # runs of 4 levels
+    (128, 128, 130, 3, (1, 1), dict(sfc_flux=-0.5)),   # runs of 16
+])
+def test_droplet_transport_tiles(nx, ny, nz, nb, bc, kw):
+    """the droplet right-hand side over its tiles, bin groups and level runs: one
+    pollen_all_in_one2 with the previous RHS kept outside the cells, against the oracle at
+    1e-12 (binary64, terms of the same order summed in the oracle's order up to contraction)"""
+    from oracle import Oracle
+    from population_balance_amd import droplets
+    from population_balance_amd.lesgo import Lesgo
+    from test_gpu_droplets import _load, _routine_state
+    cfg = abi.make_config(nx, ny, nz)
+    ds = droplets.DropletSet(nb)
+    ds.fill(cfg, pbe=False, bc=bc, **kw)
+    print(f"\n[case] droplet tiles {nx}x{ny}x{nz} bins {nb} bc {bc} {kw}", flush=True)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    st = _routine_state(cfg, ds)
+    st["RHS_PCon"] = st["RHS_PCon"] + 1e-3
+    _load(o, lg, st, jt_total=2)
+    for c in (o, lg):
+        c.set_time(2, 2)
+    o.call("pollen_all_in_one2")
+    lg.pollen_all_in_one2()
+    for n in ("RHS_PCon", "PCon"):
+        a, b = lg.download(n), o.field(n)
+        err = rel_l2(a, b, nx)
+        print(f"  {n}: {err:.2e}", end="")
+        assert err < TOL, (n, err)
+        for q in range(nb):
+            e = rel_l2(a[q], b[q], nx)
+            assert e < TOL, (n, q, e)
+    print()
+    assert np.array_equal(lg.download("RHS_PCon")[..., nx:], st["RHS_PCon"][..., nx:])
+    assert np.array_equal(lg.download("RHS_PCon")[:, -1], st["RHS_PCon"][:, -1])
+    lg.close()
+    o.close()
