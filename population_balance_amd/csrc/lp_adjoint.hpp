@@ -394,21 +394,6 @@ __global__ void k_tau_frozen(const T *__restrict__ S11, const T *__restrict__ S1
 // transposed would scatter into it, in the scan's order), so no pass needs atomics.
 // ------------------------------------------------------------------------------------
 
-// d smart_face / d (cup, cupup, cdn) on the branch smart_face selects
-__device__ __forceinline__ void smart_coef(double cup, double cupup, double cdn, double &au, double &auu,
-                                           double &ad) {
-  au = 1.0; auu = 0.0; ad = 0.0;
-  const double den = cup - cupup;
-  if (den == 0.0) return;
-  const double num = cdn - cup;
-  const double a = 2.0 * num, b = 0.75 * num + 0.25 * den, c = 4.0 * den;
-  const double pd = den > 0.0 ? fmax(0.0, fmin(fmin(a, b), c)) : fmin(0.0, fmax(fmax(a, b), c));
-  if (pd == 0.0) return;                                              // the upwind cell
-  if (pd == a) { au = 0.0; ad = 1.0; return; }                        // the downwind cell
-  if (pd == b) { au = 0.75; auu = -0.125; ad = 0.375; return; }       // QUICK
-  au = 3.0; auu = -2.0;                                               // psi = 4
-}
-
 // step_pollen2 and calcbeta_pcon transposed (every point of every bin):
 // lb, lr the adjoints of the step's PCon and RHS_PCon (lr becomes that of the RHS_PCon the
 // step reads); mu = adjoint of this step's RHS_PCon; ac = adjoint of the old PCon through
@@ -439,220 +424,272 @@ struct DropAdjP {
   int bc_x, bc_y, settling;
 };
 
-// x (Y false) and y (Y true) transport transposed in gather form for one cell of one bin.  A cell adds the terms the line scan of
-// the fluxes transposed scatters into it, in the scan's order: the interior faces c-1, c,
-// c+1, c+2, then the end faces, the Kc diffusion of cells c-1, c, c+1 (ghosts at the line
-// ends), and last the folds of the ghosts' adjoints at the two end cells.  The terms of a
-// face are recomputed by each cell that reads them; cell c = f >= 1 writes face f's
-// adjoint into auv (the bin's (ld, ny+1, nz) face array), cell 0 or n-1 the end faces.
+// The branch that smart_face takes at a face with the difference num across it and den across
+// the face before it (downstream of the upwind cell), as the coefficients of the upwind, the
+// second upwind and the downwind cell: (1, 0, 0), (0, 0, 1), QUICK (3/4, -1/8, 3/8) or psi = 4
+// (3, -2, 0); all have a zero low word.
+struct SmartBranch {
+  bool up, dn, qk;
+  __device__ __forceinline__ SmartBranch(double num, double den) {
+    const unsigned long long m = den > 0.0 ? 0ull : 0x8000000000000000ull;
+    const double n = __longlong_as_double(__double_as_longlong(num) ^ m), d = fabs(den);
+    const double q = 0.375 * n + 0.125 * d, t = fmin(fmin(n, q), d + d);
+    up = !(t > 0.0);
+    dn = t == n;
+    qk = t == q;
+  }
+  __device__ __forceinline__ static double hi(int h) { return __hiloint2double(h, 0); }
+  __device__ __forceinline__ double au() const { return hi(up ? 0x3ff00000 : (dn ? 0 : (qk ? 0x3fe80000 : 0x40080000))); }
+  __device__ __forceinline__ double auu() const { return hi(up || dn ? 0 : (qk ? 0xbfc00000 : 0xc0000000)); }
+  __device__ __forceinline__ double ad() const { return hi(up ? 0 : (dn ? 0x3ff00000 : (qk ? 0x3fd80000 : 0))); }
+};
+
+// the inputs of one line (x or y) through a cell that do not depend on the bin
+struct DropLine {
+  unsigned o[6];       // byte offsets within a level of cells c-3 .. c-1, c+1 .. c+3 (ghosts: as nb_x below)
+  double U[4];         // faces c-1 .. c+2
+  double u0, un;       // faces 0 and n (bc 0 and 2)
+  double Hm, Hp;       // Kc_t on the faces of the cell
+};
+
+// The x (Y false) or y (Y true) transport of one bin transposed in gather form for one cell.  A
+// cell adds the terms the line scan of the fluxes transposed scatters into it, in the scan's
+// order: the interior faces c-1, c, c+1, c+2, then the end faces, the Kc diffusion of cells
+// c-1, c, c+1 (ghosts at the line ends), and last the folds of the ghosts' adjoints at the two
+// end cells.  The terms of a face are recomputed by each cell that reads them; cell c adds face
+// c's adjoint to af, the end cells the far end's to ae.
 template <bool Y>
-__device__ __forceinline__ double drop_line_cell(double A, int i, int j, int k, int b, const double *__restrict__ C,
-                                                 const double *__restrict__ mu, const double *__restrict__ uv0,
-                                                 double *__restrict__ auv, const double *__restrict__ kc,
+__device__ __forceinline__ double drop_line_cell(double A, int c, const DropLine &L, const double *__restrict__ Cl,
+                                                 const double *__restrict__ Ml, unsigned lvb, unsigned o, double Cc,
+                                                 double Mc, const double *__restrict__ Ul, unsigned o0, double &af, double &ae,
                                                  const DropGeo &g, const DropAdjP &P) {
-  const int n = Y ? g.ny : g.nx, c = Y ? j : i, bc = Y ? P.bc_y : P.bc_x;
-  const long st = Y ? g.ld : 1, ol = Y ? (long)i : (long)j * g.ld, ob = (long)b * g.nv;
-  const double *Cl = C + ob + (long)k * g.np + ol, *Ml = mu + ob + (long)k * g.np + ol, *Kl = kc + (long)k * g.np + ol;
-  const double *U = uv0 + (long)k * g.fp + ol;
-  double *AU = auv + (long)b * g.fp * g.nz + (long)k * g.fp + ol;
+  const int n = Y ? g.ny : g.nx, bc = Y ? P.bc_y : P.bc_x;
   const double id = Y ? P.idy : P.idx, id2 = Y ? P.idy2 : P.idx2;
-  auto Cv = [&](int q) { return Cl[q * st]; };
-  auto Mv = [&](int q) { return Ml[q * st]; };
-  auto Kv = [&](int q) { return Kl[q * st]; };
-  // the cell's stencil, loaded together: C at c-3 .. c+3, mu at c-2 .. c+2, Kc at c-2 .. c+2
-  // (periodic), faces c-1 .. c+2; indices off the line are clamped (their values go unused)
-  double Cw[7], Mw[5], Kw[5], Uw[4];
+  double Cw[7], Mw[5];  // cells c-3 .. c+3 with the ghosts, c-2 .. c+2
 #pragma unroll
-  for (int d = 0; d < 7; ++d) Cw[d] = Cv(min(max(c + d - 3, 0), n - 1));
+  for (int d = 0; d < 7; ++d) Cw[d] = d == 3 ? Cc : buf_load(Cl, lvb, L.o[d < 3 ? d : d - 1]);
 #pragma unroll
-  for (int d = 0; d < 5; ++d) Mw[d] = Mv(min(max(c + d - 2, 0), n - 1));
+  for (int d = 0; d < 5; ++d) Mw[d] = d == 2 ? Mc : buf_load(Ml, lvb, L.o[d < 2 ? d + 1 : d]);
+  const double s0 = signbit(L.u0) ? 1.0 : 0.0, s1 = signbit(-L.u0) ? 1.0 : 0.0;
+  if (bc == 2) {
 #pragma unroll
-  for (int d = 0; d < 5; ++d) {
-    const int q = c + d - 2;
-    Kw[d] = Kv(q < 0 ? q + n : (q >= n ? q - n : q));
+    for (int d = 0; d < 7; ++d) {
+      const int q = c + d - 3;
+      Cw[d] *= q < 0 ? s0 : (q >= n ? s1 : 1.0);
+    }
   }
+  double a[4], D[6];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) Uw[d] = U[min(max(c + d - 1, 0), n) * st];
-  const double u0 = U[0], Cf = Cv(0), Cn = Cv(n - 1);
-  double g0 = 0.0, gL = 0.0, s0 = 0.0, s1 = 0.0;  // the ghost cells
-  if (bc == 0) { g0 = Cn; gL = Cf; }
-  else if (bc == 1) { if (Y) g0 = Cf; else gL = Cn; }
-  else {
-    s0 = signbit(u0) ? 1.0 : 0.0;
-    s1 = signbit(-u0) ? 1.0 : 0.0;
-    g0 = Cf * s0; gL = Cn * s1;
-  }
-  // interior face f (between cells f-1 and f): a = u_f m / d, the SMART branch coefficients;
-  // facew takes face c + df from the stencil, face any face from memory
-  auto pick = [&](int f, double uf, double &au, double &auu, double &ad, double &cup, double &cupup, double &cdn,
-                  double cm2, double cm1, double c0, double cp1) {
-    const bool pos = uf >= 0.0;
-    if (pos) { cup = cm1; cupup = f >= 2 ? cm2 : g0; cdn = c0; }
-    else { cup = c0; cupup = f + 1 <= n - 1 ? cp1 : gL; cdn = cm1; }
-    smart_coef(cup, cupup, cdn, au, auu, ad);
-    return pos;
-  };
-  auto facew = [&](int df, double &a, double &au, double &auu, double &ad, double &cup, double &cupup, double &cdn) {
-    const double uf = Uw[df + 1];
-    a = uf * id * (Mw[df + 2] - Mw[df + 1]);
-    return pick(c + df, uf, au, auu, ad, cup, cupup, cdn, Cw[df + 1], Cw[df + 2], Cw[df + 3], Cw[df + 4]);
-  };
-  auto face = [&](int f, double &a, double &au, double &auu, double &ad, double &cup, double &cupup, double &cdn) {
-    const double uf = U[f * st];
-    a = uf * id * (Mv(f) - Mv(f - 1));
-    return pick(f, uf, au, auu, ad, cup, cupup, cdn, Cv(max(f - 2, 0)), Cv(f - 1), Cv(f), Cv(min(f + 1, n - 1)));
-  };
-  auto diff = [&](int q, double &Kp, double &Km) {  // returns the cell's m / d^2
-    const double Kq = Kv(q);
-    Kp = 0.5 * (Kq + Kv(q + 1 < n ? q + 1 : 0));
-    Km = 0.5 * (Kq + Kv(q >= 1 ? q - 1 : n - 1));
-    return Mv(q) * id2;
-  };
-  auto diffw = [&](int dq, double &Kp, double &Km) {
-    const double Kq = Kw[dq + 2];
-    Kp = 0.5 * (Kq + Kw[dq + 3]);
-    Km = 0.5 * (Kq + Kw[dq + 1]);
-    return Mw[dq + 2] * id2;
-  };
-  double a, au, auu, ad, cu, cuu, cd;
-  if (c - 1 >= 1 && !facew(-1, a, au, auu, ad, cu, cuu, cd)) A += auu * a;
+  for (int d = 0; d < 4; ++d) a[d] = L.U[d] * id * (Mw[d + 1] - Mw[d]);
+#pragma unroll
+  for (int d = 0; d < 6; ++d) D[d] = Cw[d + 1] - Cw[d];
+  bool pos[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) pos[d] = L.U[d] >= 0.0;
+  // face c + d - 1 lies between cells c + d - 2 and c + d - 1, with D[d + 1] across it
+  auto branch = [&](int d) { return SmartBranch(D[d + 1], pos[d] ? D[d] : D[d + 2]); };
+  const SmartBranch B0 = branch(0), B1 = branch(1), B2 = branch(2), B3 = branch(3);
+  if (c >= 2 && !pos[0]) A += B0.auu() * a[0];
   if (c >= 1) {
-    const bool pos = facew(0, a, au, auu, ad, cu, cuu, cd);
-    A += pos ? ad * a : au * a;
-    AU[c * st] += smart_face(cu, cuu, cd) * id * (Mw[2] - Mw[1]);
+    A += (pos[1] ? B1.ad() : B1.au()) * a[1];
+    af += smart_between(L.U[1], Cw[2], Cw[3], D[1], D[2], D[3]) * id * (Mw[2] - Mw[1]);
   }
-  if (c + 1 <= n - 1) {
-    const bool pos = facew(1, a, au, auu, ad, cu, cuu, cd);
-    A += pos ? au * a : ad * a;
-  }
-  if (c + 2 <= n - 1 && facew(2, a, au, auu, ad, cu, cuu, cd)) A += auu * a;
+  if (c <= n - 2) A += (pos[2] ? B2.au() : B2.ad()) * a[2];
+  if (c <= n - 3 && pos[3]) A += B3.auu() * a[3];
   // faces 0 and n: they reach cells 0, 1, n-2 and n-1 only
+  const unsigned st = Y ? 8u * g.ld : 8u;  // o0: cell 0 of the line
+  auto Cv = [&](int q) { return buf_load(Cl, lvb, o0 + q * st); };
+  auto Mv = [&](int q) { return buf_load(Ml, lvb, o0 + q * st); };
   double a0 = 0.0, aL = 0.0;
-  if (c <= 1 || c >= n - 2) {
-    const double m0 = Mv(0), mL = -Mv(n - 1);
-    a0 = u0 * id * m0; aL = U[n * st] * id * mL;
-    if (bc == 0) {
+  if (bc == 0) {
+    if (c <= 1 || c >= n - 2) {
+      const double m0 = Mv(0), mL = -Mv(n - 1);
+      a0 = L.u0 * id * m0; aL = L.un * id * mL;
       int iu, iuu, idn;
-      if (u0 >= 0.0) { iu = n - 1; iuu = n - 2; idn = 0; }
+      if (L.u0 >= 0.0) { iu = n - 1; iuu = n - 2; idn = 0; }
       else { iu = 0; iuu = 1; idn = n - 1; }
-      if (c == iu || c == iuu || c == idn) {
-        smart_coef(Cv(iu), Cv(iuu), Cv(idn), au, auu, ad);
-        A += (c == iu ? au : c == iuu ? auu : ad) * (a0 + aL);
-      }
+      const double cu = Cv(iu), cuu = Cv(iuu), cd = Cv(idn);
+      const SmartBranch B(cd - cu, cu - cuu);
+      if (c == iu || c == iuu || c == idn) A += (c == iu ? B.au() : c == iuu ? B.auu() : B.ad()) * (a0 + aL);
       if (c == 0) {
-        const double f0 = smart_face(Cv(iu), Cv(iuu), Cv(idn));
-        AU[0] += f0 * id * m0;
-        AU[n * st] += f0 * id * mL;
+        const double f0 = smart_face(cu, cuu, cd);
+        af += f0 * id * m0;
+        ae += f0 * id * mL;
       }
-    } else if (bc == 1) {  // x: face 0 carries nothing, face n the last cell; y: the mirror
-      if (Y && c == 0) { AU[0] += Cf * id * m0; A += a0; }
-      if (!Y && c == n - 1) { AU[n * st] += Cn * id * mL; A += aL; }
-    } else if (c == 0) {   // the ghosts are the end faces
-      AU[0] += g0 * id * m0;
-      AU[n * st] += gL * id * mL;
+    }
+  } else if (bc == 1) {  // x: face 0 carries nothing, face n the last cell; y: the mirror
+    if (Y && c == 0) { af += Cc * id * Mc; A += L.U[1] * id * Mc; }
+    if (!Y && c == n - 1) { ae += Cc * id * -Mc; A += L.U[2] * id * -Mc; }
+  } else {
+    a0 = L.U[1] * id * Mc;  // used at the near end only
+    aL = L.U[2] * id * -Mc;
+    if (c == 0) {  // the ghosts are the end faces
+      af += Cw[2] * id * Mc;
+      ae += Cv(n - 1) * s1 * id * -Mv(n - 1);
     }
   }
-  double Kp, Km;
-  if (c >= 1) { const double m = diffw(-1, Kp, Km); A += Kp * m; }
-  { const double m = diffw(0, Kp, Km); A -= (Kp + Km) * m; }
-  if (c + 1 <= n - 1) { const double m = diffw(1, Kp, Km); A += Km * m; }
-  if (c == 0 || c == n - 1) {  // the ghosts' adjoints, summed in the scan's order
-    double ag0 = 0.0, agL = 0.0;
-    const bool lo = c == 0;  // the near end's face and diffusion come from the stencil
-    if (lo ? facew(1, a, au, auu, ad, cu, cuu, cd) : face(1, a, au, auu, ad, cu, cuu, cd)) ag0 += auu * a;
-    if (!(lo ? face(n - 1, a, au, auu, ad, cu, cuu, cd) : facew(0, a, au, auu, ad, cu, cuu, cd))) agL += auu * a;
-    if (bc == 2) { ag0 += a0; agL += aL; }
-    { const double m = lo ? diffw(0, Kp, Km) : diff(0, Kp, Km); ag0 += Km * m; }
-    { const double m = lo ? diff(n - 1, Kp, Km) : diffw(0, Kp, Km); agL += Kp * m; }
-    if (bc == 0) A += c == n - 1 ? ag0 : agL;
-    else if (bc == 1) { if (Y && c == 0) A += ag0; if (!Y && c == n - 1) A += agL; }
-    else A += c == 0 ? s0 * ag0 : s1 * agL;
+  if (c >= 1) A += L.Hm * (Mw[1] * id2);
+  A -= (L.Hp + L.Hm) * (Mc * id2);
+  if (c <= n - 2) A += L.Hp * (Mw[3] * id2);
+  // the ghosts' adjoints, summed in the scan's order: that of cell -1 is read by cell 0 (its
+  // face 1 and diffusion are cell 0's), of cell n by cell n-1; periodic, they are the other end
+  if (bc == 0) {
+    if (c == n - 1) {
+      const double c0 = Cv(0), c1 = Cv(1), u1 = buf_load(Ul, lvb + 8 * g.ld, o0 + st), m0 = Mv(0);
+      double ag = 0.0;
+      if (u1 >= 0.0) ag += SmartBranch(c1 - c0, c0 - Cc).auu() * (u1 * id * (Mv(1) - m0));
+      A += ag + L.Hp * (m0 * id2);
+    } else if (c == 0) {
+      const double cn1 = Cv(n - 1), cn2 = Cv(n - 2), un1 = buf_load(Ul, lvb + 8 * g.ld, o0 + (n - 1) * st), mn = Mv(n - 1);
+      double ag = 0.0;
+      if (!(un1 >= 0.0)) ag += SmartBranch(cn1 - cn2, Cc - cn1).auu() * (un1 * id * (mn - Mv(n - 2)));
+      A += ag + L.Hm * (mn * id2);
+    }
+  }
+  else if (c == 0 && (Y || bc == 2)) {
+    double ag = pos[2] ? B2.auu() * a[2] : 0.0;
+    if (bc == 2) ag += a0;
+    ag += L.Hm * (Mc * id2);
+    A += bc == 2 ? s0 * ag : ag;
+  } else if (c == n - 1 && (!Y || bc == 2)) {
+    double ag = pos[1] ? 0.0 : B1.auu() * a[1];
+    if (bc == 2) ag += aL;
+    ag += L.Hp * (Mc * id2);
+    A += bc == 2 ? s1 * ag : ag;
   }
   return A;
 }
 
-// z in gather form for one cell (x < nx) of one bin: w faces 1..nz-1 (face 0
-// carries nothing, face nz-1 repeats nz-2, face 1 is central for upward flow).  A face
-// adds to three distinct cells, so cell c takes the terms of faces c-1 .. c+2 and then the
-// Kc diffusion terms of levels c-1, c, c+1, in the order of the level scan; cell c = k
-// writes the bin's adjoint of w face k into awi (a volume per bin), cell nz-2 also face nz-1's.
-__device__ __forceinline__ double drop_z_cell(double A, int i, int j, int c, int b, const double *__restrict__ C,
-                                              const double *__restrict__ mu, const double *__restrict__ w,
-                                              double *__restrict__ awi_all, const double *__restrict__ kc,
-                                              const double *__restrict__ wsb, const DropGeo &g, const DropAdjP &P) {
+// z in gather form for one cell of one bin: w faces 1..nz-1 (face 0 carries nothing, face nz-1
+// repeats nz-2, face 1 is central for upward flow).  A face adds to three distinct cells, so cell
+// c takes the terms of faces c-1 .. c+2 and then the Kc diffusion terms of levels c-1, c, c+1, in
+// the order of the level scan; cell c adds the adjoint of w face c to af, cell nz-2 also face
+// nz-1's to ae.  c is uniform over the block.  W: faces c-1 .. c+3; Hm, Hp: Kc_t on the faces.
+__device__ __forceinline__ double drop_z_cell(double A, int c, const double *__restrict__ C,
+                                              const double *__restrict__ M, unsigned lvb, unsigned o, double Cc,
+                                              double Mc, const double (&W)[5], double Hm, double Hp, double ws,
+                                              double &af, double &ae, const DropGeo &g, const DropAdjP &P) {
   const int nz = g.nz;
-  const long o = (long)j * g.ld + i, np = g.np, ob = (long)b * g.nv;
-  const double ws = P.settling ? wsb[b] : 0.0;
-  auto lv = [&](int q) { return (long)min(max(q, 0), nz - 1) * np + o; };  // clamped level q
-  // the cell's stencil, loaded together: C at c-3 .. c+3, mu at c-2 .. c+2, w at c-1 .. c+3,
-  // Kc at c-1 .. c+1; levels off the column are clamped (their values go unused)
-  double Cw[7], Mw[5], Ww[5], Kw[3];
+  auto lv = [&](const double *F, int q) { return buf_load(F + (long)min(max(q, 0), nz - 1) * g.np, lvb, o); };
+  double Cw[7], Mw[5];  // cells c-3 .. c+3, c-2 .. c+2 (clamped: those off the column go unused)
 #pragma unroll
-  for (int d = 0; d < 7; ++d) Cw[d] = C[ob + lv(c + d - 3)];
+  for (int d = 0; d < 7; ++d) Cw[d] = d == 3 ? Cc : lv(C, c + d - 3);
 #pragma unroll
-  for (int d = 0; d < 5; ++d) Mw[d] = mu[ob + lv(c + d - 2)];
+  for (int d = 0; d < 5; ++d) Mw[d] = d == 2 ? Mc : lv(M, c + d - 2);
 #pragma unroll
-  for (int d = 0; d < 5; ++d) Ww[d] = w[lv(c + d - 1)];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) Kw[d] = kc[lv(c + d - 1)];
-#pragma unroll
-  for (int dk = -1; dk <= 2; ++dk) {  // faces k = c-1 .. c+2 within 1 .. nz-2
-    const int k = c + dk;
+  for (int d = 0; d < 4; ++d) {  // faces k = c-1 .. c+2 within 1 .. nz-2
+    const int k = c + d - 1;
     if (k < 1 || k > nz - 2) continue;
-    const double wk = Ww[dk + 1] - ws;
-    const double m = Mw[dk + 2] - Mw[dk + 1];
+    const double wk = W[d] - ws;
+    const bool pos = wk >= 0.0, mid = k == 1 && pos;
+    const double m = Mw[d + 1] - Mw[d];
     double at = wk * P.idz * m;
-    if (k == nz - 2) at += (Ww[dk + 2] - 0.0) * P.idz * (-Mw[dk + 2]);  // face nz-1 joins nz-2
-    double au, auu, ad, face;
-    int ku, kuu, kdn;
-    if (k == 1 && wk >= 0.0) {
-      face = 0.5 * (Cw[dk + 3] + Cw[dk + 2]);
-      ku = 1; kdn = 0; kuu = -1; au = 0.5; ad = 0.5; auu = 0.0;
-    } else {
-      double cup, cupup, cdn;
-      if (wk >= 0.0) { ku = k - 1; kuu = k - 2; kdn = k; cup = Cw[dk + 2]; cupup = Cw[dk + 1]; cdn = Cw[dk + 3]; }
-      else { ku = k; kuu = k + 1; kdn = k - 1; cup = Cw[dk + 3]; cupup = Cw[dk + 4]; cdn = Cw[dk + 2]; }
-      face = smart_face(cup, cupup, cdn);
-      smart_coef(cup, cupup, cdn, au, auu, ad);
+    if (k == nz - 2) at += (W[d + 1] - 0.0) * P.idz * (-Mw[d + 1]);  // face nz-1 joins nz-2
+    const double D0 = Cw[d + 1] - Cw[d], D1 = Cw[d + 2] - Cw[d + 1], D2 = Cw[d + 3] - Cw[d + 2];
+    const SmartBranch B(D1, pos ? D0 : D2);
+    if (d == 0) A += pos ? 0.0 : B.auu() * at;
+    if (d == 1) {
+      const double face = mid ? 0.5 * (Cw[3] + Cw[2]) : smart_between(wk, Cw[2], Cw[3], D0, D1, D2);
+      af += face * P.idz * m;
+      if (k == nz - 2) ae += face * P.idz * (-Mw[2]);
+      A += (mid ? 0.5 : (pos ? B.ad() : B.au())) * at;
     }
-    if (dk == 0) {
-      double *awi = awi_all + ob;
-      awi[(long)k * np + o] += face * P.idz * m;
-      if (k == nz - 2) awi[(long)(nz - 1) * np + o] += face * P.idz * (-Mw[2]);
-    }
-    if (ku == c) A += au * at;
-    else if (kdn == c) A += ad * at;
-    else if (kuu == c) A += auu * at;
+    if (d == 2) A += (mid ? 0.5 : (pos ? B.au() : B.ad())) * at;
+    if (d == 3) A += pos ? B.auu() * at : 0.0;
   }
-  if (c >= 1 && c - 1 <= nz - 3) A += 0.5 * (Kw[1] + Kw[0]) * (Mw[1] * P.idz2);  // level c-1
-  if (c <= nz - 2) {                                                            // level c
-    const double m = Mw[2] * P.idz2;
-    if (c <= nz - 3) A -= 0.5 * (Kw[2] + Kw[1]) * m;
-    if (c >= 1) A -= 0.5 * (Kw[1] + Kw[0]) * m;
+  if (c >= 1 && c - 1 <= nz - 3) A += Hm * (Mw[1] * P.idz2);  // level c-1
+  if (c <= nz - 2) {                                          // level c
+    const double m = Mc * P.idz2;
+    if (c <= nz - 3) A -= Hp * m;
+    if (c >= 1) A -= Hm * m;
   }
-  if (c + 1 <= nz - 2) A += 0.5 * (Kw[2] + Kw[1]) * (Mw[3] * P.idz2);           // level c+1
+  if (c + 1 <= nz - 2) A += Hp * (Mw[3] * P.idz2);            // level c+1
   return A;
 }
 
-// the three directions for one cell of one bin (blocks of 64 x by 4 y cells, grid z over
-// level + nz bin): x, then y (levels below nz-1), then z, each as the passes above
-__global__ void __launch_bounds__(256) k_adj_drop_xyz(const double *__restrict__ C, const double *__restrict__ mu,
-                                                      double *__restrict__ ac, const double *__restrict__ ui0,
+// The three directions for one cell and a run of bins: x, then y (levels below nz-1), then z,
+// each as above; blocks of 64 x by 4 y cells, grid z over level + nz group.  The face
+// velocities, Kc_t and offsets are read once for all bins, and the faces' adjoints summed over
+// the bins in index order: aui, avi, awi hold a face array or volume per group, zero where
+// nothing is written here; ac is read, cb (the adjoint of PCon) written.  Bound by its loads
+// through L1, 33 per cell and bin; one bin per thread took 78, and the face arrays of each bin
+// were cleared, added to and summed by further passes.  128x128x65 with 15 bins: 496 us, with
+// the clearing, the sums and a copy 520; 868 and 1090 before.  Two wavefronts per SIMD 545
+// us, four 534 (spills).
+__global__ void __launch_bounds__(256, 3) k_adj_drop_xyz(const double *__restrict__ C, const double *__restrict__ mu,
+                                                      const double *__restrict__ ac, double *__restrict__ cb,
+                                                      const double *__restrict__ ui0,
                                                       const double *__restrict__ vi0, const double *__restrict__ w,
                                                       double *__restrict__ aui, double *__restrict__ avi,
                                                       double *__restrict__ awi, const double *__restrict__ kc,
-                                                      const double *__restrict__ wsb, DropGeo g, DropAdjP P) {
+                                                      const double *__restrict__ wsb, DropGeo g, DropAdjP P, int ngrp) {
   const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
   if (i >= g.nx || j >= g.ny) return;
-  const int b = (int)blockIdx.z / g.nz, k = (int)blockIdx.z - b * g.nz;
-  const long s = (long)b * g.nv + (long)k * g.np + (long)j * g.ld + i;
-  double A = ac[s];
-  if (k < g.nz - 1) {
-    A = drop_line_cell<false>(A, i, j, k, b, C, mu, ui0, aui, kc, g, P);
-    A = drop_line_cell<true>(A, i, j, k, b, C, mu, vi0, avi, kc, g, P);
+  const int grp = (int)blockIdx.z / g.nz, k = (int)blockIdx.z - grp * g.nz;
+  const int b0 = (int)((long)grp * g.npc / ngrp), b1 = (int)((long)(grp + 1) * g.npc / ngrp);
+  const int nx = g.nx, ny = g.ny, nz = g.nz, ld = g.ld;
+  const unsigned lvb = 8u * (unsigned)g.np, lvf = lvb + 8u * ld;
+  const unsigned r0 = 8u * (j * ld), c0 = 8u * i, o = r0 + c0;
+  // cells of a line around c: wrapped when periodic; else the end cell, or for an inlet's zero
+  // ghost an offset past the level
+  auto nb = [](int q, int n, int bc, int zero) -> int {
+    const int v = bc == 0 ? (q < 0 ? q + n : (q >= n ? q - n : q)) : min(max(q, 0), n - 1);
+    return bc == 1 && ((zero < 0 && q < 0) || (zero > 0 && q >= n)) ? -1 : v;
+  };
+  const long lv = (long)k * g.np;
+  DropLine X, Y;
+#pragma unroll
+  for (int d = 0; d < 6; ++d) {
+    const int e = d < 3 ? d - 3 : d - 2, qx = nb(i + e, nx, P.bc_x, -1), qy = nb(j + e, ny, P.bc_y, 1);
+    X.o[d] = qx < 0 ? kGone : r0 + 8u * qx;
+    Y.o[d] = qy < 0 ? kGone : c0 + 8u * (qy * ld);
   }
-  A = drop_z_cell(A, i, j, k, b, C, mu, w, awi, kc, wsb, g, P);
-  ac[s] = A;
+  const double *ul = ui0 + (long)k * g.fp, *vl = vi0 + (long)k * g.fp, *kl = kc + lv;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    X.U[d] = buf_load(ul, lvf, r0 + 8u * min(max(i + d - 1, 0), nx));
+    Y.U[d] = buf_load(vl, lvf, c0 + 8u * (min(max(j + d - 1, 0), ny) * ld));
+  }
+  X.u0 = buf_load(ul, lvf, r0);
+  X.un = buf_load(ul, lvf, r0 + 8u * nx);
+  Y.u0 = buf_load(vl, lvf, c0);
+  Y.un = buf_load(vl, lvf, c0 + 8u * (ny * ld));
+  const double K = buf_load(kl, lvb, o);
+  X.Hm = 0.5 * (K + buf_load(kl, lvb, r0 + 8u * (i ? i - 1 : nx - 1)));
+  X.Hp = 0.5 * (K + buf_load(kl, lvb, r0 + 8u * (i + 1 < nx ? i + 1 : 0)));
+  Y.Hm = 0.5 * (K + buf_load(kl, lvb, c0 + 8u * ((j ? j - 1 : ny - 1) * ld)));
+  Y.Hp = 0.5 * (K + buf_load(kl, lvb, c0 + 8u * ((j + 1 < ny ? j + 1 : 0) * ld)));
+  const double Zm = 0.5 * (K + buf_load(kc + (long)max(k - 1, 0) * g.np, lvb, o));
+  const double Zp = 0.5 * (K + buf_load(kc + (long)min(k + 1, nz - 1) * g.np, lvb, o));
+  double W[5];
+#pragma unroll
+  for (int d = 0; d < 5; ++d) W[d] = buf_load(w + (long)min(max(k + d - 1, 0), nz - 1) * g.np, lvb, o);
+  double ax = 0.0, axe = 0.0, ay = 0.0, aye = 0.0, az = 0.0, aze = 0.0;
+  for (int b = b0; b < b1; ++b) {
+    const double *Cb = C + (long)b * g.nv, *Mb = mu + (long)b * g.nv;
+    const double Cc = buf_load(Cb + lv, lvb, o), Mc = buf_load(Mb + lv, lvb, o);
+    double A = buf_load(ac + (long)b * g.nv + lv, lvb, o);
+    if (k < nz - 1) {
+      A = drop_line_cell<false>(A, i, X, Cb + lv, Mb + lv, lvb, o, Cc, Mc, ul, r0, ax, axe, g, P);
+      A = drop_line_cell<true>(A, j, Y, Cb + lv, Mb + lv, lvb, o, Cc, Mc, vl, c0, ay, aye, g, P);
+    }
+    A = drop_z_cell(A, k, Cb, Mb, lvb, o, Cc, Mc, W, Zm, Zp, P.settling ? wsb[b] : 0.0, az, aze, g, P);
+    double *out = cb + (long)b * g.nv + lv + o / 8;
+    out[0] = A;
+    if (i == nx - 1)
+      for (int q = 1; q <= ld - nx; ++q) out[q] = 0.0;  // the padding columns
+  }
+  const long fz = g.fp * nz;
+  double *au = aui + grp * fz + (long)k * g.fp, *av = avi + grp * fz + (long)k * g.fp;
+  double *aw = awi + (long)grp * g.nv + lv;
+  if (k < nz - 1) {
+    au[o / 8] = ax;
+    if (P.bc_x == 1 ? i == nx - 1 : i == 0) au[r0 / 8 + nx] = axe;
+    av[o / 8] = ay;
+    if (P.bc_y != 1 && j == 0) av[c0 / 8 + (long)ny * ld] = aye;
+  }
+  if (k >= 1 && k <= nz - 2) aw[o / 8] = az;
+  if (k == nz - 2) aw[o / 8 + g.np] = aze;
 }
 
 // the face-velocity reconstruction transposed, along x:
@@ -660,16 +697,15 @@ __global__ void __launch_bounds__(256) k_adj_drop_xyz(const double *__restrict__
 // l the adjoint of the faces (face nx folded into 0) and S = sum l:
 //   adjoint of dudx(m), m < nx-1: dx (sum_{i>m} l(i) - S (nx-1-m)/nx);  of u(m): S/nx.
 // The same along y.
-// The face adjoints of all bins summed (bin by bin in index order, from zero), for
-// k_adj_face_line: one coalesced pass instead of npc strided loads per face inside the
-// line passes.
+// The face adjoints of all groups of bins summed (from zero), for k_adj_face_line: one
+// coalesced pass instead of strided loads per group inside the line passes.
 __global__ void k_adj_face_bins(const double *__restrict__ aui, const double *__restrict__ avi,
-                                double *__restrict__ lu, double *__restrict__ lv, DropGeo g) {
+                                double *__restrict__ lu, double *__restrict__ lv, DropGeo g, int ngrp) {
   const long fz = g.fp * g.nz;
   const long s = gtid();
   if (s >= fz) return;
   double a = 0.0, b = 0.0;
-  for (int q = 0; q < g.npc; ++q) {
+  for (int q = 0; q < ngrp; ++q) {
     a += aui[(long)q * fz + s];
     b += avi[(long)q * fz + s];
   }
@@ -710,12 +746,12 @@ __global__ void __launch_bounds__(256) k_adj_face_line(const double *__restrict_
   }
 }
 
-// afw += the w-face adjoints summed over the bins
-__global__ void k_adj_face_w(const double *__restrict__ awi, double *__restrict__ afw, DropGeo g) {
+// afw += the w-face adjoints summed over the groups of bins
+__global__ void k_adj_face_w(const double *__restrict__ awi, double *__restrict__ afw, DropGeo g, int ngrp) {
   const long s = gtid();
   if (s >= g.nv) return;
   double v = 0.0;
-  for (int b = 0; b < g.npc; ++b) v += awi[(long)b * g.nv + s];
+  for (int b = 0; b < ngrp; ++b) v += awi[(long)b * g.nv + s];
   afw[s] += v;
 }
 

@@ -143,7 +143,7 @@ struct lp_ctx {
   double *ushift = nullptr;
   double *nyq = nullptr;    // filt_da of binary64 velocities, 3 fields: A [nz][ny], B [nz][nx], C [nz]
   double *nyq_part = nullptr;  // their partial column sums [3][nz][kNyqSlices][nx]
-  double *adj_drop = nullptr;  // droplet adjoint scratch: mu, ac, awi volumes + aui, avi faces
+  double *adj_drop = nullptr;  // droplet adjoint scratch: mu, ac volumes, awi, aui, avi
   double *tavg = nullptr;      // running time averages (tavg_nq binary64 volumes)
   int tavg_nq = 0;
   double tavg_time = 0.0;      // tavg_total_time
@@ -2738,13 +2738,16 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
   const lp_droplet_config &D = cf.drop;
   const bool drops = D.npcon > 0 && c->jt_total >= D.pcon_init;
   double *dmu = nullptr, *dac = nullptr, *awi = nullptr, *aui = nullptr, *avi = nullptr;
+  // runs of bins, each with its own face adjoints: one, or as many as give four blocks per CU
+  const long dblk = (long)((gg.nx + 63) / 64) * ((gg.ny + 3) / 4) * gg.nz;
+  const int ngrp = (int)std::min<long>(std::max(D.npcon, 1), (1024 + dblk - 1) / dblk);
   DropGeo dg{};
   if (drops) {
     dg = drop_geo(c);
     const size_t fz = (size_t)dg.fp * gg.nz, nb = (size_t)D.npcon;
-    // mu, ac, awi (a volume per bin) and aui, avi (a face array per bin)
-    if (!c->adj_drop) RCHK(dalloc((void **)&c->adj_drop, sizeof(double) * nb * (3 * (size_t)nv + 2 * fz)));
-    dmu = c->adj_drop; dac = dmu + nb * nv; awi = dac + nb * nv; aui = awi + nb * nv; avi = aui + nb * fz;
+    // mu, ac (a volume per bin), awi (a volume per run of bins) and aui, avi (a face array per run)
+    if (!c->adj_drop) RCHK(dalloc((void **)&c->adj_drop, sizeof(double) * (2 * nb * nv + ngrp * (nv + 2 * fz))));
+    dmu = c->adj_drop; dac = dmu + nb * nv; awi = dac + nb * nv; aui = awi + ngrp * nv; avi = aui + ngrp * fz;
     // base face velocities from the filtered u, v and dudx, dvdy; Kc_t from the frozen Nu_t
     hipLaunchKernelGGL(k_face_u<double>, dim3((unsigned)(((long)gg.ny * gg.nz + 3) / 4)), dim3(256), 0, c->s, uf, ux,
                        c->ui0, dg, gg.dx);
@@ -2752,7 +2755,7 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
                        c->s, vf, vy, c->vi0, dg, gg.dy);
     hipLaunchKernelGGL(k_kc<double>, grid1(dg.nv), dim3(256), 0, c->s, nut, (double *)c->f[LP_MAGS], c->kcell, dg,
                        D.Sc);
-    const long nfill = (long)(nb * (nv + 2 * fz));
+    const long nfill = (long)(ngrp * (nv + 2 * fz));
     hipLaunchKernelGGL(k_fill<double>, grid1(nfill), dim3(256), 0, c->s, awi, nfill, 0.0);
     HIPCHK(hipGetLastError());
     const int euler = (c->jt_total == D.pcon_init || c->jt_total == D.src_jt0) && !D.init_pcon;
@@ -2761,13 +2764,12 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
     const double *PC = (const double *)c->f[LP_PCON];
     hipLaunchKernelGGL(k_adj_drop_update, grid1(dg.nv * D.npcon), dim3(256), 0, c->s, (const double *)cb, rcb,
                        (const double *)arz, (const double *)c->d_vfac, D.active, dmu, dac, dg, dt, euler);
-    // 64 x 4 cells per block, grid z over (level, bin) (nz * npcon checked on entry)
+    // 64 x 4 cells per block, grid z over (level, run of bins) (nz * npcon checked on entry)
     hipLaunchKernelGGL(k_adj_drop_xyz, dim3((unsigned)((gg.nx + 63) / 64), (unsigned)((gg.ny + 3) / 4),
-                       (unsigned)(gg.nz * D.npcon)), dim3(64, 4), 0, c->s, PC, (const double *)dmu, dac,
+                       (unsigned)(gg.nz * ngrp)), dim3(64, 4), 0, c->s, PC, (const double *)dmu, (const double *)dac, cb,
                        (const double *)c->ui0, (const double *)c->vi0, (const double *)wf, aui, avi, awi,
-                       (const double *)c->kcell, (const double *)c->d_ws, dg, P);
+                       (const double *)c->kcell, (const double *)c->d_ws, dg, P, ngrp);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(cb, dac, sizeof(double) * nb * nv, hipMemcpyDeviceToDevice, c->s));
   }
   // ---- convection: P^T, the products transposed, T^T ----
   double *pbx = B[6], *pby = B[7], *pbz = B[8];
@@ -2814,13 +2816,13 @@ static int do_step_adjoint(lp_ctx *c, const double *nut, const double *ust, doub
                      avx, avy, awx, awy, afu, afv, afw, ag, 1.0 / dz, 1.0 / (zl * den), wall);
   HIPCHK(hipGetLastError());
   if (drops) {  // the droplet faces read the filtered u, v, w and dudx, dvdy
-    hipLaunchKernelGGL(k_adj_face_w, gv, dim3(256), 0, c->s, (const double *)awi, afw, dg);
-    // the bin sums of the u and v face adjoints go where mu, ac and awi were (dead now:
-    // 3 npcon nv >= 2 fp nz)
+    hipLaunchKernelGGL(k_adj_face_w, gv, dim3(256), 0, c->s, (const double *)awi, afw, dg, ngrp);
+    // the sums of the u and v face adjoints go where mu, ac and awi were (dead now:
+    // 3 nv >= 2 fp nz)
     const long fz = (long)dg.fp * gg.nz;
     double *lu = dmu, *lv = dmu + fz;
     hipLaunchKernelGGL(k_adj_face_bins, grid1(fz), dim3(256), 0, c->s, (const double *)aui, (const double *)avi, lu, lv,
-                       dg);
+                       dg, ngrp);
     hipLaunchKernelGGL(k_adj_face_line<false>, dim3((unsigned)(((long)gg.ny * gg.nz + 3) / 4)), dim3(256), 0, c->s,
                        (const double *)lu, aux, afu, dg, gg.dx);
     hipLaunchKernelGGL(k_adj_face_line<true>, dim3((unsigned)(((long)gg.nx * gg.nz + 3) / 4)), dim3(256), 0, c->s,

@@ -204,3 +204,61 @@ def test_droplet_transport_tiles(nx, ny, nz, nb, bc, kw):
     assert np.array_equal(lg.download("RHS_PCon")[:, -1], st["RHS_PCon"][:, -1])
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,nb,bc", [(96, 32, 7, 5, (1, 0)),    # a part-filled block, one bin per run
+                                            (32, 64, 6, 2, (2, 1)),
+                                            (128, 64, 20, 7, (0, 2)),  # runs of several bins
+                                            (192, 96, 16, 3, (1, 1))])  # one run
+def test_droplet_adjoint_runs(nx, ny, nz, nb, bc):
+    """the transposed droplet transport over its blocks and runs of bins against the oracle;
+    1e-11, and 1e-10 for the concentration's adjoint, as the adjoint's tests at 32x32x9 (its
+    diffusion terms cancel to a few parts in 1e4 of themselves)"""
+    import ctypes as C
+    import torch
+    from harness import random_fields
+    from oracle import Oracle
+    from population_balance_amd import droplets, ic
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(nx, ny, nz)
+    ds = droplets.DropletSet(nb)
+    ds.fill(cfg, bc=bc, inertia=False)
+    g = cfg.grid
+    print(f"\n[case] droplet adjoint runs {nx}x{ny}x{nz} bins {nb} bc {bc}", flush=True)
+    rng = np.random.default_rng(6)
+    shc = abi.field_shape(g, "PCon", nb)
+
+    def phys(a):
+        a[..., nx:] = 0.0
+        return np.ascontiguousarray(a)
+    n = random_fields(cfg, ["u", "v", "w", "RHSx", "RHSy", "RHSz", "Nu_t", "ustar"], seed=5)
+    ub0, rb0 = np.stack([phys(n[q]) for q in ("u", "v", "w")]), np.stack([phys(n[q]) for q in ("RHSx", "RHSy", "RHSz")])
+    cb0, rcb0 = phys(rng.standard_normal(shc)), phys(rng.standard_normal(shc))
+    rb0[:, -1] = 0.0
+    rcb0[:, -1] = 0.0
+    nut = phys(1e-3 * (1.0 + 0.1 * np.clip(n["Nu_t"], -3, 3)))
+    ust = 1.0 + 0.1 * np.clip(n["ustar"], -3, 3)
+    st = dict(zip(("u", "v", "w"), ic.turbulent_ic(g, seed=4)))
+    st["PCon"] = phys(droplets.initial_concentration(cfg, ds) * (1.0 + 0.3 * rng.random(shc)))
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    for c, put in ((o, o.set_field), (lg, lg.upload)):
+        for name, a in st.items():
+            put(name, a)
+        c.set_time(3, 3)
+    dp = C.POINTER(C.c_double)
+    o.L.or_step_adjoint2.argtypes = [C.c_void_p] + [dp] * 6
+    p = lambda a: a.ctypes.data_as(dp)  # noqa: E731
+    ref = [a.copy() for a in (ub0, rb0, cb0, rcb0)]
+    assert o.L.or_step_adjoint2(o.h, p(nut), p(ust), *(p(a) for a in ref)) == 0
+    dev = [torch.from_numpy(a).to("cuda") for a in (ub0, rb0, cb0, rcb0)]
+    lg.step_adjoint(torch.from_numpy(nut).to("cuda"), torch.from_numpy(ust).to("cuda"), *dev)
+    out = [a.cpu().numpy() for a in dev]
+    for name, a, b, tol in zip(("u", "RHS", "PCon", "RHS_PCon"), out, ref, (1e-11, 1e-11, 1e-10, 1e-11)):
+        top = nz - 1 if name == "RHS" else nz
+        err = rel_l2(a[:, :top], b[:, :top], nx)
+        print(f"  {name}: {err:.2e}", end="")
+        assert err < tol, (name, err)
+    print()
+    assert not out[2][..., nx:].any()
+    lg.close()
+    o.close()
