@@ -23,7 +23,38 @@ struct ObkP {
   double g_;       // g / (u_star^2 / z_i)
 };
 
-// fixed-order block sum of 1024 lanes' partials (red: 1024 doubles of LDS); lane 0
+// element offset of point q of a plane (q < nx ny: 32-bit division)
+__device__ __forceinline__ long plane_at(unsigned q, const Geo &g) {
+  const unsigned y = q / (unsigned)g.nx;
+  return (long)y * g.ld + (q - y * (unsigned)g.nx);
+}
+
+// Fixed-order block sums of N values of 1024 lanes (red: N * 1024 doubles of LDS), the lane
+// o apart added for o = 512 .. 1: through LDS down to one wavefront, by shuffles within it.
+// Lane 0 holds the totals.  One workgroup is latency alone: k_obukhov at 128x96 takes 16.5 us
+// (four sums one after the other, 40 barriers and 64-bit divisions per point: 20.9),
+// k_theta_sfc 9.5 (12.8).
+template <int N> __device__ __forceinline__ void block_sums1024(double (&v)[N], double *red) {
+#pragma unroll
+  for (int q = 0; q < N; ++q) red[q * 1024 + threadIdx.x] = v[q];
+  __syncthreads();
+  for (int o = 512; o >= 64; o >>= 1) {
+    if ((int)threadIdx.x < o)
+#pragma unroll
+      for (int q = 0; q < N; ++q) red[q * 1024 + threadIdx.x] += red[q * 1024 + threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      double r = red[q * 1024 + threadIdx.x];
+      for (int o = 32; o > 0; o >>= 1) r += __shfl_down(r, o, 64);
+      v[q] = r;
+    }
+  }
+}
+
+// fixed-order block sum of 1024 lanes' partials (red: 1024 doubles of LDS); every lane
 // returns the total
 __device__ __forceinline__ double block_sum1024(double v, double *red) {
   red[threadIdx.x] = v;
@@ -44,7 +75,7 @@ __global__ __launch_bounds__(1024) void k_obukhov(const double *__restrict__ u, 
                                                   const double *__restrict__ th, double *__restrict__ t3,
                                                   double *__restrict__ psi, T *__restrict__ ust,
                                                   double *__restrict__ ob, Geo g, ObkP P) {
-  __shared__ double red[1024];
+  __shared__ double red[4 * 1024];
   __shared__ double res[2];
   const long nxy = (long)g.nx * g.ny;
   const double dnxy = (double)nxy;
@@ -53,18 +84,16 @@ __global__ __launch_bounds__(1024) void k_obukhov(const double *__restrict__ u, 
   if (P.zero_psi)  // :1184
     for (long i = threadIdx.x; i < g.np; i += blockDim.x) psi[i] = 0.0;
   __syncthreads();
-  double su = 0.0, sp = 0.0, st = 0.0, sh = 0.0;
-  for (long q = threadIdx.x; q < nxy; q += blockDim.x) {
-    const long i = (q / g.nx) * g.ld + q % g.nx;
-    su += sqrt(u[i] * u[i] + v[i] * v[i]);
-    sp += psi[i];
-    st += t3[i];
-    sh += th ? th[i] : 0.0;
+  double v4[4] = {0.0, 0.0, 0.0, 0.0};
+  for (unsigned q = threadIdx.x; q < (unsigned)nxy; q += 1024) {
+    const long i = plane_at(q, g);
+    v4[0] += sqrt(u[i] * u[i] + v[i] * v[i]);
+    v4[1] += psi[i];
+    v4[2] += t3[i];
+    v4[3] += th ? th[i] : 0.0;
   }
-  su = block_sum1024(su, red);
-  sp = block_sum1024(sp, red);
-  st = block_sum1024(st, red);
-  sh = block_sum1024(sh, red);
+  block_sums1024<4>(v4, red);
+  const double su = v4[0], sp = v4[1], st = v4[2], sh = v4[3];  // lane 0
   if (threadIdx.x == 0) {
     if (!P.stab) {  // :1183-1193
       const double us = su / dnxy * P.vonk / (P.lz0 - sp / dnxy);
@@ -97,8 +126,8 @@ __global__ __launch_bounds__(1024) void k_obukhov(const double *__restrict__ u, 
     }
   }
   __syncthreads();
-  for (long q = threadIdx.x; q < nxy; q += blockDim.x) {
-    const long i = (q / g.nx) * g.ld + q % g.nx;
+  for (unsigned q = threadIdx.x; q < (unsigned)nxy; q += 1024) {
+    const long i = plane_at(q, g);
     if (P.stab) psi[i] = res[0];
     ust[i] = (T)res[1];
   }
@@ -114,12 +143,13 @@ __global__ __launch_bounds__(1024) void k_theta_sfc(const T *__restrict__ ust, c
   __shared__ double val;
   const long nxy = (long)g.nx * g.ny;
   const double dnxy = (double)nxy;
-  double s = 0.0;
-  for (long q = threadIdx.x; q < nxy; q += blockDim.x) s += (double)ust[(q / g.nx) * g.ld + q % g.nx] / dnxy;
-  s = block_sum1024(s, red);
-  if (threadIdx.x == 0) val = -ob[3] * sflux / (s * vonk * dz / 2.0);
+  double s1[1] = {0.0};
+#pragma unroll 4
+  for (unsigned q = threadIdx.x; q < (unsigned)nxy; q += 1024) s1[0] += (double)ust[plane_at(q, g)] / dnxy;
+  block_sums1024<1>(s1, red);
+  if (threadIdx.x == 0) val = -ob[3] * sflux / (s1[0] * vonk * dz / 2.0);
   __syncthreads();
-  for (long q = threadIdx.x; q < nxy; q += blockDim.x) dTdz[(q / g.nx) * g.ld + q % g.nx] = (T)val;
+  for (unsigned q = threadIdx.x; q < (unsigned)nxy; q += 1024) dTdz[plane_at(q, g)] = (T)val;
 }
 
 // :827-874 advection on the 3/2 grid, written over u_m (each node reads only its own
@@ -211,7 +241,8 @@ static __global__ __launch_bounds__(1024) void k_level_mean(const double *__rest
   const int k = blockIdx.x;
   const long nxy = (long)g.nx * g.ny;
   double s = 0.0;
-  for (long q = threadIdx.x; q < nxy; q += blockDim.x) s += th[(long)k * g.np + (q / g.nx) * g.ld + q % g.nx];
+#pragma unroll 4
+  for (unsigned q = threadIdx.x; q < (unsigned)nxy; q += blockDim.x) s += th[(long)k * g.np + plane_at(q, g)];
   s = block_sum1024(s, red);
   if (threadIdx.x == 0) bar[k] = s / (double)nxy;
 }
