@@ -81,7 +81,9 @@ template <typename T, int R, int SIGN> struct Dft {
     } else if constexpr (R == 2 || R == 3 || R == 4) {
       SmallDft<T, R, SIGN>::run(v);
     } else {
-      constexpr int A = (R == 8) ? 2 : (R == 12) ? 3 : (R % 4 == 0) ? 4 : (R % 2 == 0) ? 2 : 3;
+      // 2 x 4 and 3 x 4 in binary64, 4 x 2 and 4 x 3 in binary32: the same cost, other roundings
+      constexpr bool W = sizeof(T) == 8;
+      constexpr int A = (W && R == 8) ? 2 : (W && R == 12) ? 3 : (R % 4 == 0) ? 4 : (R % 2 == 0) ? 2 : 3;
       constexpr int B = R / A;
       cx<T> y[A][B];
 #pragma unroll
