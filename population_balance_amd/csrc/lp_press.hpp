@@ -16,7 +16,7 @@
 // read and written again.  Segments give 8 to 32 times the threads, one read of H and one
 // write of p_hat.  16 modes (128 or 256 bytes a row) per block keep every access whole
 // 128-byte lines (modes are taken in the spectra's own pitch, not as kx + lh ky), and at
-// 124 VGPRs (binary32) two blocks of 512 threads share a CU, so that one block's loads run
+// 122 VGPRs (binary32) two blocks of 512 threads share a CU, so that one block's loads run
 // beside the other's sweeps.  RNDS false leaves out the loop over rounds, which would cost
 // 60 registers.  Measured, one thread per mode -> this: binary32 spectra 246 -> 99 us at
 // 256 x 256 x 257 (H, 1/bet and p_hat: 480 MB, 4.9 TB/s), 94 -> 32 us at 192 x 192 x 128;
@@ -64,14 +64,33 @@ static __global__ void k_press_factors(const double *__restrict__ kxt, const dou
   }
 }
 
-// element of a spectrum or table at a byte offset that fits 32 bits (a plane holds at most
-// 256 x 144 values of 16 bytes, and memory far fewer than 2^32 bytes of them)
-template <typename E> __device__ __forceinline__ E at_byte(const E *base, unsigned off) {
-  return *reinterpret_cast<const E *>(reinterpret_cast<const char *>(base) + off);
+// Addresses.  A volume of spectra may be larger than 4 GiB (256 x 256 modes from 7282 rows of
+// 16 bytes on), so a row's place in it takes 64 bits.  The rows of a wavefront's 64 / kPsModes
+// segments follow one another: the address of the first (row0) is uniform and stays in scalar
+// registers, and a lane adds a 32-bit offset within the next (64 / kPsModes) kPsRows + 1 rows of at
+// most 256 x 144 values, 22 MB.  row >= row0.
+__host__ __device__ constexpr unsigned row_off(int row, int row0, unsigned ps, unsigned o, unsigned bytes) {
+  return ((unsigned)(row - row0) * ps + o) * bytes;
+}
+__host__ __device__ constexpr long row_base(int row0, unsigned ps) { return (long)row0 * (long)ps; }
+
+template <typename E>
+__device__ __forceinline__ E at_row(const E *base, int row, int row0, unsigned ps, unsigned o) {
+  return *reinterpret_cast<const E *>(reinterpret_cast<const char *>(base + row_base(row0, ps)) +
+                                      row_off(row, row0, ps, o, sizeof(E)));
 }
 
-template <typename E> __device__ __forceinline__ void put_byte(E *base, unsigned off, E v) {
-  *reinterpret_cast<E *>(reinterpret_cast<char *>(base) + off) = v;
+template <typename E>
+__device__ __forceinline__ void put_row(E *base, int row, int row0, unsigned ps, unsigned o, E v) {
+  *reinterpret_cast<E *>(reinterpret_cast<char *>(base + row_base(row0, ps)) + row_off(row, row0, ps, o, sizeof(E))) = v;
+}
+
+// the plane of an H level or gradient, levels 1 .. nz-1 at planes 0 .. nz-2, of row j (clamped)
+__host__ __device__ constexpr int press_plane(int j, int nz) { return j < 1 ? 0 : j > nz - 1 ? nz - 2 : j - 1; }
+
+// the first segment of the thread's wavefront
+__device__ __forceinline__ int wave_seg() {
+  return __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64 * (64 / kPsModes));
 }
 
 template <int S> struct SegLds {
@@ -109,8 +128,9 @@ __device__ __forceinline__ cx<double> seg_enter(SegLds<S> &L, int s, int l, doub
 }
 
 // The two sweeps of one block, u(j) = r(j) - f(j) u(j-1) with rows up, then
-// p(j) = u(j) - fb(j, f(j)) p(j+1) down.  load(j0, Lr) fills r and f of this thread's rows
-// j0 .. j0 + Lr - 1 (clamped beyond n); out(j, p(j), p(j+1)) takes the solution.  u: scratch
+// p(j) = u(j) - fb(j, f(j)) p(j+1) down.  load(j0, jw, Lr) fills r and f of this thread's rows
+// j0 .. j0 + Lr - 1 (clamped beyond n); out(j, jw, p(j), p(j+1)) takes the solution.  jw is the
+// first row of the wavefront's segments (uniform, it may lie beyond n).  u: scratch
 // for the rounds but the last (n > S kPsRows), [n][plane], this thread's own rows.
 template <int S, bool RNDS, typename Load, typename Fb, typename Out>
 __device__ __forceinline__ void seg_solve(SegLds<S> &L, int s, int l, int n, Load load, Fb fb, Out out,
@@ -119,11 +139,12 @@ __device__ __forceinline__ void seg_solve(SegLds<S> &L, int s, int l, int n, Loa
   const int per = (n + S - 1) / S;
   const int Lr = per < kPsRows ? per : kPsRows;
   const int rounds = RNDS ? (n + S * Lr - 1) / (S * Lr) : 1;
+  const int sw = wave_seg();
   cx<double> carry = mk<double>(0.0, 0.0), last;
   for (int rd = 0; rd < rounds; ++rd) {
-    const int j0 = (rd * S + s) * Lr;
+    const int j0 = (rd * S + s) * Lr, jw = (rd * S + sw) * Lr;
     const int nr = n - j0 < Lr ? n - j0 : Lr;  // rows of this segment (none: <= 0)
-    load(j0, Lr);
+    load(j0, jw, Lr);
     double A = 1.0;
     cx<double> B = mk<double>(0.0, 0.0);
 #pragma unroll
@@ -147,10 +168,10 @@ __device__ __forceinline__ void seg_solve(SegLds<S> &L, int s, int l, int n, Loa
   }
   carry = mk<double>(0.0, 0.0);
   for (int rd = rounds - 1; rd >= 0; --rd) {
-    const int j0 = (rd * S + s) * Lr;
+    const int j0 = (rd * S + s) * Lr, jw = (rd * S + sw) * Lr;
     const int nr = n - j0 < Lr ? n - j0 : Lr;
     if (rd + 1 < rounds) {
-      load(j0, Lr);  // f again; r is replaced by the forward sweep's values
+      load(j0, jw, Lr);  // f again; r is replaced by the forward sweep's values
 #pragma unroll
       for (int q = 0; q < kPsRows; ++q)
         if (q < nr) r[q] = u[(size_t)(j0 + q) * plane];
@@ -172,7 +193,7 @@ __device__ __forceinline__ void seg_solve(SegLds<S> &L, int s, int l, int n, Loa
         const double g = fb(j0 + q, f[q]);
         const cx<double> up = v;
         v = mk<double>(r[q].x - g * v.x, r[q].y - g * v.y);
-        out(j0 + q, v, up);
+        out(j0 + q, jw, v, up);
       }
   }
 }
@@ -196,12 +217,13 @@ __device__ __forceinline__ void seg_solve_serial(cx<double> (&end)[kPsModes], in
   const int per = (n + S - 1) / S;
   const int Lr = per < kPsRows ? per : kPsRows;
   const int rounds = RNDS ? (n + S * Lr - 1) / (S * Lr) : 1;
+  const int sw = wave_seg();
   double rb[kPsRows];
   if (s == 0) end[l] = mk<double>(0.0, 0.0);
   for (int rd = 0; rd < rounds; ++rd) {
-    const int j0 = (rd * S + s) * Lr;
+    const int j0 = (rd * S + s) * Lr, jw = (rd * S + sw) * Lr;
     const int nr = n - j0 < Lr ? n - j0 : Lr;
-    load(j0, Lr);
+    load(j0, jw, Lr);
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) rb[q] = 1.0 / f[q];
     __syncthreads();
@@ -225,10 +247,10 @@ __device__ __forceinline__ void seg_solve_serial(cx<double> (&end)[kPsModes], in
   }
   if (s == 0) end[l] = mk<double>(0.0, 0.0);
   for (int rd = rounds - 1; rd >= 0; --rd) {
-    const int j0 = (rd * S + s) * Lr;
+    const int j0 = (rd * S + s) * Lr, jw = (rd * S + sw) * Lr;
     const int nr = n - j0 < Lr ? n - j0 : Lr;
     if (rd + 1 < rounds) {
-      load(j0, Lr);
+      load(j0, jw, Lr);
 #pragma unroll
       for (int q = 0; q < kPsRows; ++q) {
         rb[q] = 1.0 / f[q];
@@ -253,7 +275,7 @@ __device__ __forceinline__ void seg_solve_serial(cx<double> (&end)[kPsModes], in
     }
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q)
-      if (q < nr) out(j0 + q, r[q], r[q]);
+      if (q < nr) out(j0 + q, jw, r[q], r[q]);
   }
 }
 
@@ -289,21 +311,22 @@ __global__ __launch_bounds__(kPsModes *S, RNDS ? 1 : sizeof(TH) == 4 ? 4 : 3) vo
   bool bad = false;
   // the coefficient below the diagonal: 1/dz^2, -1 in the lid row and for the mean's sum
   auto below = [&](int j) { return !live || j == 0 ? 0.0 : (mean || j == nz) ? -1.0 : idz2; };
-  auto load = [&](int j0, int Lr) {
+  auto load = [&](int j0, int jw, int Lr) {
     cx<TH> hz[kPsRows + 1], hx[kPsRows], hy[kPsRows];
     double ib[kPsRows];
-    auto plane_of = [&](int j) { return (unsigned)(j < 1 ? 0 : j > nz - 1 ? nz - 2 : j - 1); };
+    const int pw = press_plane(jw, nz), tw0 = jw > nz ? nz : jw;
     auto row_of = [&](int q) { return j0 + (q < Lr ? q : Lr - 1); };
+    auto at_h = [&](const cx<TH> *H, int j) { return at_row(H, press_plane(j, nz), pw, psu, ocu); };
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) {
       const int j = row_of(q);
-      ib[q] = at_byte(tab, ((unsigned)(j > nz ? nz : j) * psu + ocu) * 8u);
-      hz[q] = at_byte(Hz, (plane_of(j) * psu + ocu) * (unsigned)sizeof(cx<TH>));
+      ib[q] = at_row(tab, j > nz ? nz : j, tw0, psu, ocu);
+      hz[q] = at_h(Hz, j);
     }
-    hz[kPsRows] = at_byte(Hz, (plane_of(j0 + Lr) * psu + ocu) * (unsigned)sizeof(cx<TH>));
+    hz[kPsRows] = at_h(Hz, j0 + Lr);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < kPsRows; ++q) hx[q] = at_byte(Hx, (plane_of(row_of(q)) * psu + ocu) * (unsigned)sizeof(cx<TH>));
+    for (int q = 0; q < kPsRows; ++q) hx[q] = at_h(Hx, row_of(q));
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) {  // (Hz(j+1) - Hz(j))/dz, H_z zero at level nz
       const int j = j0 + q;
@@ -315,7 +338,7 @@ __global__ __launch_bounds__(kPsModes *S, RNDS ? 1 : sizeof(TH) == 4 ? 4 : 3) vo
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < kPsRows; ++q) hy[q] = at_byte(Hy, (plane_of(row_of(q)) * psu + ocu) * (unsigned)sizeof(cx<TH>));
+    for (int q = 0; q < kPsRows; ++q) hy[q] = at_h(Hy, row_of(q));
     const cx<TH> b0 = bw[oc], t0 = tw_[oc];
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) {
@@ -344,8 +367,8 @@ __global__ __launch_bounds__(kPsModes *S, RNDS ? 1 : sizeof(TH) == 4 ? 4 : 3) vo
       }
     }
   };
-  auto out = [&](int j, cx<double> p, cx<double>) {
-    if (store) put_byte(ph, ((unsigned)j * psu + (unsigned)o) * 16u, p);
+  auto out = [&](int j, int jw, cx<double> p, cx<double>) {
+    if (store) put_row(ph, j, jw, psu, (unsigned)o, p);
   };
   // above the diagonal 1/dz^2 as below; 1 in the wall row (bet = -1), nothing in the lid row
   if constexpr (DIV) {
@@ -394,10 +417,10 @@ __global__ __launch_bounds__(kPsModes *S) void k_press_adj(
   const cx<double> z0 = mk<double>(0.0, 0.0);
   cx<double> r[kPsRows];
   double f[kPsRows];
-  auto load = [&](int j0, int Lr) {
+  auto load = [&](int j0, int jw, int Lr) {
     cx<double> a[kPsRows], b[kPsRows];
     double ib[kPsRows];
-    auto plane_of = [&](int j) { return (unsigned)(j < 1 ? 0 : j > nz - 1 ? nz - 2 : j - 1); };
+    const int pw = press_plane(jw, nz), tw0 = jw > nz ? nz : jw, sw0 = jw > nz - 1 ? nz - 1 : jw;
     auto row_of = [&](int q) {
       const int j = j0 + (q < Lr ? q : Lr - 1);
       return j > nz ? nz : j;
@@ -405,15 +428,15 @@ __global__ __launch_bounds__(kPsModes *S) void k_press_adj(
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) {
       const int j = row_of(q);
-      ib[q] = at_byte(tab, ((unsigned)j * psu + ocu) * 8u);  // bet
-      r[q] = at_byte(Sp, ((unsigned)(j < nz ? j : nz - 1) * psu + ocu) * 16u);
+      ib[q] = at_row(tab, j, tw0, psu, ocu);  // bet
+      r[q] = at_row(Sp, j < nz ? j : nz - 1, sw0, psu, ocu);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < kPsRows; ++q) a[q] = at_byte(Sx, (plane_of(row_of(q)) * psu + ocu) * 16u);
+    for (int q = 0; q < kPsRows; ++q) a[q] = at_row(Sx, press_plane(row_of(q), nz), pw, psu, ocu);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < kPsRows; ++q) b[q] = at_byte(Sy, (plane_of(row_of(q)) * psu + ocu) * 16u);
+    for (int q = 0; q < kPsRows; ++q) b[q] = at_row(Sy, press_plane(row_of(q), nz), pw, psu, ocu);
 #pragma unroll
     for (int q = 0; q < kPsRows; ++q) {
       const int j = row_of(q);
@@ -435,7 +458,7 @@ __global__ __launch_bounds__(kPsModes *S) void k_press_adj(
     if (!live || j == nz) return 0.0;
     return j == 0 ? -idz2 : j == 1 ? idz2 * fj : j == nz - 1 ? -(dz * dz) * fj : fj;
   };
-  auto out = [&](int j, cx<double> lj, cx<double> nxt) {
+  auto out = [&](int j, int, cx<double> lj, cx<double> nxt) {
     if (!store) return;
     if (mean) {  // :303-312: p(1) = -dz bw, p(j) = p(j-1) + dz Hz(j)
       if (j == nz) tw[o] = z0;
