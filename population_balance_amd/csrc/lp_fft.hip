@@ -791,6 +791,11 @@ hipError_t row_c2r(Dt dtc, Dt dto, int M, const C2rSet *sets, int n, long in_pit
 #undef CASE
 }
 
+// Planes of a column launch: they lie along y, where a grid has at most 65535 blocks.  Lists of
+// more (the test filters' 21 fields from 3121 levels on) are launched one set and this many
+// planes at a time, whole groups of eight.
+constexpr int kMaxPlanes = 65528;
+
 // col0 > 0: the columns col0..ncols-1 only (same grid, one column per block)
 template <typename T, int NYI, int NYO, int N>
 static hipError_t launch_col_n(int padmode, int fwd, int inv, const ColSet *sets, int n, long in_pitch, long in_plane,
@@ -826,7 +831,6 @@ static hipError_t launch_col_n(int padmode, int fwd, int inv, const ColSet *sets
     groups += xcd_planes(x.nplanes, 0);
   }
   const unsigned gy = (unsigned)(xcd_order<T>() ? 8 * groups : planes);
-  if (gy > 65535u) return hipErrorInvalidValue;
   if (col0 > 0) {
     if constexpr (NYI == NYO) {
       hipExtLaunchKernelGGL((k_col_op<T, NYI, NYO, N, 1>), dim3((unsigned)(ncols - col0), gy), dim3(kColLanes), 0, s,
@@ -847,6 +851,29 @@ template <typename T, int NYI, int NYO>
 static hipError_t launch_col(int padmode, int fwd, int inv, const ColSet *sets, int n, long in_pitch, long in_plane,
                              int ncols, long out_pitch, long out_plane, const SpecTables &tab, hipStream_t s, Dt dt,
                              int col0 = 0, LaunchEv ev = {}) {
+  long gy = 0;
+  for (int f = 0; f < n; ++f) gy += xcd_order<T>() ? 8L * xcd_planes(sets[f].nplanes, 0) : sets[f].nplanes;
+  if (gy > kMaxPlanes) {
+    for (int f = 0; f < n; ++f) {
+      const int np = sets[f].nplanes;
+      int p0 = 0;
+      do {
+        ColSet x = sets[f];
+        x.in = (const cx<T> *)x.in + p0 * in_plane;
+        x.nplanes = np - p0 < kMaxPlanes ? np - p0 : kMaxPlanes;
+        if (x.dc) x.dc += p0;
+        for (int j = 0; j < x.nout && j < 3; ++j)
+          x.outs[j].ptr = (cx<T> *)x.outs[j].ptr + p0 * (x.outs[j].plane ? x.outs[j].plane : out_plane);
+        const bool last = f == n - 1 && np - p0 <= kMaxPlanes;
+        const hipError_t e = launch_col_n<T, NYI, NYO, 1>(
+            padmode, fwd, inv, &x, 1, in_pitch, in_plane, ncols, out_pitch, out_plane, tab, s, dt, col0,
+            LaunchEv{f == 0 && p0 == 0 ? ev.start : nullptr, last ? ev.stop : nullptr});
+        if (e != hipSuccess) return e;
+        p0 += kMaxPlanes;
+      } while (p0 < np);
+    }
+    return hipSuccess;
+  }
   return n == 1 ? launch_col_n<T, NYI, NYO, 1>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols, out_pitch,
                                                out_plane, tab, s, dt, col0, ev)
                 : launch_col_n<T, NYI, NYO, kMaxSets>(padmode, fwd, inv, sets, n, in_pitch, in_plane, ncols,
