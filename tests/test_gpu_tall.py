@@ -43,16 +43,17 @@ def test_padd_planes(prec):
     o.close()
 
 
-@pytest.mark.parametrize("nz", [3121])
-def test_steps_tall(nz):
-    """binary64 steps with the dynamic model, whose test filters take 21 nz planes; bounds as in
-    test_lag_level_runs (the averages are rounded to REAL(4), and RHS holds their result)"""
+@pytest.mark.parametrize("nz,model", [(2100, 5), (3121, 5), (3121, 4)])
+def test_steps_tall(nz, model):
+    """binary64 steps, two fields a launch (2100 levels) and one (3121); the test filters of model
+    5 take 21 nz planes.  Bounds as in test_lag_level_runs (the averages are rounded to REAL(4),
+    and RHS holds their result)"""
     from harness import load_gpu, load_oracle, seeded_state
     from oracle import Oracle
     from population_balance_amd.lesgo import Lesgo
-    cfg = _tall(32, 32, nz, cs_count=1)
+    cfg = _tall(32, 32, nz, cs_count=1, model=model)
     o, lg = Oracle(cfg), Lesgo(cfg)
-    print(f"\n[case] steps 32x32x{nz}", flush=True)
+    print(f"\n[case] steps 32x32x{nz} model {model}", flush=True)
     st = seeded_state(cfg)
     load_oracle(o, st)
     load_gpu(lg, st)
@@ -64,6 +65,72 @@ def test_steps_tall(nz):
         err = rel_l2(lg.download(n)[:top], o.field(n)[:top], cfg.grid.nx)
         print(f"  {n}: {err:.2e}", end="")
         assert err < (1e-6 if n[0] in "CF" else 1e-11 if n[0] == "R" else TOL), (n, err)
+    print()
+    lg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("nz", [4200, 6200])
+def test_steps_tall_theta_mixed(nz):
+    """binary32 steps with theta, two fields a launch and one, at the bound of
+    test_steps_with_theta_mixed"""
+    from test_gpu_theta import _cfg, _load, _pair, _theta_state
+    cfg = _cfg(nz=nz, L_z=(nz - 1) / 32.0, wt_s=0.1, dTdz_top=0.01, precision=abi.LP_MIXED)
+    g = cfg.grid
+    o, lg = _pair(cfg)
+    st = _theta_state(cfg)
+    for n in ("RHS_T", "Nu_t", "ustar"):
+        st.pop(n)
+    _load(o, lg, st)
+    print(f"\n[case] steps with theta mixed 32x32x{nz}", flush=True)
+    o.step(2)
+    lg.step(2)
+    errs = {n: rel_l2(lg.download(n), o.field(n), g.nx) for n in ("u", "v", "w")}
+    th0 = st["theta"]
+    errs["theta change"] = rel_l2(lg.download("theta") - th0, o.field("theta") - th0, g.nx)
+    print({k: f"{v:.2e}" for k, v in errs.items()})
+    assert max(errs.values()) < 1e-5, errs
+    lg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("nz", [2100, 3121])
+def test_adjoint_tall(nz):
+    """the adjoint step, two fields a launch and one, at the bound of test_adjoint_row_segments"""
+    import ctypes as C
+    import torch
+    from harness import random_fields
+    from oracle import Oracle
+    from population_balance_amd import ic
+    from population_balance_amd.lesgo import Lesgo
+    cfg = _tall(32, 32, nz)
+    g = cfg.grid
+    print(f"\n[case] adjoint 32x32x{nz}", flush=True)
+    vel = dict(zip(("u", "v", "w"), ic.turbulent_ic(g, seed=4)))
+    n = random_fields(cfg, ["u", "v", "w", "RHSx", "RHSy", "RHSz", "Nu_t", "ustar"], seed=5)
+    ub0 = np.stack([n["u"], n["v"], n["w"]])
+    rb0 = np.stack([n["RHSx"], n["RHSy"], n["RHSz"]])
+    rb0[:, -1] = 0.0
+    nut = 1e-3 * (1.0 + 0.1 * np.clip(n["Nu_t"], -3, 3))
+    ust = 1.0 + 0.1 * np.clip(n["ustar"], -3, 3)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    for name, a in vel.items():
+        o.set_field(name, a)
+        lg.upload(name, a)
+    o.set_time(3)
+    lg.set_time(3)
+    dp = C.POINTER(C.c_double)
+    o.L.or_step_adjoint.argtypes = [C.c_void_p, dp, dp, dp, dp]
+    p = lambda a: a.ctypes.data_as(dp)  # noqa: E731
+    ub_o, rb_o = ub0.copy(), rb0.copy()
+    assert o.L.or_step_adjoint(o.h, p(nut), p(ust), p(ub_o), p(rb_o)) == 0
+    ub, rb, tn, tu = (torch.from_numpy(a).to("cuda") for a in (ub0, rb0, nut, ust))
+    lg.step_adjoint(tn, tu, ub, rb)
+    for q in range(3):
+        eu = rel_l2(ub[q].cpu().numpy(), ub_o[q], g.nx)
+        er = rel_l2(rb[q].cpu().numpy()[:nz - 1], rb_o[q][:nz - 1], g.nx)
+        print(f"  {eu:.2e} {er:.2e}", end="")
+        assert eu < TOL and er < TOL, (q, eu, er)
     print()
     lg.close()
     o.close()
