@@ -262,3 +262,77 @@ def test_droplet_adjoint_runs(nx, ny, nz, nb, bc):
     assert not out[2][..., nx:].any()
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(96, 32, 7), (192, 64, 5)])
+def test_dealias_uneven_mixed(nx, ny, nz):
+    """the binary32 rows of 72, 96, 144 and 192 points, at the bound that the binary32 filt_da,
+    which takes as many passes, has"""
+    from oracle import Oracle
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(nx, ny, nz, precision=abi.LP_MIXED)
+    o, lg = Oracle(abi.copy_config(cfg, precision=abi.LP_FP64)), Lesgo(cfg)
+    g = cfg.grid
+    print(f"\n[case] dealias mixed {nx}x{ny}x{nz}", flush=True)
+    u = np.random.default_rng(11).standard_normal((g.nz, g.ny, g.ld)).astype(np.float32)
+    big = np.zeros((g.nz, g.ny2, g.ld_big), np.float32)
+    lg.dealias1(u, big)
+    ref = o.dealias1(u.astype(np.float64))
+    e1 = rel_l2(big, ref, g.nx2)
+    big = ref.astype(np.float32)
+    out = np.zeros_like(u)
+    lg.dealias2(out, big.copy())
+    e2 = rel_l2(out, o.dealias2(big.astype(np.float64)), g.nx)
+    print(f"  {e1:.2e} {e2:.2e}")
+    assert e1 < 1e-6 and e2 < 1e-6, (e1, e2)
+    lg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("ny,nz", [(32, 7), (64, 9)])
+def test_steps_192(ny, nz):
+    """whole binary64 steps with 144-point convection rows; bounds as in test_lag_level_runs"""
+    from harness import load_gpu, load_oracle, seeded_state
+    from oracle import Oracle
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(192, ny, nz)
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    print(f"\n[case] steps 192x{ny}x{nz}", flush=True)
+    st = seeded_state(cfg)
+    load_oracle(o, st)
+    load_gpu(lg, st)
+    for _ in range(3):
+        o.step(1)
+        lg.step(1)
+    for n, top in [(n, nz - 1) for n in ("u", "v", "w", "RHSx", "RHSy", "RHSz")] + [("p", nz)]:
+        err = rel_l2(lg.download(n)[:top], o.field(n)[:top], 192)
+        print(f"  {n}: {err:.2e}", end="")
+        assert err < (1e-11 if n[0] == "R" else TOL), (n, err)
+    print()
+    lg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(96, 32, 17), (192, 32, 9), (96, 192, 8)])
+def test_steps_theta_uneven_mixed(nx, ny, nz):
+    """binary32 steps with theta over the 72- and 144-point rows (convection, the padding of
+    velocities and theta), at the bound of test_steps_with_theta_mixed"""
+    from test_gpu_theta import _load, _pair, _theta_state
+    cfg = abi.make_config(nx, ny, nz, precision=abi.LP_MIXED, L_z=1.5)
+    abi.set_scalar_defaults(cfg.scal, s_flag=1)
+    cfg.scal.wt_s, cfg.scal.dTdz_top = 0.1, 0.01
+    o, lg = _pair(cfg)
+    st = _theta_state(cfg)
+    for n in ("RHS_T", "Nu_t", "ustar"):
+        st.pop(n)
+    _load(o, lg, st)
+    print(f"\n[case] steps with theta mixed {nx}x{ny}x{nz}", flush=True)
+    o.step(2)
+    lg.step(2)
+    errs = {n: rel_l2(lg.download(n), o.field(n), nx) for n in ("u", "v", "w")}
+    th0 = st["theta"]
+    errs["theta change"] = rel_l2(lg.download("theta") - th0, o.field("theta") - th0, nx)
+    print({k: f"{v:.2e}" for k, v in errs.items()})
+    assert max(errs.values()) < 1e-5, errs
+    lg.close()
+    o.close()
