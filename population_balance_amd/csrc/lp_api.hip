@@ -825,9 +825,6 @@ extern "C" int lp_get_time(lp_ctx *c, int32_t *jt, int32_t *jt_total) {
 // spectral pipelines (all asynchronous on c->s)
 // ------------------------------------------------------------------------------------
 // compulsory bytes of the FFT passes (input read once, output written once)
-static double bytes_r2c(int nx, int rows, int nlev, int ncols_out, size_t e) {
-  return (double)rows * nlev * ((double)nx * e + (double)ncols_out * 2 * e);
-}
 static double bytes_c2r(int nx, int rows, int nlev, int ncols_in, size_t ei, size_t eo) {
   return (double)rows * nlev * ((double)ncols_in * 2 * ei + (double)nx * eo);
 }
@@ -1514,7 +1511,7 @@ static int divstress_from_spectra(lp_ctx *c, const DivField *F, int n) {
     for (int q = 0; q < m; ++q) {
       const DivField &a = F[i + q];
       d[q] = DivSet{a.sx, a.sy, a.work};
-      o[q] = C2rSet{a.work, a.divt, g.nz, nullptr, a.tz, a.is_w ? 2 : 1};
+      o[q] = C2rSet{a.work, a.divt, g.nz, a.tz, a.is_w ? 2 : 1};
     }
     prof_begin(c, LP_K_COL_DIV);
     HIPCHK(col_div(c->fdt, g.ny, d, m, g.nz, c->sp, ps, g.lh, c->tab, c->s));
@@ -1764,12 +1761,11 @@ static int do_pollen_rhs(lp_ctx *c, const double *prev, bool fuse_step = false, 
   PollenParams P;
   P.idx = 1.0 / gg.dx; P.idy = 1.0 / gg.dy; P.idz = 1.0 / gg.dz;
   P.idx2 = 1.0 / (gg.dx * gg.dx); P.idy2 = 1.0 / (gg.dy * gg.dy); P.idz2 = 1.0 / (gg.dz * gg.dz);
-  P.ghat = D.g / (D.u_star * D.u_star / D.z_i);
   P.psf = D.sfc_flux > 0 ? 0.0 : D.sfc_flux;  // :2287-2467, lbcp = 1
   P.frac = D.src_frac;
   P.frac1 = 1.0 - D.src_frac;
   P.bc_x = D.bc_x; P.bc_y = D.bc_y;
-  P.settling = D.settling; P.inertia = D.inertia;
+  P.settling = D.settling;
   P.src_on = c->jt_total >= D.src_jt0 && c->jt_total < D.src_jt1;
   P.src_k0 = D.src_k - 1;
   const double nb = (double)dg.nv * dg.npc * 8.0;

@@ -18,9 +18,9 @@
 
 namespace lp {
 
-// lanes per transform: 16 for the long transforms (Q = 12 for M = 192, 9 for M = 144),
+// lanes per transform: 16 for the longest (Q = 12 for M = 192; row_lanes gives 16 for M = 144),
 // which keeps the per-lane values of a transform within the register budget
-__host__ __device__ constexpr int cv_lanes(int M) { return (M == 192 || M == 144) ? 16 : row_lanes(M); }
+__host__ __device__ constexpr int cv_lanes(int M) { return M == 192 ? 16 : row_lanes(M); }
 
 template <typename T, int M> struct CvCfg {
   static constexpr int P = cv_lanes(M);

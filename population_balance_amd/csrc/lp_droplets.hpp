@@ -141,11 +141,10 @@ __device__ __forceinline__ double sign1(double x) { return signbit(x) ? -1.0 : 1
 struct PollenParams {
   double idx, idy, idz;     // 1/dx, 1/dy, 1/dz
   double idx2, idy2, idz2;  // 1/dx^2 ...
-  double ghat;              // g/(u*^2/z_i): PCon_acc time-scale divisor
   double psf;               // surface flux (lbcp = 1 keeps only negative values)
   double frac, frac1;       // source shares of levels src_k and src_k+1
   int bc_x, bc_y;           // 0 periodic, 1 inlet, 2 upwind-sign ghosts
-  int settling, inertia;
+  int settling;
   int src_on, src_k0;       // source active this step; its lower level (0-based)
 };
 

@@ -85,7 +85,6 @@ template <typename T, typename TO> struct C2rArg {
   int np;
   int w;  // div: 1 the w-node form
   const TO *tz;
-  const double *shift;
 };
 
 // ---------------------------------------------------------------------------------
@@ -215,9 +214,7 @@ __global__ __launch_bounds__(kR2cBlock) void k_row_r2c(Sets<R2cArg<T, TI>, N> A,
 // wall at level 1 and no lid term) the transform plus dz^-1 (tz(k) - tz(k-1)) on levels
 // 1..nz-2.  The padding columns are zero (BOGUS on the uv top level).  tz has the layout of
 // out.  IKX: the input is multiplied by i*ikx[kx] first, which turns the (kx, y) spectrum of f
-// into that of df/dx (ddx.f90:15-24; kx is uniform along y).  shift (optional): shift[plane] is
-// added to every stored value of the plane in binary64 (the inverse of k_row_r2c's shift;
-// padding columns stay zero).
+// into that of df/dx (ddx.f90:15-24; kx is uniform along y).
 template <typename T, typename TO, int M, int N, bool DIV, bool IKX = false>
 __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(Sets<C2rArg<T, TO>, N> A, long in_pitch, long in_plane,
                                                        int ncols_in, unsigned rows, unsigned total, long out_pitch,
@@ -293,14 +290,11 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(Sets<C2rArg<T, TO>, 
   // neighbour levels, clamped: uv k + 1 and k, w k and k - 1
   const TO *tzr = DIV ? S.tz + od : nullptr;
   const long up = isw || top ? 0 : out_plane, dn = isw && mid ? out_plane : 0;
-  const double *shp = DIV ? nullptr : S.shift;
-  const double sh = shp && valid ? shp[plane] : 0.0;
   auto fin = [&](T v, int x) -> TO {
     if constexpr (DIV) {
       const TO r = fmadd(cst, tzr[x + up] - tzr[x - dn], (TO)v);
       return isw ? (mid ? r : (TO)v) : (top ? (TO)LP_BOGUS : r);
     } else {
-      if (shp) return (TO)((double)v + sh);  // the plane's shift back, in binary64
       return (TO)v;
     }
   };
@@ -720,7 +714,7 @@ static hipError_t launch_c2r_n(const C2rSet *sets, int n, long in_pitch, long in
     const C2rSet &x = sets[f];
     if (x.nplanes < 1 || (DIV && (!x.tz || x.nplanes < 2))) return hipErrorInvalidValue;
     A.first[f] = (int)(xorder ? groups : planes);
-    A.s[f] = C2rArg<T, TO>{(const cx<T> *)x.in, (TO *)x.out, x.nplanes, x.div == 2 ? 1 : 0, (const TO *)x.tz, x.shift};
+    A.s[f] = C2rArg<T, TO>{(const cx<T> *)x.in, (TO *)x.out, x.nplanes, x.div == 2 ? 1 : 0, (const TO *)x.tz};
     planes += x.nplanes;
     groups += xcd_planes(x.nplanes, 0);
   }
@@ -753,10 +747,10 @@ static hipError_t launch_c2r(const C2rSet *sets, int n, long in_pitch, long in_p
 
 hipError_t row_c2r(Dt dtc, Dt dto, int M, const C2rSet *sets, int n, long in_pitch, long in_plane, int ncols_in,
                    int rows, long out_pitch, long out_plane, hipStream_t s, const double *ikx, double cst) {
-  if (n < 1) return hipErrorInvalidValue;
+  if (n < 1 || (dtc == F32 && dto == F64)) return hipErrorInvalidValue;
   const bool div = sets[0].div != 0;
   for (int f = 0; f < n; ++f)
-    if ((sets[f].div != 0) != div || (sets[f].shift && !(dtc == F32 && dto == F64))) return hipErrorInvalidValue;
+    if ((sets[f].div != 0) != div) return hipErrorInvalidValue;
   if (div) {
     if (dtc != dto || ikx || out_pitch < 2 * M) return hipErrorInvalidValue;
 #define CASE(m)                                                                                                   \
@@ -779,11 +773,8 @@ hipError_t row_c2r(Dt dtc, Dt dto, int M, const C2rSet *sets, int n, long in_pit
     if (dtc == F64 && dto == F32)                                                                                   \
       return launch_c2r<double, float, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s,     \
                                           dtc, ikx, cst);                                                           \
-    if (dtc == F32 && dto == F32)                                                                                   \
-      return launch_c2r<float, float, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s, dtc, \
-                                         ikx, cst);                                                                 \
-    return launch_c2r<float, double, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s, dtc,  \
-                                        ikx, cst);
+    return launch_c2r<float, float, m>(sets, n, in_pitch, in_plane, ncols_in, rows, out_pitch, out_plane, s, dtc,   \
+                                       ikx, cst);
   switch (M) {
     LP_ROW_LENGTHS(CASE)
     default: return hipErrorInvalidValue;

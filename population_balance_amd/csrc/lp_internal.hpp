@@ -55,9 +55,8 @@ hipError_t row_r2c(Dt dt, Dt din, int M, const R2cSet *sets, int n, long in_pitc
                    long out_pitch, long out_plane, int ncols_out, hipStream_t s);
 
 // Row pass: complex half spectra (ncols_in columns present, rest zero) -> real rows
-// of length 2M; columns [2M, out_pitch) set to zero.  Compute type dtc, store type dto.
-//  shift (dtc F32 -> dto F64): shift[plane] is added to every value of the plane in binary64,
-//  undoing row_r2c's shift.
+// of length 2M; columns [2M, out_pitch) set to zero.  Compute type dtc, store type dto (dtc, or
+// F32 from F64).
 //  div 1 / 2 (dtc == dto; all sets of a launch or none): the z-derivative term of divstress
 //  from tz (the layout of out): 1 (divstress_uv) adds cst (tz(k+1) - tz(k)) and writes BOGUS on
 //  the top level; 2 (divstress_w) adds cst (tz(k) - tz(k-1)) on levels 1..nplanes-2.
@@ -65,7 +64,6 @@ struct C2rSet {
   const void *in;
   void *out;
   int nplanes;
-  const double *shift = nullptr;
   const void *tz = nullptr;
   int div = 0;
 };
