@@ -388,7 +388,8 @@ __global__ void k_tau_frozen(const T *__restrict__ S11, const T *__restrict__ S1
 // ------------------------------------------------------------------------------------
 // droplets (pollen_all_in_one2, scalars_module_crossflow_mod.f90:1494-1786, with
 // pollen_RHS_calc2 :1894-4472, calcbeta_pcon :1795-1843, step_pollen2 :4481-4508), all
-// bins in one launch per pass, with per-bin face adjoints summed at the end.  Frozen: Kc_t (from Nu_t).  The transport is linear in C on each branch
+// bins in one launch per pass, the faces' adjoints summed over a run of bins in registers and
+// over the runs at the end.  Frozen: Kc_t (from Nu_t).  The transport is linear in C on each branch
 // of the SMART limiter: its transpose uses the branch the base C selects.  The three
 // directions are gathers (a thread per cell adds what the line scan of the fluxes
 // transposed would scatter into it, in the scan's order), so no pass needs atomics.

@@ -26,7 +26,8 @@ template <typename T> __device__ __forceinline__ cx<T> mk(T a, T b) { cx<T> r; r
 template <typename T> __device__ __forceinline__ cx<T> operator+(cx<T> a, cx<T> b) { return mk(a.x + b.x, a.y + b.y); }
 template <typename T> __device__ __forceinline__ cx<T> operator-(cx<T> a, cx<T> b) { return mk(a.x - b.x, a.y - b.y); }
 template <typename T> __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
-  // binary32: the products fused as the compiler fuses the plain expression in most kernels
+  // binary32: the products fused as the compiler fuses the plain expression in most kernels;
+  // binary64: see Dft in lp_fft4.hpp
   if constexpr (sizeof(T) == 4) return mk(fmadd(a.x, b.x, -(a.y * b.y)), fmadd(a.y, b.x, a.x * b.y));
   return mk(fmadd(-a.y, b.y, a.x * b.x), fmadd(a.x, b.y, a.y * b.x));
 }

@@ -782,7 +782,7 @@ hipError_t row_c2r(Dt dtc, Dt dto, int M, const C2rSet *sets, int n, long in_pit
 #undef CASE
 }
 
-// Planes of a column launch: they lie along y, where a grid has at most 65535 blocks.  Lists of
+// Planes of a column launch: they lie along y, where the device takes 65536 blocks.  Lists of
 // more (the test filters' 21 fields from 3121 levels on) are launched one set and this many
 // planes at a time, whole groups of eight.
 constexpr int kMaxPlanes = 65528;

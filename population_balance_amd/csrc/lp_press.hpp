@@ -7,9 +7,13 @@
 // p(j) = u(j) - c(j)/bet(j) p(j+1) downwards.  A recurrence over levels is affine in the
 // value that enters it, so a block of 16 modes x S segments of rows sweeps every segment
 // once from zero (its affine map: a factor and an offset), scans the S maps over LDS, and
-// sweeps again from the value that really enters.  The factors are at most 1 in magnitude,
-// so the scan is as stable as the serial sweep.  The rows stay in registers between the two
-// directions.
+// sweeps again from the value that really enters.  The factors of the interior rows are below
+// 1 in magnitude (|bet(j)| >= kx^2 + ky^2 + 1/dz^2 by induction), so that their maps shrink what
+// they join.  Those of the end rows may be large: the lid row's -1/bet(nz) is -337 for kx = 1,
+// dz = 1/256, nz = 257, and in the transposed systems it is 1/(dz^2 bet(nz)), 2.2e7, with -1/dz^2
+// for the wall row downwards.  They amplify nothing, because an end row is the last of its sweep:
+// no row is entered through its map, and its own value is formed from its neighbour's as in
+// the serial sweep.  The rows stay in registers between the two directions.
 //
 // What bounds it: one thread per mode held 33 K (256 x 256) to 0.5 K (32 x 32) threads, too
 // few to keep memory busy, each on a serial chain of 2 (nz + 1) rows with its p_hat written,
@@ -199,7 +203,10 @@ __device__ __forceinline__ void seg_solve(SegLds<S> &L, int s, int l, int n, Loa
 }
 
 // x / b rounded as the division rounds it, from rb = 1 / b rounded: the quotient's residual is
-// exact in one fused multiply-add, and the correction by it rounds correctly (Markstein 1990)
+// exact in one fused multiply-add, and the correction by it rounds correctly (Markstein 1990).
+// That holds for finite x, b, rb and x rb with |x| and |x / b| above 2^-960 or x = 0; below, the
+// residual may be subnormal and the last place off, and an infinite x gives NaN where the division
+// gives an infinity (a step reports either, in the velocity).  b = 0 is reported on its own (err).
 __device__ __forceinline__ double div_by(double x, double b, double rb) {
   const double q = x * rb;
   return fma(fma(-q, b, x), rb, q);
