@@ -196,10 +196,11 @@ template <typename V> __device__ __forceinline__ V buf_load(const V *base, unsig
 // it to RF (RHS_PCon_f = RHS_PCon, :1521, done by exchanging the two buffers) the last eight
 // blocks of each run copy them back from RF, otherwise (RF null) they are left alone.
 //
-// 192x192x128, 15 bins with inertia: 705 us for 1.56 GB of HBM traffic (2.2 TB/s).  One
+// 192x192x128, 15 bins with inertia: 700 us for 2.80 GB beyond the L2s (2.18 read, 0.62
+// written, 4.0 TB/s; the concentrations once and their right-hand side are 1.14).  One
 // point per thread with both faces of each direction and the end cells by branches was
 // bound by its vector instructions (630 per point and bin, now 190) and took 1155 us.  Now
-// the loads through L1 bound it (9 per point and bin and 23 per point and group): without
+// the loads bound it (9 through L1 per point and bin and 23 per point and group): without
 // the arithmetic it takes 700 us, without the neighbours along x 590, along y 620, without
 // both 470.  Groups of 3 bins 752, of 4 724, of 5 705 (more do not fit three wavefronts per
 // SIMD); the value two levels up or the next bin's loads in flight early: no gain.
