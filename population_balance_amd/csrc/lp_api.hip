@@ -119,7 +119,7 @@ struct lp_ctx {
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_aux_fork = nullptr, ev_aux = nullptr;
   bool prof_off = false;  // work on s2 that overlaps other kernels is not profiled
-  void *cv_spec[3] = {};  // convec's own spectral scratch (divstress runs meanwhile)
+  void *cv_spec[3] = {};  // convec's own spectral scratch (divstress runs meanwhile): max(2, group) of them
   bool fork_pending = false;  // the step's convec is still to be started on s2
   Dt fdt = F64;  // field type
   void *f[LP_NFIELDS] = {};
@@ -129,7 +129,7 @@ struct lp_ctx {
   SpecTables tab{};
   // scratch
   void *spec[4] = {};         // small spectra (lh x ny x nz) of the field type
-  void *specb[3] = {};        // big spectra (the nx/2 kept columns, pitch cv_pitch) x ny2 x nz
+  void *specb[3] = {};        // big spectra (the nx/2 kept columns, pitch cv_pitch) x ny2 x nz: `group` of them
   // Internal spectra keep rows of sp complex values: lh rounded up to 16, so that every row
   // starts on a 128-byte boundary.
   long sp = 0;
@@ -694,11 +694,14 @@ extern "C" int lp_create(const lp_config *cfg, lp_ctx **out) {
   c->group = group_of(spec_b);
   size_t vol_b = (size_t)nv * fe;
   for (auto &p : c->spec) CK(mem.want(&p, spec_b));
-  for (auto &p : c->specb) CK(mem.want(&p, specb_b));
+  // of specb and cv_spec as many as a launch takes fields (the adjoint takes two of cv_spec): a
+  // context as large as the card leaves none unused
+  const int nsets = c->group < 3 ? c->group : 3;
+  for (int q = 0; q < nsets; ++q) CK(mem.want(&c->specb[q], specb_b));
   const size_t cv_field = (size_t)c->cv_pitch * g.ny2 * g.nz * 2 * fe;
   CK(mem.want(&c->cvb, 6 * cv_field));
   for (auto &p : c->uvw_spec) CK(mem.want(&p, spec_b));
-  for (auto &p : c->cv_spec) CK(mem.want(&p, spec_b));
+  for (int q = 0; q < std::max(nsets, 2); ++q) CK(mem.want(&c->cv_spec[q], spec_b));
   CK(mem.want(&c->cvp, 3 * cv_field));
   for (auto &p : c->tmp) CK(mem.want(&p, vol_b));
   for (auto &p : c->S) CK(mem.want(&p, vol_b));

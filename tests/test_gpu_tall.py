@@ -134,3 +134,21 @@ def test_adjoint_tall(nz):
     print()
     lg.close()
     o.close()
+
+
+def test_context_memory():
+    """a context whose passes take one field a launch keeps no spectra for more: at 32x32x20000,
+    binary64, model 1, no more than the 911.3 bytes a point that contexts took when every pass
+    took one field"""
+    import torch
+    from population_balance_amd.lesgo import Lesgo
+    Lesgo(abi.make_config(32, 32, 4)).close()
+    cfg = _tall(32, 32, 20000, model=1)
+    print("\n[case] memory of a 32x32x20000 context", flush=True)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    lg = Lesgo(cfg)
+    used = free - torch.cuda.mem_get_info()[0]
+    lg.close()
+    print(f"  {used / (32 * 32 * 20000):.1f} bytes a point")
+    assert used <= 911.3 * 32 * 32 * 20000
