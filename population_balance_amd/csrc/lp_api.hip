@@ -1696,18 +1696,32 @@ static int do_press(lp_ctx *c) {
   HIPCHK(hipStreamWaitEvent(c->s, c->ev_aux, 0));
   cx<double> *ph = (cx<double> *)c->phat;
   prof_begin(c, LP_K_PRESS_TRIDIAG);
-#define PRESS(S, R)                                                                                             \
-  FDISPATCH(c, T, hipLaunchKernelGGL((k_press_tridiag<T, S, R>), dim3((unsigned)(ps / kPsModes)),              \
-                                     dim3(kPsModes * S), 0, c->s, (const cx<T> *)c->Hs[0],                     \
-                                     (const cx<T> *)c->Hs[1], (const cx<T> *)c->Hs[2], (const cx<T> *)c->bw,   \
-                                     (const cx<T> *)c->tw, c->kx, c->ky, ph, (const double *)c->bet, gg.lh,   \
-                                     gg.ny, gg.nz, c->sp, gg.dz, c->d_err))
-  switch (press_segs(gg.nz + 1)) {
-    case 8: PRESS(8, false); break;
-    case 16: PRESS(16, false); break;
-    default:
-      if (press_rounds(gg.nz + 1)) PRESS(32, true);
-      else PRESS(32, false);
+  const long pblocks = ps / kPsModes;
+#define PRESS(T, S, R)                                                                                          \
+  hipLaunchKernelGGL((k_press_tridiag<T, S, R>), dim3((unsigned)pblocks), dim3(kPsModes * S), 0, c->s,         \
+                     (const cx<T> *)c->Hs[0], (const cx<T> *)c->Hs[1], (const cx<T> *)c->Hs[2],                \
+                     (const cx<T> *)c->bw, (const cx<T> *)c->tw, c->kx, c->ky, ph, (const double *)c->bet,     \
+                     gg.lh, gg.ny, gg.nz, c->sp, gg.dz, c->d_err)
+  const int rows = gg.nz + 1;
+  if (c->fdt == F64) {
+    switch (press_segs64(rows, pblocks)) {
+      case 8: PRESS(double, 8, false); break;
+      case 16:
+        if (serial_rounds(rows, 16) > 1) PRESS(double, 16, true);
+        else PRESS(double, 16, false);
+        break;
+      default:
+        if (serial_rounds(rows, 32) > 1) PRESS(double, 32, true);
+        else PRESS(double, 32, false);
+    }
+  } else {
+    switch (press_segs(rows)) {
+      case 8: PRESS(float, 8, false); break;
+      case 16: PRESS(float, 16, false); break;
+      default:
+        if (press_rounds(rows)) PRESS(float, 32, true);
+        else PRESS(float, 32, false);
+    }
   }
 #undef PRESS
   HIPCHK(hipGetLastError());

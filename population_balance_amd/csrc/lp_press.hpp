@@ -42,6 +42,22 @@ __host__ __device__ constexpr int press_segs(int n) {
 }
 __host__ __device__ constexpr bool press_rounds(int n) { return n > 32 * kPsRows; }
 
+// The binary64 solve hands the elimination from segment to segment, so a block of 32 segments,
+// which leaves room for no other on its CU, stands still while one of them sweeps.  With a block
+// for every CU, 16 segments in rounds are better beyond 144 rows: two blocks share a CU and one
+// loads while the other sweeps.  16 against 32 segments: 165 against 242 us at 256 x 256 x 160
+// (one thread per mode 162), 226 / 305 at 256 x 256 x 257 (281), 299 / 567 at 300 levels (342), 387
+// / 641 at 400 (468), 69 / 102 at 128 x 128 x 257 (158).  With fewer blocks than CUs there is
+// nothing to share a CU with: 323 / 274 at 32 x 32 x 2000 (64 blocks), 63 / 63 at 64 x 64 x 300 (192).
+// The rounds are equal in length.
+__host__ __device__ constexpr int press_segs64(int n, long blocks) {
+  return n > 16 * kPsRows && blocks >= 256 ? 16 : press_segs(n);
+}
+__host__ __device__ constexpr int serial_rounds(int n, int S) { return (n + S * kPsRows - 1) / (S * kPsRows); }
+__host__ __device__ constexpr int serial_rows(int n, int S) {
+  return (n + S * serial_rounds(n, S) - 1) / (S * serial_rounds(n, S));
+}
+
 // press_stag_array.f90:149-329 / tridag_array.f90:30-155: bet(j) of each mode's system
 // (a = c = 1/dz^2, b = -(kx^2 + ky^2 + 2/dz^2) inside; the wall row b = -1, c = 1; the lid
 // row a = -1, b = 1), bet(j) = b(j) - a(j) (c(j-1)/bet(j-1)), in [(nz+1)][ny][pitch]; inv:
@@ -221,9 +237,8 @@ template <int S, bool RNDS, typename Load, typename Num, typename Up, typename O
 __device__ __forceinline__ void seg_solve_serial(cx<double> (&end)[kPsModes], int s, int l, int n, Load load, Num num,
                                                  Up above, Out out, cx<double> (&r)[kPsRows], double (&f)[kPsRows],
                                                  cx<double> *__restrict__ u, unsigned plane) {
-  const int per = (n + S - 1) / S;
-  const int Lr = per < kPsRows ? per : kPsRows;
-  const int rounds = RNDS ? (n + S * Lr - 1) / (S * Lr) : 1;
+  const int rounds = RNDS ? serial_rounds(n, S) : 1;
+  const int Lr = serial_rows(n, S);
   const int sw = wave_seg();
   double rb[kPsRows];
   if (s == 0) end[l] = mk<double>(0.0, 0.0);
@@ -291,7 +306,7 @@ __device__ __forceinline__ void seg_solve_serial(cx<double> (&end)[kPsModes], in
 // mean mode (a = -1, 1/bet = 1, no backward sweep), zero on the Nyquist row and column.
 // H levels 1..nz-1 at planes 0..nz-2 (complex TH), bw / tw_ one plane, ph planes 0..nz.
 template <typename TH, int S, bool RNDS>
-__global__ __launch_bounds__(kPsModes *S, RNDS ? 1 : sizeof(TH) == 4 ? 4 : 3) void k_press_tridiag(
+__global__ __launch_bounds__(kPsModes *S, RNDS && sizeof(TH) == 4 ? 1 : sizeof(TH) == 4 ? 4 : 3) void k_press_tridiag(
     const cx<TH> *__restrict__ Hx, const cx<TH> *__restrict__ Hy, const cx<TH> *__restrict__ Hz,
     const cx<TH> *__restrict__ bw, const cx<TH> *__restrict__ tw_, const double *__restrict__ kxt,
     const double *__restrict__ kyt, cx<double> *ph, const double *__restrict__ tab, int lh, int ny, int nz,

@@ -336,3 +336,31 @@ def test_steps_theta_uneven_mixed(nx, ny, nz):
     assert max(errs.values()) < 1e-5, errs
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nz", [143, 144, 287, 288, 500])
+def test_pressure_rounds(nz):
+    """the binary64 pressure solve where a block's segments go in rounds of equal length (128 x 64
+    points: 320 blocks): one round, two, and more, at 1e-12 of the oracle"""
+    from harness import random_fields
+    from oracle import Oracle
+    from population_balance_amd import ic
+    from population_balance_amd.lesgo import Lesgo
+    cfg = abi.make_config(128, 64, nz)
+    g = cfg.grid
+    o, lg = Oracle(cfg), Lesgo(cfg)
+    print(f"\n[case] pressure rounds nz={nz}", flush=True)
+    u, v, w = ic.turbulent_ic(g, seed=24, log_law=False)
+    n = random_fields(cfg, ["u", "v", "w", "divtz"], seed=24)
+    for name, a in (("u", u + 0.1 * n["u"]), ("v", v + 0.1 * n["v"]), ("w", w + 0.1 * n["w"]), ("divtz", n["divtz"])):
+        o.set_field(name, a)
+        lg.upload(name, a)
+    o.call("press_stag_array")
+    lg.press_stag_array()
+    for name, top in (("p", nz), ("dpdx", nz - 1), ("dpdy", nz - 1)):
+        err = rel_l2(lg.download(name)[:top], o.field(name)[:top], g.nx)
+        print(f"  {name}: {err:.2e}", end="")
+        assert err < TOL, (name, err)
+    print()
+    lg.close()
+    o.close()

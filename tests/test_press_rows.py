@@ -28,11 +28,12 @@ static void check(const char *what, int row, int row0, int rows, unsigned ps, un
 
 int main(int argc, char **argv) {
   const int nx = std::atoi(argv[1]), ny = std::atoi(argv[2]), nz = std::atoi(argv[3]);
-  const int n = nz + 1, S = press_segs(n), W = 64 / kPsModes;
   const unsigned pitch = (nx / 2 + 1 + 15) / 16 * 16, ps = pitch * ny;
-  const int per = (n + S - 1) / S, Lr = per < kPsRows ? per : kPsRows;
-  const int rounds = press_rounds(n) ? (n + S * Lr - 1) / (S * Lr) : 1;
-  if ((long)rounds * S * Lr < n) return std::printf("rows left out\n"), 1;
+  const bool serial = std::atoi(argv[4]);  // the binary64 solve's split, else the scan's
+  const int n = nz + 1, S = serial ? press_segs64(n, ps / kPsModes) : press_segs(n), W = 64 / kPsModes;
+  const int per = (n + S - 1) / S, Lr = serial ? serial_rows(n, S) : per < kPsRows ? per : kPsRows;
+  const int rounds = serial ? serial_rounds(n, S) : press_rounds(n) ? (n + S * Lr - 1) / (S * Lr) : 1;
+  if ((long)rounds * S * Lr < n || Lr > kPsRows) return std::printf("rows left out\n"), 1;
   const unsigned at[2] = {0, ps - 1};
   auto low = [](int a, int b) { return a < b ? a : b; };
   for (int rd = 0; rd < rounds; ++rd)
@@ -66,9 +67,10 @@ def program(tmp_path_factory):
     return str(exe)
 
 
+@pytest.mark.parametrize("serial", [0, 1])
 @pytest.mark.parametrize("nx,ny,nz", [(32, 32, 4), (64, 32, 71), (64, 32, 72), (64, 64, 143), (96, 64, 288),
-                                      (256, 256, 257), (256, 256, 7281), (256, 256, 9000), (128, 128, 27000),
-                                      (32, 32, 270000)])
-def test_row_addresses(program, nx, ny, nz):
-    r = subprocess.run([program, str(nx), str(ny), str(nz)], capture_output=True, text=True)
+                                      (128, 64, 144), (128, 128, 289), (256, 256, 257), (256, 256, 7281),
+                                      (256, 256, 9000), (128, 128, 27000), (32, 32, 270000)])
+def test_row_addresses(program, nx, ny, nz, serial):
+    r = subprocess.run([program, str(nx), str(ny), str(nz), str(serial)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
