@@ -1788,12 +1788,18 @@ static int do_pollen_rhs(lp_ctx *c, const double *prev, bool fuse_step = false, 
   const double nb = (double)dg.nv * dg.npc * 8.0;
   prof_begin(c, LP_K_POLLEN_RHS);
   const long prow = 256 / pollen_tile(gg.nx), pgrp = (dg.npc + kPollenBins - 1) / kPollenBins;
-  const long pblk = ((gg.ny + prow - 1) / prow * (gg.nx / pollen_tile(gg.nx)) + 7) / 8 * 8;
+  const long ntile = (gg.ny + prow - 1) / prow * (gg.nx / pollen_tile(gg.nx));
+  P.per = ntile >= kPollenXcd ? (int)((ntile + 7) / 8) : 0;
   // level runs of at most kPollenLevels, halved down to 2 while there are fewer than two
-  // blocks per CU (a run computes its first face and reads four levels before its own work)
+  // blocks per CU, and to 1 while there is at most one (a run computes its first face and reads
+  // four levels before its own work).  Runs of 1 against 2 levels: 32x32x17 with 3 bins 12.5 against
+  // 16.1 us, 64x64x33 with 2 bins (256 blocks in runs of 2) 11.9 / 13.1, but 96x64x33 with 3 (384
+  // blocks) 24.2 / 21.0
   int lev = kPollenLevels;
-  while (lev > 2 && pblk * pgrp * ((gg.nz - 1 + lev - 1) / lev) < 512) lev /= 2;
-  const dim3 pgrid((unsigned)(pblk + 8), (unsigned)pgrp, (unsigned)((gg.nz - 1 + lev - 1) / lev));
+  auto blocks = [&](int l) { return ntile * pgrp * ((gg.nz - 1 + l - 1) / l); };
+  while (lev > 2 && blocks(lev) < 512) lev /= 2;
+  if (lev == 2 && blocks(2) <= 256) lev = 1;
+  const dim3 pgrid((unsigned)(P.per ? 8 * P.per : ntile), (unsigned)pgrp, (unsigned)((gg.nz - 1 + lev - 1) / lev + 1));
   auto rhs = [&](auto kern, auto T_) {
     using T = decltype(T_);
     hipLaunchKernelGGL(kern, pgrid, dim3(256), 0, c->s, PC, RH, prev, c->ui0, c->vi0, (const double *)c->f[LP_W],

@@ -146,6 +146,7 @@ struct PollenParams {
   int bc_x, bc_y;           // 0 periodic, 1 inlet, 2 upwind-sign ghosts
   int settling;
   int src_on, src_k0;       // source active this step; its lower level (0-based)
+  int per;                  // tiles per XCD; 0: tiles in the order of the blocks
 };
 
 // Half of the SMART face's correction, psi(r) den / 2 (smart_face): num and den with the sign
@@ -182,19 +183,21 @@ template <typename V> __device__ __forceinline__ V buf_load(const V *base, unsig
 // velocities of the bin (:2243-2276), ghosts (:2478-2590), SMART faces (:2877-3475), flux
 // divergence and SGS diffusion (:3559-3677) and the point source (:4222-4256).
 //
-// A thread takes one (x, y) and marches up the run of levels blockIdx.z with the
+// A thread takes one (x, y) and marches up the run of levels blockIdx.z - 1 with the
 // concentrations, differences, face values and diffusive fluxes of the last level of its
 // bins (blockIdx.y = group) in registers: a level loads one new value along z and computes
 // one z face instead of two; the bin-independent inputs (face velocities, accelerations,
 // Kc_t) are loaded once per group.  A periodic row or column needs no end cases (its end
 // faces use the face-1 velocity, which is that of face n + 1 too): the neighbours are read
 // at wrapped indices, and the ghosts of the other boundary conditions are loads too.
-// Offsets within a level are 32-bit bytes from uniform addresses.  XCD q (blockIdx.x % 8)
-// takes consecutive tiles of pollen_tile(nx) x (256 / pollen_tile(nx)) points, so that the
-// rows above and below are in its L2, and three of four in the CU's L1.
+// Offsets within a level are 32-bit bytes from uniform addresses.  With kPollenXcd tiles of
+// pollen_tile(nx) x (256 / pollen_tile(nx)) points or more, XCD q (blockIdx.x % 8) takes
+// consecutive ones (P.per), so that the rows above and below are in its L2, and three of four in
+// the CU's L1; fewer would leave XCDs without work (4 tiles at 32x32: 38 us for 33 levels and 16
+// bins, in the order of the blocks 20) and go in order.
 // Points outside the cells keep the values of the previous RHS: when the caller has moved
-// it to RF (RHS_PCon_f = RHS_PCon, :1521, done by exchanging the two buffers) the last eight
-// blocks of each run copy them back from RF, otherwise (RF null) they are left alone.
+// it to RF (RHS_PCon_f = RHS_PCon, :1521, done by exchanging the two buffers) the blocks of
+// blockIdx.z = 0 copy them back from RF, otherwise (RF null) they are left alone.
 //
 // 192x192x128, 15 bins with inertia: 700 us for 2.80 GB beyond the L2s (2.18 read, 0.62
 // written, 4.0 TB/s; the concentrations once and their right-hand side are 1.14).  One
@@ -209,6 +212,7 @@ __host__ __device__ inline int pollen_tile(int nx) { return nx % 64 == 0 ? 64 : 
 static constexpr unsigned kGone = 0xfffffff0u;  // past any level: reads 0
 // levels per run, at most (8: 745 us, 32: 770, 64: 875 at 192x192x128)
 static constexpr int kPollenLevels = 16;
+static constexpr int kPollenXcd = 64;  // tiles from which an XCD's are consecutive
 template <typename T, bool SIGNS, bool INERT>
 __global__ __launch_bounds__(256, SIGNS ? 2 : 3) void k_pollen_rhs(
     const double *__restrict__ PC, double *__restrict__ RH, const double *__restrict__ RF,
@@ -221,21 +225,20 @@ __global__ __launch_bounds__(256, SIGNS ? 2 : 3) void k_pollen_rhs(
   const int nx = g.nx, ny = g.ny, nz = g.nz, ld = g.ld, np = (int)g.np;
   const int b0 = blockIdx.y * G;  // first bin of the group (uniform)
   const int nb = g.npc - b0 < G ? g.npc - b0 : G;
-  const int kb = (int)((long)blockIdx.z * (nz - 1) / gridDim.z), ke = (int)((long)(blockIdx.z + 1) * (nz - 1) / gridDim.z);
-  const int nblk = ((int)gridDim.x - 8) / 8;
-  if ((int)blockIdx.x >= 8 * nblk) {  // points outside the cells
+  if (blockIdx.z == 0) {  // points outside the cells: the padding columns, then the top level
     if (!RF) return;
-    const int pad = ld - nx, lev = pad * ny;
-    const int n = lev * (ke - kb) + (ke == nz - 1 ? np : 0);
-    for (int t = ((int)blockIdx.x - 8 * nblk) * 256 + (int)threadIdx.x; t < n; t += 8 * 256) {
-      const int k = kb + t / lev, q = t % lev;
-      const long o = t < lev * (ke - kb) ? (long)k * np + (q / pad) * ld + nx + q % pad
-                                         : (long)(nz - 1) * np + (t - lev * (ke - kb));
+    const int pad = ld - nx, lev = pad * ny, cols = lev * (nz - 1);
+    for (int t = (int)(blockIdx.x * 256 + threadIdx.x); t < cols + np; t += (int)gridDim.x * 256) {
+      const int k = t / lev, q = t % lev;
+      const long o = t < cols ? (long)k * np + (q / pad) * ld + nx + q % pad : (long)(nz - 1) * np + (t - cols);
       for (int bb = 0; bb < nb; ++bb) RH[(long)(b0 + bb) * g.nv + o] = RF[(long)(b0 + bb) * g.nv + o];
     }
     return;
   }
-  const int tile = (int)(blockIdx.x & 7) * nblk + (int)(blockIdx.x >> 3), tw = pollen_tile(nx), ntx = nx / tw;
+  const int kb = (int)((long)(blockIdx.z - 1) * (nz - 1) / (gridDim.z - 1));
+  const int ke = (int)((long)blockIdx.z * (nz - 1) / (gridDim.z - 1));
+  const int tw = pollen_tile(nx), ntx = nx / tw;
+  const int tile = P.per ? (int)(blockIdx.x & 7) * P.per + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
   const int i = tile % ntx * tw + (int)threadIdx.x % tw, j = tile / ntx * (256 / tw) + (int)threadIdx.x / tw;
   if (j >= ny) return;
   const int p = j * ld + i;
