@@ -290,23 +290,35 @@ __global__ __launch_bounds__(row_block<T>()) void k_row_c2r(Sets<C2rArg<T, TO>, 
   // neighbour levels, clamped: uv k + 1 and k, w k and k - 1
   const TO *tzr = DIV ? S.tz + od : nullptr;
   const long up = isw || top ? 0 : out_plane, dn = isw && mid ? out_plane : 0;
-  auto fin = [&](T v, int x) -> TO {
-    if constexpr (DIV) {
-      const TO r = fmadd(cst, tzr[x + up] - tzr[x - dn], (TO)v);
-      return isw ? (mid ? r : (TO)v) : (top ? (TO)LP_BOGUS : r);
-    } else {
-      return (TO)v;
-    }
-  };
 #pragma unroll
   for (int j = 0; j < F::G; ++j) {
     cx<T> a[P];
     if (F::stage2(j, t, sc, a) && valid) {
+      if constexpr (DIV) {
+        // tz first: the compiler, which cannot tell it from the output, would wait for each
+        // value's loads between two stores
+        TO z[P][2];
 #pragma unroll
-      for (int k1 = 0; k1 < P; ++k1) {
-        const int n = t + P * j + Q * k1;
-        dst[2 * n] = fin(a[k1].x, 2 * n);
-        dst[2 * n + 1] = fin(a[k1].y, 2 * n + 1);
+        for (int k1 = 0; k1 < P; ++k1)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int x = 2 * (t + P * j + Q * k1) + h;
+            z[k1][h] = tzr[x + up] - tzr[x - dn];
+          }
+#pragma unroll
+        for (int k1 = 0; k1 < P; ++k1)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const TO v = h ? (TO)a[k1].y : (TO)a[k1].x, r = fmadd(cst, z[k1][h], v);
+            dst[2 * (t + P * j + Q * k1) + h] = isw ? (mid ? r : v) : (top ? (TO)LP_BOGUS : r);
+          }
+      } else {
+#pragma unroll
+        for (int k1 = 0; k1 < P; ++k1) {
+          const int n = t + P * j + Q * k1;
+          dst[2 * n] = (TO)a[k1].x;
+          dst[2 * n + 1] = (TO)a[k1].y;
+        }
       }
     }
   }
