@@ -1789,7 +1789,6 @@ static int do_pollen_rhs(lp_ctx *c, const double *prev, bool fuse_step = false, 
   prof_begin(c, LP_K_POLLEN_RHS);
   const long prow = 256 / pollen_tile(gg.nx), pgrp = (dg.npc + kPollenBins - 1) / kPollenBins;
   const long ntile = (gg.ny + prow - 1) / prow * (gg.nx / pollen_tile(gg.nx));
-  P.per = ntile >= kPollenXcd ? (int)((ntile + 7) / 8) : 0;
   // level runs of at most kPollenLevels, halved down to 2 while there are fewer than two
   // blocks per CU, and to 1 while there is at most one (a run computes its first face and reads
   // four levels before its own work).  Runs of 1 against 2 levels: 32x32x17 with 3 bins 12.5 against
@@ -1799,7 +1798,10 @@ static int do_pollen_rhs(lp_ctx *c, const double *prev, bool fuse_step = false, 
   auto blocks = [&](int l) { return ntile * pgrp * ((gg.nz - 1 + l - 1) / l); };
   while (lev > 2 && blocks(lev) < 512) lev /= 2;
   if (lev == 2 && blocks(2) <= 256) lev = 1;
-  const dim3 pgrid((unsigned)(P.per ? 8 * P.per : ntile), (unsigned)pgrp, (unsigned)((gg.nz - 1 + lev - 1) / lev + 1));
+  P.runs = (gg.nz - 1 + lev - 1) / lev;
+  P.per = ntile >= kPollenXcd ? (int)((ntile + 7) / 8) : ntile < 8 && P.runs >= kPollenRuns ? -1 : 0;
+  const dim3 pgrid((unsigned)(P.per > 0 ? 8 * P.per : P.per == 0 ? ntile : 8 * ((P.runs + 7) / 8) * ntile), (unsigned)pgrp,
+                   (unsigned)(P.per >= 0 ? P.runs + 1 : 2));
   auto rhs = [&](auto kern, auto T_) {
     using T = decltype(T_);
     hipLaunchKernelGGL(kern, pgrid, dim3(256), 0, c->s, PC, RH, prev, c->ui0, c->vi0, (const double *)c->f[LP_W],

@@ -146,7 +146,8 @@ struct PollenParams {
   int bc_x, bc_y;           // 0 periodic, 1 inlet, 2 upwind-sign ghosts
   int settling;
   int src_on, src_k0;       // source active this step; its lower level (0-based)
-  int per;                  // tiles per XCD; 0: tiles in the order of the blocks
+  int runs;                 // runs of levels
+  int per;                  // tiles per XCD; 0: tiles in the order of the blocks; -1: runs split over XCDs
 };
 
 // Half of the SMART face's correction, psi(r) den / 2 (smart_face): num and den with the sign
@@ -194,7 +195,9 @@ template <typename V> __device__ __forceinline__ V buf_load(const V *base, unsig
 // pollen_tile(nx) x (256 / pollen_tile(nx)) points or more, XCD q (blockIdx.x % 8) takes
 // consecutive ones (P.per), so that the rows above and below are in its L2, and three of four in
 // the CU's L1; fewer would leave XCDs without work (4 tiles at 32x32: 38 us for 33 levels and 16
-// bins, in the order of the blocks 20) and go in order.
+// bins, in the order of the blocks 20) and go in order.  Fewer tiles than XCDs and kPollenRuns
+// runs or more: an XCD takes consecutive runs, the levels of a tile staying in its L2 (32x32x300,
+// 4 bins: 28 us, in the order of the blocks 40 to 55).
 // Points outside the cells keep the values of the previous RHS: when the caller has moved
 // it to RF (RHS_PCon_f = RHS_PCon, :1521, done by exchanging the two buffers) the blocks of
 // blockIdx.z = 0 copy them back from RF, otherwise (RF null) they are left alone.
@@ -212,7 +215,8 @@ __host__ __device__ inline int pollen_tile(int nx) { return nx % 64 == 0 ? 64 : 
 static constexpr unsigned kGone = 0xfffffff0u;  // past any level: reads 0
 // levels per run, at most (8: 745 us, 32: 770, 64: 875 at 192x192x128)
 static constexpr int kPollenLevels = 16;
-static constexpr int kPollenXcd = 64;  // tiles from which an XCD's are consecutive
+static constexpr int kPollenXcd = 64;   // tiles from which an XCD's are consecutive
+static constexpr int kPollenRuns = 64;  // runs from which an XCD's are, with fewer than 8 tiles
 template <typename T, bool SIGNS, bool INERT>
 __global__ __launch_bounds__(256, SIGNS ? 2 : 3) void k_pollen_rhs(
     const double *__restrict__ PC, double *__restrict__ RH, const double *__restrict__ RF,
@@ -235,10 +239,19 @@ __global__ __launch_bounds__(256, SIGNS ? 2 : 3) void k_pollen_rhs(
     }
     return;
   }
-  const int kb = (int)((long)(blockIdx.z - 1) * (nz - 1) / (gridDim.z - 1));
-  const int ke = (int)((long)blockIdx.z * (nz - 1) / (gridDim.z - 1));
   const int tw = pollen_tile(nx), ntx = nx / tw;
-  const int tile = P.per ? (int)(blockIdx.x & 7) * P.per + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  const int xcd = (int)(blockIdx.x & 7), xi = (int)(blockIdx.x >> 3);
+  int tile, run;
+  if (P.per >= 0) {
+    tile = P.per ? xcd * P.per + xi : (int)blockIdx.x;
+    run = (int)blockIdx.z - 1;
+  } else {
+    const int ntile = ntx * ((ny + 256 / tw - 1) / (256 / tw));
+    tile = xi % ntile;
+    run = xcd * ((P.runs + 7) / 8) + xi / ntile;
+    if (run >= P.runs) return;
+  }
+  const int kb = (int)((long)run * (nz - 1) / P.runs), ke = (int)((long)(run + 1) * (nz - 1) / P.runs);
   const int i = tile % ntx * tw + (int)threadIdx.x % tw, j = tile / ntx * (256 / tw) + (int)threadIdx.x / tw;
   if (j >= ny) return;
   const int p = j * ld + i;

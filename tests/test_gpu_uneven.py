@@ -364,3 +364,14 @@ def test_pressure_rounds(nz):
     print()
     lg.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,nb,bc,kw", [
+    (32, 32, 70, 3, (2, 2), {}),      # 69 runs of one level split over the XCDs, the last XCD's part empty
+    (32, 32, 140, 7, (0, 1), {}),     # two groups, runs of 2
+    (96, 192, 9, 6, (1, 0), {}),      # 72 tiles, an XCD's consecutive
+    (64, 64, 65, 2, (0, 0), {}),      # 16 tiles in the order of the blocks
+])
+def test_droplet_transport_split(nx, ny, nz, nb, bc, kw):
+    """the droplet right-hand side in each order of tiles and runs, as test_droplet_transport_tiles"""
+    test_droplet_transport_tiles(nx, ny, nz, nb, bc, kw)
