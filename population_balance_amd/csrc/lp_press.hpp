@@ -22,9 +22,9 @@
 // 128-byte lines (modes are taken in the spectra's own pitch, not as kx + lh ky), and at
 // 122 VGPRs (binary32) two blocks of 512 threads share a CU, so that one block's loads run
 // beside the other's sweeps.  RNDS false leaves out the loop over rounds, which would cost
-// 60 registers.  Measured, one thread per mode -> this: binary32 spectra 246 -> 93 us at
-// 256 x 256 x 257 (H, 1/bet and p_hat: 415 MB, 4.5 TB/s), 94 -> 31 us at 192 x 192 x 128;
-// binary64 80 -> 32 us at 128 x 128 x 129, 23 -> 12 us at 32 x 32 x 33; the transposed solve
+// 60 registers.  Measured, one thread per mode -> this: binary32 spectra 246 -> 94 us at
+// 256 x 256 x 257 (H, 1/bet and p_hat: 415 MB, 4.4 TB/s), 94 -> 31 us at 192 x 192 x 128;
+// binary64 80 -> 33 us at 128 x 128 x 129, 23 -> 12 us at 32 x 32 x 33; the transposed solve
 // 95 -> 19 us at 128 x 128 x 65.
 #pragma once
 #include "lp_kernels.hpp"
